@@ -65,6 +65,57 @@ TA_EXPORT int thrust_amd_free_universal(void* ptr) {
   return (int)hipHostFree(ptr);
 }
 
+namespace ta {
+
+// Device-to-device copy.  Bound by HBM; the shape is the one that moves the most bytes per second on
+// this device (256 threads, one 16-byte vector each, 4 KiB per workgroup: many workgroups that live
+// for one load and one store keep the memory system busier than few that loop).  1 GiB: 0.347 ms =
+// 6.2 TB/s; the runtime's own copy, whose 256 workgroups loop, 0.428 ms = 5.0 TB/s.
+__global__ __launch_bounds__(256) void copy_kernel(char* __restrict__ dst, const char* __restrict__ src, uint64_t bytes) {
+  // dst and src are equally misaligned: the same number of bytes before the first boundary of both
+  const uint64_t lead = (16 - (reinterpret_cast<uintptr_t>(dst) & 15)) & 15;
+  const uint64_t head = lead < bytes ? lead : bytes;
+  const uint64_t vecs = (bytes - head) / 16;
+  const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < vecs) reinterpret_cast<uint4*>(dst + head)[i] = reinterpret_cast<const uint4*>(src + head)[i];
+  if (blockIdx.x == 0 && threadIdx.x < 16) {
+    const uint64_t tail = head + vecs * 16 + threadIdx.x;
+    if (threadIdx.x < head) dst[threadIdx.x] = src[threadIdx.x];
+    if (tail < bytes) dst[tail] = src[tail];
+  }
+}
+
+// Below this the copy lives in the caches and the runtime's kernel is as fast (64 MiB: 19.7 us here,
+// 19.5 us there; 256 MiB: 88.8 against 98.9 us), without the two pointer lookups.
+constexpr size_t COPY_KERNEL_MIN_BYTES = (size_t)128 << 20;
+
+// True for memory of the given device (not of another device, nor host memory, which the runtime
+// copies in its own way).
+static bool is_own_device_memory(const void* p, int device) {
+  hipPointerAttribute_t attr;
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return attr.type == hipMemoryTypeDevice && attr.device == device;
+}
+
+static int copy_on_device(void* dst, const void* src, size_t bytes, hipStream_t stream) {
+  int device = 0;
+  if (bytes >= COPY_KERNEL_MIN_BYTES && ((reinterpret_cast<uintptr_t>(dst) ^ reinterpret_cast<uintptr_t>(src)) & 15) == 0 &&
+      hipGetDevice(&device) == hipSuccess && is_own_device_memory(dst, device) && is_own_device_memory(src, device)) {
+    const uint64_t blocks = bytes / 16 / 256 + 1;
+    if (blocks <= 0x7fffffffull) {
+      TA_LAUNCH("copy", stream, copy_kernel, dim3((uint32_t)blocks), dim3(256), static_cast<char*>(dst), static_cast<const char*>(src), (uint64_t)bytes);
+      TA_CHECK_LAUNCH();
+      return 0;
+    }
+  }
+  return (int)hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, stream);
+}
+
+}  // namespace ta
+
 TA_EXPORT int thrust_amd_memcpy(void* dst, const void* src, size_t bytes, int kind, void* stream) {
   if (bytes == 0) return 0;
   if (!dst || !src) return (int)hipErrorInvalidValue;
@@ -77,7 +128,7 @@ TA_EXPORT int thrust_amd_memcpy(void* dst, const void* src, size_t bytes, int ki
       TA_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, s));
       return (int)hipStreamSynchronize(s);
     case THRUST_AMD_D2D:
-      return (int)hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, s);
+      return ta::copy_on_device(dst, src, bytes, s);
     default:
       return (int)hipErrorInvalidValue;
   }
