@@ -1,4 +1,5 @@
-// thrust_amd_sort_keys / thrust_amd_sort_pairs: onesweep least-significant-digit radix sort.
+// thrust_amd_sort_keys / thrust_amd_sort_pairs: onesweep least-significant-digit radix sort (up to 8192
+// keys: one workgroup, small_sort.hpp).
 //
 //   init       zeroes the digit histograms, the per-pass tile descriptors and tickets
 //   histogram  one read of the keys builds the 256-bin histogram of EVERY 8-bit digit
@@ -11,9 +12,8 @@
 //              look-back over the tiles before it, and scatters keys (and values)
 //   copy-back  only if an odd number of passes ran
 //
-// Ranking inside a tile uses the wave64 match pattern: for each of the 8 digit bits one
-// ballot, folded into a 64-bit peer mask with v_bitop3; rank = wave-private LDS counter
-// + number of peers in lower lanes (v_mbcnt accumulates onto the counter's value).  Lanes hold keys wave-striped (lane l of wave w holds
+// Ranking inside a tile uses the wave64 match pattern (radix_rank.hpp): rank = wave-private LDS counter
+// + number of peers in lower lanes.  Lanes hold keys wave-striped (lane l of wave w holds
 // keys l, 64+l, ... of the wave's span), so (round, lane) order is memory order and the
 // pass is stable.  Keys and values are then exchanged through LDS so that global stores
 // are contiguous per digit run.
@@ -30,12 +30,13 @@
 #include "common.hpp"
 #include "dispatch.hpp"
 #include "launch.hpp"
+#include "radix_rank.hpp"
+#include "small_sort.hpp"
+#include "sort_codec.hpp"
 #include "sort_tickets.hpp"
 
 namespace ta {
 
-constexpr int RADIX_BITS = 8;
-constexpr int RADIX_SIZE = 1 << RADIX_BITS;
 constexpr int MAX_PASSES = 8;
 constexpr uint64_t SORT_MAX_N = (1ull << 32) - 1;       // positions and counts are 32-bit
 constexpr uint64_t SORT_MAX_N_NARROW = (1ull << 30) - 1;  // ... and fit 30 bits up to here
@@ -48,27 +49,6 @@ struct Descriptor {
   static constexpr D VALUE_MASK = ((D)1 << SHIFT) - 1;
   static constexpr D PARTIAL = (D)1 << SHIFT;
   static constexpr D INCLUSIVE = (D)2 << SHIFT;
-};
-
-// Key <-> radix encoding, decided at run time (uniform across the grid).
-//   sign:   sign bit for signed integers and floats, else 0
-//   fmask:  all ones for floating point, else 0
-//   dmask:  all ones for descending order, else 0
-template <typename K>
-struct KeyCodec {
-  K sign, fmask, dmask;
-  uint32_t plain;  // all three masks are zero: encode/decode are the identity
-  TA_DEVICE K encode(K k) const {
-    using SK = typename std::make_signed<K>::type;
-    const K neg = (K)((SK)k >> (sizeof(K) * 8 - 1));
-    return k ^ ((neg & fmask) | sign) ^ dmask;
-  }
-  TA_DEVICE K decode(K e) const {
-    using SK = typename std::make_signed<K>::type;
-    e ^= dmask;
-    const K pos = (K)((SK)e >> (sizeof(K) * 8 - 1));
-    return e ^ ((~pos & fmask) | sign);
-  }
 };
 
 struct SortCtl {
@@ -265,9 +245,6 @@ __global__ __launch_bounds__(RADIX_SIZE) void sort_scan_kernel(uint32_t* __restr
 }
 
 // ------------------------------------------------------------------ onesweep pass
-// f(a, b, c) = a & ~(b ^ c): truth table index = a*4 + b*2 + c.
-constexpr int BITOP_AND_XNOR = 0x90;
-
 template <typename K, typename V, bool HAS_VALUES, int BLOCK, int ITEMS>
 struct PassShape {
   static constexpr int WAVES = BLOCK / WAVE;
@@ -400,38 +377,17 @@ __global__ __launch_bounds__(BLOCK) void onesweep_pass_kernel(
   }
 
   // ---- rank inside the wave by digit
-  // Per digit bit: v_bfe_i32 (lane's bit as 0 / -1), one ballot, and two v_bitop3 folding
-  // "same bit as mine" into the 64-bit peer mask.  The wave-private counter is read by every
-  // lane and then raised by the size of the peer group; LDS executes a wave's instructions
-  // in order, so the next round reads the updated count.
   uint32_t* my_cnt = s_cnt + wave * RADIX_SIZE;
   // ranks are < TILE <= 65536: two per register
   static_assert(TILE <= 65536 && ITEMS % 2 == 0, "rank packing");
   uint32_t rank2[ITEMS / 2];
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
-    const uint32_t d = digit_of(e[r]);
-    const uint32_t old = my_cnt[d];
-    uint32_t peers_lo = ~0u, peers_hi = ~0u;
-#pragma unroll
-    for (int b = 0; b < RADIX_BITS; ++b) {
-      int sb;
-      // opaque to the optimiser so that the compare below is made on sb itself
-      asm volatile("v_bfe_i32 %0, %1, %2, 1" : "=v"(sb) : "v"(d), "n"(b));
-      const uint64_t m = __builtin_amdgcn_ballot_w64(sb != 0);
-      peers_lo = __builtin_amdgcn_bitop3_b32(peers_lo, (uint32_t)m, (uint32_t)sb, BITOP_AND_XNOR);
-      peers_hi = __builtin_amdgcn_bitop3_b32(peers_hi, (uint32_t)(m >> 32), (uint32_t)sb, BITOP_AND_XNOR);
-    }
-    // the count of peers in lower lanes is accumulated onto the counter's value
-    const uint32_t rank = __builtin_amdgcn_mbcnt_hi(peers_hi, __builtin_amdgcn_mbcnt_lo(peers_lo, old));
-    // The lowest lane of every group of peers bumps the counter for all of them: one LDS
-    // write per distinct digit instead of an atomic per key, which an LDS bank serialises
-    // when many lanes hold the same digit (float exponents, skewed keys).
-    if (rank == old) my_cnt[d] = old + (uint32_t)__builtin_popcount(peers_lo) + (uint32_t)__builtin_popcount(peers_hi);
+    const uint32_t rank = wave_rank_round(digit_of(e[r]), my_cnt);
     if (r % 2 == 0) rank2[r / 2] = rank;
     else rank2[r / 2] |= rank << 16;
-    // pin the packed rank here: otherwise the add is sunk past the barrier and `old` and
-    // `below` of every round stay live
+    // pin the packed rank here: otherwise the add is sunk past the barrier and its operands
+    // of every round stay live
     asm volatile("" : "+v"(rank2[r / 2]));
     // keep the scheduler from computing all peer masks first (two live registers per
     // round): rounds are finished in pairs
@@ -610,19 +566,6 @@ __global__ __launch_bounds__(256) void sort_copy_back_kernel(K* __restrict__ key
 }
 
 // ------------------------------------------------------------------ host side
-template <typename K>
-static KeyCodec<K> make_codec(int dtype, int descending) {
-  KeyCodec<K> c;
-  const bool is_float = dtype == THRUST_AMD_F32 || dtype == THRUST_AMD_F64;
-  const bool is_signed = is_float || dtype == THRUST_AMD_I8 || dtype == THRUST_AMD_I16 ||
-                         dtype == THRUST_AMD_I32 || dtype == THRUST_AMD_I64;
-  c.sign = is_signed ? (K)((K)1 << (sizeof(K) * 8 - 1)) : (K)0;
-  c.fmask = is_float ? (K)~(K)0 : (K)0;
-  c.dmask = descending ? (K)~(K)0 : (K)0;
-  c.plain = (!is_signed && !descending) ? 1u : 0u;
-  return c;
-}
-
 template <typename K, typename V, bool HAS_VALUES>
 struct SortPlan {
   // Large tiles (16K-18K keys of 4 bytes) keep the number of tiles in flight, and with it
@@ -666,6 +609,8 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   if (*temp_bytes < lay.total) return (int)hipErrorInvalidValue;
   if (n <= 1 || geo.passes == 0) return 0;
   if (!keys || (HAS_VALUES && !values)) return (int)hipErrorInvalidValue;
+  if (n <= SMALL_SORT_MAX)
+    return small_sort(keys, values, (uint32_t)n, dtype, HAS_VALUES ? sizeof(V) : 0, descending, begin_bit, end_bit, stream);
 
   char* base = static_cast<char*>(temp);
   SortCtl* ctl = reinterpret_cast<SortCtl*>(base + off_ctl);
