@@ -20,6 +20,7 @@ NP_DTYPES = {
     U32: np.uint32, I64: np.int64, U64: np.uint64, F32: np.float32, F64: np.float64,
 }
 DTYPE_OF_NP = {np.dtype(v): k for k, v in NP_DTYPES.items()}
+ITEM_SIZES = {k: np.dtype(v).itemsize for k, v in NP_DTYPES.items()}
 DTYPE_NAMES = {I8: "i8", U8: "u8", I16: "i16", U16: "u16", I32: "i32", U32: "u32",
                I64: "i64", U64: "u64", F32: "f32", F64: "f64"}
 # thrust_amd_binop
@@ -133,7 +134,7 @@ class DeviceArray:
         torch = _torch()
         self.n = int(n)
         self.dtype = dtype
-        self.itemsize = np.dtype(NP_DTYPES[dtype]).itemsize
+        self.itemsize = ITEM_SIZES[dtype]
         nbytes = max(self.n * self.itemsize, 16)
         self.storage = storage if storage is not None else torch.empty(
             nbytes, dtype=torch.uint8, device="cuda")
@@ -162,11 +163,27 @@ class DeviceArray:
 
 
 def stream_ptr():
-    return _torch().cuda.current_stream().cuda_stream
+    torch = _torch()
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None:  # the handle itself: 0.3 us, where building a Stream object around it takes 3
+        return raw(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
-def _scalar(dtype, value):
-    return np.array([value], dtype=NP_DTYPES[dtype])
+_ZERO = np.zeros(1, dtype=np.uint64)  # the zero of every dtype; read only
+_ZERO_PTR = _ZERO.ctypes.data
+
+
+class _Scalar:
+    """One value of a dtype in host memory; `ptr` is its address while this object lives."""
+    __slots__ = ("ptr", "_keep")
+
+    def __init__(self, dtype, value):
+        if type(value) is int and value == 0:
+            self._keep, self.ptr = _ZERO, _ZERO_PTR
+        else:
+            self._keep = np.array([value], dtype=NP_DTYPES[dtype])
+            self.ptr = self._keep.ctypes.data
 
 
 class Temp:
@@ -188,11 +205,23 @@ class Temp:
 
 
 def _run(fn_name, temp, call):
-    lib = load()
-    fn = getattr(lib, fn_name)
+    """The two-phase protocol.  A buffer that an earlier call left in `temp` is offered as it is: an entry point
+    refuses one that is too small before it launches anything, and only then is the size asked for."""
+    fn = getattr(_lib or load(), fn_name)
+    stream = stream_ptr()
     temp = temp or Temp()
-    tptr = temp.ensure(lambda t, b: call(fn, t, b))
-    check(call(fn, tptr, ctypes.byref(temp.bytes)), fn_name)
+    if temp.buf is not None:
+        held = temp.buf.numel()
+        temp.bytes.value = held
+        status = call(fn, temp.buf.data_ptr(), ctypes.byref(temp.bytes), stream)
+        if status == 0:
+            return temp
+        tptr = temp.ensure(lambda t, b: call(fn, t, b, stream))
+        if temp.buf.numel() == held:  # it was large enough: the call failed for another reason
+            check(status, fn_name)
+    else:
+        tptr = temp.ensure(lambda t, b: call(fn, t, b, stream))
+    check(call(fn, tptr, ctypes.byref(temp.bytes), stream), fn_name)
     return temp
 
 
@@ -215,9 +244,9 @@ def profile_collect():
 
 def reduce(x, op=PLUS, init=0, temp=None, out=None):
     out = out or DeviceArray(1, x.dtype)
-    iv = _scalar(x.dtype, init)
-    _run("thrust_amd_reduce", temp, lambda fn, t, b: fn(
-        t, b, x.ptr, x.n, x.dtype, op, iv.ctypes.data, out.ptr, stream_ptr()))
+    iv = _Scalar(x.dtype, init)
+    _run("thrust_amd_reduce", temp, lambda fn, t, b, stream: fn(
+        t, b, x.ptr, x.n, x.dtype, op, iv.ptr, out.ptr, stream))
     return out
 
 
@@ -229,39 +258,39 @@ def convert(x, out_dtype, out=None):
 
 def sequence(n, dtype, init=0, step=1, out=None):
     out = out or DeviceArray(n, dtype)
-    iv, sv = _scalar(dtype, init), _scalar(dtype, step)
-    check(load().thrust_amd_sequence(out.ptr, n, dtype, iv.ctypes.data, sv.ctypes.data, stream_ptr()), "thrust_amd_sequence")
+    iv, sv = _Scalar(dtype, init), _Scalar(dtype, step)
+    check(load().thrust_amd_sequence(out.ptr, n, dtype, iv.ptr, sv.ptr, stream_ptr()), "thrust_amd_sequence")
     return out
 
 
 def transform_reduce(x, unary, op=PLUS, init=0, temp=None, out=None):
     out = out or DeviceArray(1, x.dtype)
-    iv = _scalar(x.dtype, init)
-    _run("thrust_amd_transform_reduce", temp, lambda fn, t, b: fn(
-        t, b, x.ptr, x.n, x.dtype, unary, op, iv.ctypes.data, out.ptr, stream_ptr()))
+    iv = _Scalar(x.dtype, init)
+    _run("thrust_amd_transform_reduce", temp, lambda fn, t, b, stream: fn(
+        t, b, x.ptr, x.n, x.dtype, unary, op, iv.ptr, out.ptr, stream))
     return out
 
 
 def count_if(x, cmp, threshold=0, temp=None, read_count=True):
     num = DeviceArray(1, U64)
-    tv = _scalar(x.dtype, threshold)
-    _run("thrust_amd_count_if", temp, lambda fn, t, b: fn(
-        t, b, x.ptr, x.n, x.dtype, cmp, tv.ctypes.data, num.ptr, stream_ptr()))
+    tv = _Scalar(x.dtype, threshold)
+    _run("thrust_amd_count_if", temp, lambda fn, t, b, stream: fn(
+        t, b, x.ptr, x.n, x.dtype, cmp, tv.ptr, num.ptr, stream))
     return _count(num, read_count)
 
 
 def inner_product(a, b_, init=0, temp=None, out=None):
     out = out or DeviceArray(1, a.dtype)
-    iv = _scalar(a.dtype, init)
-    _run("thrust_amd_inner_product", temp, lambda fn, t, b: fn(
-        t, b, a.ptr, b_.ptr, a.n, a.dtype, iv.ctypes.data, out.ptr, stream_ptr()))
+    iv = _Scalar(a.dtype, init)
+    _run("thrust_amd_inner_product", temp, lambda fn, t, b, stream: fn(
+        t, b, a.ptr, b_.ptr, a.n, a.dtype, iv.ptr, out.ptr, stream))
     return out
 
 
 def inclusive_scan(x, out=None, op=PLUS, temp=None):
     out = out or DeviceArray(x.n, x.dtype)
-    _run("thrust_amd_inclusive_scan", temp, lambda fn, t, b: fn(
-        t, b, x.ptr, out.ptr, x.n, x.dtype, op, stream_ptr()))
+    _run("thrust_amd_inclusive_scan", temp, lambda fn, t, b, stream: fn(
+        t, b, x.ptr, out.ptr, x.n, x.dtype, op, stream))
     return out
 
 
@@ -275,65 +304,65 @@ def inclusive_scan_static(x, out=None, op=PLUS):
 
 def exclusive_scan(x, init=0, out=None, op=PLUS, temp=None):
     out = out or DeviceArray(x.n, x.dtype)
-    iv = _scalar(x.dtype, init)
-    _run("thrust_amd_exclusive_scan", temp, lambda fn, t, b: fn(
-        t, b, x.ptr, out.ptr, x.n, x.dtype, op, iv.ctypes.data, stream_ptr()))
+    iv = _Scalar(x.dtype, init)
+    _run("thrust_amd_exclusive_scan", temp, lambda fn, t, b, stream: fn(
+        t, b, x.ptr, out.ptr, x.n, x.dtype, op, iv.ptr, stream))
     return out
 
 
 def transform_inclusive_scan(x, unary, out=None, op=PLUS, temp=None):
     out = out or DeviceArray(x.n, x.dtype)
-    _run("thrust_amd_transform_inclusive_scan", temp, lambda fn, t, b: fn(
-        t, b, x.ptr, out.ptr, x.n, x.dtype, unary, op, stream_ptr()))
+    _run("thrust_amd_transform_inclusive_scan", temp, lambda fn, t, b, stream: fn(
+        t, b, x.ptr, out.ptr, x.n, x.dtype, unary, op, stream))
     return out
 
 
 def transform_exclusive_scan(x, unary, init=0, out=None, op=PLUS, temp=None):
     out = out or DeviceArray(x.n, x.dtype)
-    iv = _scalar(x.dtype, init)
-    _run("thrust_amd_transform_exclusive_scan", temp, lambda fn, t, b: fn(
-        t, b, x.ptr, out.ptr, x.n, x.dtype, unary, op, iv.ctypes.data, stream_ptr()))
+    iv = _Scalar(x.dtype, init)
+    _run("thrust_amd_transform_exclusive_scan", temp, lambda fn, t, b, stream: fn(
+        t, b, x.ptr, out.ptr, x.n, x.dtype, unary, op, iv.ptr, stream))
     return out
 
 
 def inclusive_scan_by_key(keys, values, op=PLUS, out=None, temp=None):
     out = out or DeviceArray(values.n, values.dtype)
-    _run("thrust_amd_inclusive_scan_by_key", temp, lambda fn, t, b: fn(
-        t, b, keys.ptr, values.ptr, out.ptr, keys.n, keys.dtype, values.dtype, op, stream_ptr()))
+    _run("thrust_amd_inclusive_scan_by_key", temp, lambda fn, t, b, stream: fn(
+        t, b, keys.ptr, values.ptr, out.ptr, keys.n, keys.dtype, values.dtype, op, stream))
     return out
 
 
 def exclusive_scan_by_key(keys, values, init=0, op=PLUS, out=None, temp=None):
     out = out or DeviceArray(values.n, values.dtype)
-    iv = _scalar(values.dtype, init)
-    _run("thrust_amd_exclusive_scan_by_key", temp, lambda fn, t, b: fn(
-        t, b, keys.ptr, values.ptr, out.ptr, keys.n, keys.dtype, values.dtype, op, iv.ctypes.data,
-        stream_ptr()))
+    iv = _Scalar(values.dtype, init)
+    _run("thrust_amd_exclusive_scan_by_key", temp, lambda fn, t, b, stream: fn(
+        t, b, keys.ptr, values.ptr, out.ptr, keys.n, keys.dtype, values.dtype, op, iv.ptr,
+        stream))
     return out
 
 
 def sort_keys(keys, descending=False, begin_bit=0, end_bit=None, temp=None):
     end_bit = keys.itemsize * 8 if end_bit is None else end_bit
-    return _run("thrust_amd_sort_keys", temp, lambda fn, t, b: fn(
-        t, b, keys.ptr, keys.n, keys.dtype, int(descending), begin_bit, end_bit, stream_ptr()))
+    return _run("thrust_amd_sort_keys", temp, lambda fn, t, b, stream: fn(
+        t, b, keys.ptr, keys.n, keys.dtype, int(descending), begin_bit, end_bit, stream))
 
 
 def sort_pairs(keys, values, descending=False, begin_bit=0, end_bit=None, temp=None):
     end_bit = keys.itemsize * 8 if end_bit is None else end_bit
-    return _run("thrust_amd_sort_pairs", temp, lambda fn, t, b: fn(
+    return _run("thrust_amd_sort_pairs", temp, lambda fn, t, b, stream: fn(
         t, b, keys.ptr, values.ptr, keys.n, keys.dtype, values.itemsize, int(descending),
-        begin_bit, end_bit, stream_ptr()))
+        begin_bit, end_bit, stream))
 
 
 def merge_sort_keys(keys, descending=False, temp=None):
     """Stable comparison sort in place (operator< / operator>)."""
-    return _run("thrust_amd_merge_sort_keys", temp, lambda fn, t, b: fn(
-        t, b, keys.ptr, keys.n, keys.dtype, int(descending), stream_ptr()))
+    return _run("thrust_amd_merge_sort_keys", temp, lambda fn, t, b, stream: fn(
+        t, b, keys.ptr, keys.n, keys.dtype, int(descending), stream))
 
 
 def merge_sort_pairs(keys, values, descending=False, temp=None):
-    return _run("thrust_amd_merge_sort_pairs", temp, lambda fn, t, b: fn(
-        t, b, keys.ptr, values.ptr, keys.n, keys.dtype, values.itemsize, int(descending), stream_ptr()))
+    return _run("thrust_amd_merge_sort_pairs", temp, lambda fn, t, b, stream: fn(
+        t, b, keys.ptr, values.ptr, keys.n, keys.dtype, values.itemsize, int(descending), stream))
 
 
 def _count(dev_u64, read=True):
@@ -346,10 +375,10 @@ def copy_if(x, cmp, threshold=0, stencil=None, out=None, temp=None, read_count=T
     out = out or DeviceArray(x.n, x.dtype)
     num = DeviceArray(1, U64)
     tested = stencil if stencil is not None else x
-    tv = _scalar(tested.dtype, threshold)
-    _run("thrust_amd_copy_if", temp, lambda fn, t, b: fn(
+    tv = _Scalar(tested.dtype, threshold)
+    _run("thrust_amd_copy_if", temp, lambda fn, t, b, stream: fn(
         t, b, x.ptr, stencil.ptr if stencil is not None else None, out.ptr, num.ptr, x.n,
-        x.itemsize, tested.dtype, cmp, tv.ctypes.data, stream_ptr()))
+        x.itemsize, tested.dtype, cmp, tv.ptr, stream))
     return out, _count(num, read_count)
 
 
@@ -357,28 +386,28 @@ def partition_copy(x, cmp, threshold=0, stencil=None, temp=None, read_count=True
     out_t, out_f = DeviceArray(x.n, x.dtype), DeviceArray(x.n, x.dtype)
     num = DeviceArray(1, U64)
     tested = stencil if stencil is not None else x
-    tv = _scalar(tested.dtype, threshold)
-    _run("thrust_amd_partition_copy", temp, lambda fn, t, b: fn(
+    tv = _Scalar(tested.dtype, threshold)
+    _run("thrust_amd_partition_copy", temp, lambda fn, t, b, stream: fn(
         t, b, x.ptr, stencil.ptr if stencil is not None else None, out_t.ptr, out_f.ptr, num.ptr,
-        x.n, x.itemsize, tested.dtype, cmp, tv.ctypes.data, stream_ptr()))
+        x.n, x.itemsize, tested.dtype, cmp, tv.ptr, stream))
     return out_t, out_f, _count(num, read_count)
 
 
 def stable_partition(x, cmp, threshold=0, stencil=None, temp=None, read_count=True):
     num = DeviceArray(1, U64)
     tested = stencil if stencil is not None else x
-    tv = _scalar(tested.dtype, threshold)
-    _run("thrust_amd_stable_partition", temp, lambda fn, t, b: fn(
+    tv = _Scalar(tested.dtype, threshold)
+    _run("thrust_amd_stable_partition", temp, lambda fn, t, b, stream: fn(
         t, b, x.ptr, stencil.ptr if stencil is not None else None, num.ptr, x.n, x.itemsize,
-        tested.dtype, cmp, tv.ctypes.data, stream_ptr()))
+        tested.dtype, cmp, tv.ptr, stream))
     return _count(num, read_count)
 
 
 def unique(x, out=None, temp=None, read_count=True):
     out = out or DeviceArray(x.n, x.dtype)
     num = DeviceArray(1, U64)
-    _run("thrust_amd_unique", temp, lambda fn, t, b: fn(
-        t, b, x.ptr, out.ptr, num.ptr, x.n, x.dtype, stream_ptr()))
+    _run("thrust_amd_unique", temp, lambda fn, t, b, stream: fn(
+        t, b, x.ptr, out.ptr, num.ptr, x.n, x.dtype, stream))
     return out, _count(num, read_count)
 
 
@@ -386,9 +415,9 @@ def unique_by_key(keys, values, keys_out=None, values_out=None, temp=None, read_
     keys_out = keys_out or DeviceArray(keys.n, keys.dtype)
     values_out = values_out or DeviceArray(values.n, values.dtype)
     num = DeviceArray(1, U64)
-    _run("thrust_amd_unique_by_key", temp, lambda fn, t, b: fn(
+    _run("thrust_amd_unique_by_key", temp, lambda fn, t, b, stream: fn(
         t, b, keys.ptr, values.ptr, keys_out.ptr, values_out.ptr, num.ptr, keys.n, keys.dtype,
-        values.itemsize, stream_ptr()))
+        values.itemsize, stream))
     return keys_out, values_out, _count(num, read_count)
 
 
@@ -396,16 +425,16 @@ def reduce_by_key(keys, values, op=PLUS, temp=None, keys_out=None, values_out=No
     keys_out = keys_out or DeviceArray(keys.n, keys.dtype)
     values_out = values_out or DeviceArray(values.n, values.dtype)
     num = DeviceArray(1, U64)
-    _run("thrust_amd_reduce_by_key", temp, lambda fn, t, b: fn(
+    _run("thrust_amd_reduce_by_key", temp, lambda fn, t, b, stream: fn(
         t, b, keys.ptr, values.ptr, keys_out.ptr, values_out.ptr, num.ptr, keys.n, keys.dtype,
-        values.dtype, op, stream_ptr()))
+        values.dtype, op, stream))
     return keys_out, values_out, _count(num, read_count)
 
 
 def merge(a, b_, descending=False, out=None, temp=None):
     out = out or DeviceArray(a.n + b_.n, a.dtype)
-    _run("thrust_amd_merge", temp, lambda fn, t, b: fn(
-        t, b, a.ptr, a.n, b_.ptr, b_.n, out.ptr, a.dtype, int(descending), stream_ptr()))
+    _run("thrust_amd_merge", temp, lambda fn, t, b, stream: fn(
+        t, b, a.ptr, a.n, b_.ptr, b_.n, out.ptr, a.dtype, int(descending), stream))
     return out
 
 
@@ -413,8 +442,8 @@ def set_operation(op, a, b_, descending=False, out=None, temp=None, read_count=T
     """Returns (out, length); out holds a.n + b.n elements unless the caller passes one."""
     out = out or DeviceArray(a.n + b_.n, a.dtype)
     num = DeviceArray(1, U64)
-    _run("thrust_amd_set_operation", temp, lambda fn, t, b: fn(
-        t, b, op, a.ptr, a.n, b_.ptr, b_.n, out.ptr, num.ptr, a.dtype, int(descending), stream_ptr()))
+    _run("thrust_amd_set_operation", temp, lambda fn, t, b, stream: fn(
+        t, b, op, a.ptr, a.n, b_.ptr, b_.n, out.ptr, num.ptr, a.dtype, int(descending), stream))
     return out, _count(num, read_count)
 
 
@@ -422,16 +451,16 @@ def set_operation_by_key(op, ka, kb, va, vb, descending=False, temp=None, keys_o
     keys_out = keys_out or DeviceArray(ka.n + kb.n, ka.dtype)
     values_out = values_out or DeviceArray(ka.n + kb.n, va.dtype)
     num = DeviceArray(1, U64)
-    _run("thrust_amd_set_operation_by_key", temp, lambda fn, t, b: fn(
+    _run("thrust_amd_set_operation_by_key", temp, lambda fn, t, b, stream: fn(
         t, b, op, ka.ptr, ka.n, kb.ptr, kb.n, va.ptr, vb.ptr if vb is not None else None, keys_out.ptr,
-        values_out.ptr, num.ptr, ka.dtype, va.itemsize, int(descending), stream_ptr()))
+        values_out.ptr, num.ptr, ka.dtype, va.itemsize, int(descending), stream))
     return keys_out, values_out, _count(num, read_count)
 
 
 def merge_by_key(ka, kb, va, vb, descending=False, temp=None, keys_out=None, values_out=None):
     keys_out = keys_out or DeviceArray(ka.n + kb.n, ka.dtype)
     values_out = values_out or DeviceArray(ka.n + kb.n, va.dtype)
-    _run("thrust_amd_merge_by_key", temp, lambda fn, t, b: fn(
+    _run("thrust_amd_merge_by_key", temp, lambda fn, t, b, stream: fn(
         t, b, ka.ptr, ka.n, kb.ptr, kb.n, va.ptr, vb.ptr, keys_out.ptr, values_out.ptr, ka.dtype,
-        va.itemsize, int(descending), stream_ptr()))
+        va.itemsize, int(descending), stream))
     return keys_out, values_out
