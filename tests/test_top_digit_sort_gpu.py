@@ -1,0 +1,72 @@
+"""The sort that runs its passes over the top digits only and orders the stretches of equal prefixes in
+one workgroup each: inputs that take it with one digit and with two, whose bins are too full for counting,
+that make it give up (a stretch too long for a workgroup), and that never take it."""
+import numpy as np
+import pytest
+
+from thrust_amd import datagen
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [8193, 20_001, 300_007, 1_000_003, 2_500_001]
+
+
+def _keys(kind, dtype, n):
+    r = datagen.splitmix64(99, n)
+    bits = np.dtype(dtype).itemsize * 8
+    u = np.uint64
+    if kind == "uniform":
+        k = r
+    elif kind == "repeated":      # the low half takes four values: many equal keys in every stretch
+        k = (r >> u(64 - bits)) & ~u((1 << (bits // 2)) - 1) | (r & u(3))
+    elif kind == "clusters":      # low bits in clusters far apart: the bins of a stretch overflow
+        k = (r >> u(64 - bits)) & ~u((1 << (bits - 16)) - 1) | (r & u(1)) << u(bits - 20) | (r >> u(3)) & u(63)
+    elif kind == "long_stretch":  # uniform but for one prefix held by more keys than a workgroup takes
+        k = r >> u(64 - bits)
+        k[n // 3:n // 3 + 9000] = (k[n // 3:n // 3 + 9000] & u((1 << (bits - 16)) - 1)) | u(0x1234) << u(bits - 16)
+    elif kind == "equal":         # no digit moves
+        k = np.full(n, 12345, dtype=np.uint64)
+    elif kind == "skewed":        # nine in ten equal
+        k = np.where(r % u(10) != 0, u(1 << 20), r)
+    elif kind == "ids":           # 0 .. n-1 shuffled: constant top digits
+        k = np.argsort(r).astype(np.uint64)
+    elif kind == "sorted":
+        k = np.sort(r >> u(64 - bits))
+    if kind == "normal":
+        k = np.random.default_rng(5).standard_normal(n) * 1000
+        return k.astype(dtype) if np.dtype(dtype).kind == "f" else (k * 1000).astype(np.int64).astype(dtype)
+    k = k.astype({32: np.uint32, 64: np.uint64}[bits]).view(dtype)
+    return np.where(np.isnan(k), dtype(1), k) if np.dtype(dtype).kind == "f" else k
+
+
+def _order(x, descending):
+    """Stable order by the radix code."""
+    bits = x.dtype.itemsize * 8
+    u = x.view(f"u{x.dtype.itemsize}")
+    top = u.dtype.type(1 << (bits - 1))
+    if x.dtype.kind == "f":
+        u = np.where(u & top, ~u, u | top)
+    elif x.dtype.kind == "i":
+        u = u ^ top
+    return np.argsort(~u if descending else u, kind="stable")
+
+
+@pytest.mark.parametrize("dtype", [np.uint32, np.int32, np.float32, np.uint64, np.float64])
+@pytest.mark.parametrize("kind", ["uniform", "normal", "repeated", "clusters", "long_stretch", "equal", "skewed", "ids", "sorted"])
+def test_sorts_by_top_digits(dev, dtype, kind):
+    temp = dev.Temp()
+    for n in SIZES:
+        if kind == "long_stretch" and n < 30_000:
+            continue
+        x = _keys(kind, dtype, n)
+        for descending in (False, True):
+            order = _order(x, descending)
+            k = dev.DeviceArray.from_numpy(x)
+            dev.sort_keys(k, descending=descending, temp=temp)
+            assert np.array_equal(k.numpy().view(np.uint8), x[order].view(np.uint8)), (n, descending)
+            for vdtype in (np.uint8, np.uint32, np.uint64) if n < 1_000_000 else (np.uint32,):
+                v = np.arange(n).astype(vdtype)
+                k, w = dev.DeviceArray.from_numpy(x), dev.DeviceArray.from_numpy(v)
+                dev.sort_pairs(k, w, descending=descending, temp=temp)
+                assert np.array_equal(k.numpy().view(np.uint8), x[order].view(np.uint8)), (n, vdtype, descending)
+                assert np.array_equal(w.numpy(), v[order]), (n, vdtype, descending)

@@ -1,0 +1,442 @@
+// The last step of a radix sort whose passes covered the top digits only: the array is in stable order of a
+// prefix of the keys, and every stretch of equal prefixes is short enough to be ordered in one workgroup.
+//
+//   bounds  for every window of `window` positions the first place at or behind its start where a new prefix
+//           begins.  A stretch that reaches further than CAP - window past the edge it crosses raises
+//           SortCtl::failed, and the chained passes sort the array as if nothing had happened (it holds the same
+//           keys, equal ones in their original order).
+//   finish  a workgroup takes the stretches that begin inside its window (at most CAP keys), orders them by the
+//           whole key in registers and LDS and writes them to their place in the caller's array.
+//
+// Inside a workgroup the keys go to as many bins as there are places (key minus smallest key, shifted so that the
+// largest falls into the last bins): one LDS atomic per key counts a bin and tells the key its place in it, a scan
+// turns counts into starts, the keys are laid out by bin, and each key counts the keys of its bin that belong in front
+// of it -- the smaller ones and, among equal ones, those that stood in front -- so the atomics' order does not show.
+// What bounds it: vector instructions (90 per key and lane) and, for 2000 keys a workgroup, the latency of its ten
+// steps; LDS is busy 40 % of the time.  2^28 uint32: 0.93 ms (2.3 TB/s) in place of two passes of 0.50; 2^27 (uint64,
+// uint32): 0.85 ms (3.8 TB/s) in place of six of 0.65.  Measured on the way: comparing inside the bins place by place 1.39
+// ms, with lanes that hold neighbouring places 1.98 (bank conflicts), 512 threads with 16 keys each and spilled
+// registers 1.30.  Workgroups that loop over windows save their dispatch where the chained passes do the sort (112 us for
+// 2^28 keys), but cost 8-byte keys registers (0.85 -> 1.19 ms).
+// A bin of more than FINISH_BIN_MAX keys (many equal keys, values in clusters) makes the workgroup run stable passes
+// over the digits that vary instead.
+#pragma once
+#include "common.hpp"
+#include "launch.hpp"
+#include "radix_rank.hpp"
+#include "sort_codec.hpp"
+
+namespace ta {
+
+constexpr int MAX_PASSES = 8;
+constexpr int TOP_SLOTS = 2;                       // passes in front of the last step, at most
+constexpr int MAX_SLOTS = TOP_SLOTS + MAX_PASSES;  // pass launches of a sort
+
+// What the launches of a sort do, decided on the device from the histograms.  A sort through all digits uses as
+// many slots as it has digits, whatever their number; one that takes the short way its first TOP_SLOTS, and the
+// others only if the bounds kernel finds a stretch that does not fit.
+struct SortCtl {
+  enum : uint32_t { SKIP, RUN, IF_FAILED };
+  uint32_t slot[MAX_SLOTS];      // action, digit, source buffer, whether it encodes / decodes the keys
+  uint32_t final_in_alt;         // result sits in the alternate buffer after the last slot,
+  uint32_t final_in_alt_failed;  // ... if the short way failed
+  uint32_t gave_up;              // a tile stopped waiting for its predecessors (see LOOKBACK_SPIN_LIMIT)
+  uint32_t fast;                 // the short way is taken, with this many digits
+  uint32_t failed;               // ... and was given up
+  uint32_t fast_src_alt;         // the last step reads the alternate buffer
+  uint32_t prefix_bit;           // lowest bit of the digits the array is ordered by then
+  uint32_t window;               // positions per workgroup of the last step
+
+  static TA_DEVICE uint32_t pack(uint32_t action, uint32_t digit, uint32_t src_alt, bool encodes, bool decodes) {
+    return action | digit << 4 | src_alt << 8 | (encodes ? 1u << 9 : 0u) | (decodes ? 1u << 10 : 0u);
+  }
+  static TA_DEVICE bool runs(uint32_t s, uint32_t failed) { return (s & 15u) == RUN || ((s & 15u) == IF_FAILED && failed != 0); }
+  static TA_DEVICE uint32_t digit(uint32_t s) { return s >> 4 & 15u; }
+  static TA_DEVICE bool src_alt(uint32_t s) { return (s >> 8 & 1u) != 0; }
+  static TA_DEVICE bool encodes(uint32_t s) { return (s >> 9 & 1u) != 0; }
+  static TA_DEVICE bool decodes(uint32_t s) { return (s >> 10 & 1u) != 0; }
+};
+
+constexpr uint32_t FINISH_BIN_MAX = 24;
+constexpr uint64_t FINISH_BLOCKS_MAX = NUM_CU * 4;  // workgroups without a window cost their dispatch
+
+template <typename K, typename V, bool HAS_VALUES>
+struct FinishShape {
+  static constexpr bool BIG = sizeof(K) == 8 || (HAS_VALUES && sizeof(V) == 8);
+  static constexpr int BLOCK = BIG ? 512 : 1024;
+  static constexpr int ITEMS = 8;
+  static constexpr int CAP = BLOCK * ITEMS;
+  static constexpr int WAVES_PER_SIMD = (BIG ? 3 : 2) * BLOCK / WAVE / 4;
+  static constexpr bool LOOPS = !BIG;  // a workgroup takes one window after the other
+  static constexpr uint32_t WINDOW_MIN = BIG ? 1536 : 2048;
+  static constexpr uint32_t STRETCH_MAX = CAP - WINDOW_MIN;  // longest stretch of one prefix that can be promised a place
+};
+
+// window: see above; sorted: the array in order of its keys' bits from prefix_bit on; bounds[ceil(n / window) + 1]
+template <typename K>
+__global__ __launch_bounds__(256) void sort_bounds_kernel(const K* __restrict__ keys_a, const K* __restrict__ keys_b, uint32_t n,
+                                                          uint32_t cap, uint32_t* __restrict__ bounds, const SortCtl* __restrict__ ctl,
+                                                          uint32_t* __restrict__ failed) {
+  if (!ctl->fast) return;
+  const uint32_t window = ctl->window;
+  const uint32_t windows = (n + window - 1) / window;
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i > windows) return;
+  if (i == 0 || i == windows) {
+    bounds[i] = i == 0 ? 0 : n;
+    return;
+  }
+  const K* __restrict__ x = ctl->fast_src_alt ? keys_b : keys_a;
+  const int bit = (int)ctl->prefix_bit;
+  const uint32_t edge = i * window;
+  const uint32_t reach = cap - window;  // a new prefix has to begin at edge + reach at the latest
+  const K here = x[edge - 1] >> bit;
+  uint32_t lo = edge, hi = n - edge < reach ? n : edge + reach;  // the answer lies in [lo, hi]
+  if (hi < n && (x[hi] >> bit) == here) {
+    __hip_atomic_store(failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bounds[i] = edge;
+    return;
+  }
+  while (lo < hi) {
+    const uint32_t mid = lo + (hi - lo) / 2;
+    if ((x[mid] >> bit) == here) lo = mid + 1;
+    else hi = mid;
+  }
+  bounds[i] = lo;
+}
+
+// Inclusive sum over each row of 16 lanes.
+TA_DEVICE uint32_t row_inclusive_scan(uint32_t x) {
+  x += dpp_move<DPP_ROW_SHR1>(0u, x);
+  x += dpp_move<DPP_ROW_SHR2>(0u, x);
+  x += dpp_move<DPP_ROW_SHR4>(0u, x);
+  x += dpp_move<DPP_ROW_SHR8>(0u, x);
+  return x;
+}
+
+template <typename K, typename V, bool HAS_VALUES>
+__global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShape<K, V, HAS_VALUES>::WAVES_PER_SIMD)) void sort_finish_kernel(
+    K* __restrict__ keys_a, const K* __restrict__ keys_b, V* __restrict__ vals_a, const V* __restrict__ vals_b, uint32_t n,
+    KeyCodec<K> codec, const uint32_t* __restrict__ bounds, const SortCtl* __restrict__ ctl, uint32_t* __restrict__ status,
+    uint64_t status_words) {
+  using Shape = FinishShape<K, V, HAS_VALUES>;
+  constexpr int BLOCK = Shape::BLOCK, ITEMS = Shape::ITEMS, CAP = Shape::CAP, WAVES = BLOCK / WAVE;
+  constexpr bool BIG = Shape::BIG;
+  constexpr int BINS = CAP;                // 16-bit counts, two to a word
+  constexpr int BIN_WORDS = BINS / 2;
+  constexpr int LOG_BINS = __builtin_ctz(BINS);
+  constexpr int MY_WORDS = BIN_WORDS / BLOCK;
+  constexpr int TRASH = 32;
+  constexpr int GROUP = 2;                 // rounds without a branch between them
+  constexpr int SIDE = 7;                  // places looked at on either side of a key
+  // 8-byte keys are told apart by 32 bits; they are then moved like values, by the 16-bit place they had before
+  constexpr bool KEYS_MOVE = sizeof(K) == 8;
+  constexpr bool HAS_IDX = KEYS_MOVE || HAS_VALUES;
+  constexpr size_t ITEM = (HAS_VALUES && sizeof(V) > sizeof(K)) ? sizeof(V) : sizeof(K);
+  constexpr size_t CODE_BYTES = (CAP + 2 * (SIDE + 1)) * sizeof(uint32_t);
+  constexpr size_t FRONT_BYTES = CODE_BYTES > CAP * ITEM ? CODE_BYTES : CAP * ITEM;
+  static_assert(BLOCK >= RADIX_SIZE && (CAP & (CAP - 1)) == 0 && CAP <= 8192 && MY_WORDS % 4 == 0, "shape");
+  static_assert(ITEMS % GROUP == 0, "groups");
+  static_assert(WAVES * RADIX_SIZE <= BIN_WORDS, "the passes' counters lie over the bins");
+
+  if (!ctl->fast || ctl->failed) {
+    // the chained passes do the sort: their tile descriptors are cleared here, not by every call's first kernel
+    const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
+    for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < status_words; i += stride) status[i] = 0;
+    return;
+  }
+  const uint32_t window = ctl->window;
+  const uint32_t windows = (n + window - 1) / window;
+  __shared__ __attribute__((aligned(16))) unsigned char s_items[FRONT_BYTES];
+  __shared__ uint16_t s_idx[HAS_IDX ? CAP : 1];
+  __shared__ __attribute__((aligned(16))) uint32_t s_bin[BIN_WORDS + 4 + TRASH];  // behind the bins: where lanes without a key count
+  __shared__ uint32_t s_wave[WAVES];
+  __shared__ uint32_t s_digit_wave[RADIX_SIZE / WAVE];
+  __shared__ K s_differ[WAVES];
+  __shared__ uint32_t s_most;
+  uint32_t* s_code = reinterpret_cast<uint32_t*>(s_items) + SIDE + 1;
+  K* s_keys = reinterpret_cast<K*>(s_items);
+  V* s_vals = reinterpret_cast<V*>(s_items);
+
+  for (uint32_t w = blockIdx.x; w < windows; w = Shape::LOOPS ? w + gridDim.x : windows) {
+  const uint32_t first = bounds[w];
+  const uint32_t count = bounds[w + 1] - first;
+  if (count == 0 || count > (uint32_t)CAP) continue;
+  if (Shape::LOOPS) __syncthreads();  // the window before is done with the LDS
+  uint32_t tid = threadIdx.x;
+  if (Shape::LOOPS) asm volatile("" : "+v"(tid));  // nothing derived from it is kept from window to window
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+  const int rounds = (int)((count + BLOCK - 1) / BLOCK);
+  const K* __restrict__ keys_in = (ctl->fast_src_alt ? keys_b : keys_a) + first;
+  const V* __restrict__ vals_in = HAS_VALUES ? (ctl->fast_src_alt ? vals_b : vals_a) + first : nullptr;
+  K* __restrict__ keys_out = keys_a + first;
+  V* __restrict__ vals_out = HAS_VALUES ? vals_a + first : nullptr;
+  // f(r, the place r * BLOCK + tid) for all rounds, in groups of straight-line code: a branch per round makes the
+  // compiler wait for each round's loads before the next one's
+  // (opaque copy: what a sweep derives from the place is not kept in registers for the next)
+  auto each_round = [&](auto f) {
+    uint32_t t = tid;
+    asm volatile("" : "+v"(t));
+#pragma unroll
+    for (int g = 0; g < ITEMS; g += GROUP) {
+      if (g < rounds) {
+#pragma unroll
+        for (int r = g; r < g + GROUP; ++r) f(r, (uint32_t)r * BLOCK + t);
+      }
+    }
+  };
+
+  // ---- load; lanes without a key repeat the last one
+  K e[ITEMS];
+  V v[HAS_VALUES ? ITEMS : 1];
+  each_round([&](int r, uint32_t p) { e[r] = keys_in[p < count ? p : count - 1]; });
+  auto load_values = [&] {
+    each_round([&](int r, uint32_t p) { v[r] = vals_in[p < count ? p : count - 1]; });
+  };
+  if constexpr (HAS_VALUES && BIG) load_values();
+  // the prefixes are in order, so the first and the last one say where all keys lie
+  const int prefix_bit = (int)ctl->prefix_bit;
+  const K lo = keys_in[0] >> prefix_bit << prefix_bit;
+  const K range = (keys_in[count - 1] | (((K)1 << prefix_bit) - 1)) - lo;
+  const int width = 64 - __builtin_clzll((uint64_t)range);  // prefix_bit >= 8
+  const int shift = width > LOG_BINS ? width - LOG_BINS : 0;
+  // what tells keys apart, in 32 bits, and a key's bin from that
+  const int code_shift = KEYS_MOVE && width > 32 ? width - 32 : 0;
+  const int bin_shift = shift - code_shift;
+  auto decoded = [&](K x) { return codec.plain ? x : codec.decode(x); };  // (uniform)
+  auto code_of = [&](K x) { return (uint32_t)((K)(x - lo) >> code_shift); };
+#pragma unroll
+  for (int i = 0; i < MY_WORDS / 4; ++i) reinterpret_cast<uint4*>(s_bin)[(uint32_t)i * BLOCK + tid] = uint4{0, 0, 0, 0};
+  if (tid == 0) s_most = 4;
+  __syncthreads();
+
+  // ---- bins
+  uint32_t slot[ITEMS];
+  auto forget = [](K& x) { asm volatile("" : "+v"(x)); };  // ... nor what it derives from a key
+  each_round([&](int r, uint32_t p) {
+    const uint32_t b = code_of(e[r]) >> bin_shift;
+    const uint32_t word = p < count ? b >> 1 : (uint32_t)(BIN_WORDS + 4) + lane % TRASH;
+    slot[r] = __hip_atomic_fetch_add(&s_bin[word], (b & 1u) ? 1u << 16 : 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    forget(e[r]);
+  });
+  __syncthreads();
+  {
+    typedef uint16_t Two __attribute__((ext_vector_type(2)));
+    uint32_t c[MY_WORDS];
+#pragma unroll
+    for (int i = 0; i < MY_WORDS / 4; ++i) *reinterpret_cast<uint4*>(c + 4 * i) = reinterpret_cast<const uint4*>(s_bin)[tid * (MY_WORDS / 4) + i];
+    uint32_t sums = 0;  // no half exceeds the number of keys
+    Two most2 = {0, 0};
+#pragma unroll
+    for (int i = 0; i < MY_WORDS; ++i) {
+      sums += c[i];
+      most2 = __builtin_elementwise_max(most2, __builtin_bit_cast(Two, c[i]));
+    }
+    const uint32_t sum = (sums & 0xffffu) + (sums >> 16);
+    const uint32_t most = most2.x > most2.y ? most2.x : most2.y;
+    if (most > 4) atomicMax(&s_most, most);  // few lanes
+    const uint32_t incl = wave_inclusive_scan(sum, OpPlus{});
+    if (lane == WAVE - 1) s_wave[wave] = incl;
+    __syncthreads();
+    static_assert(WAVES <= 16, "one DPP row holds the waves' sums");
+    const uint32_t before = row_inclusive_scan(s_wave[lane % WAVES]);
+    uint32_t at = incl - sum + (wave > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)before, __builtin_amdgcn_readfirstlane(wave - 1) & (WAVES - 1)) : 0u);
+    at |= at << 16;
+#pragma unroll
+    for (int i = 0; i < MY_WORDS; ++i) {
+      const uint32_t both = c[i] + __builtin_amdgcn_alignbit(c[i], c[i], 16);  // in either half
+      c[i] = at + (c[i] << 16);
+      at += both;
+    }
+#pragma unroll
+    for (int i = 0; i < MY_WORDS / 4; ++i) reinterpret_cast<uint4*>(s_bin)[tid * (MY_WORDS / 4) + i] = *reinterpret_cast<const uint4*>(c + 4 * i);
+  }
+  __syncthreads();
+
+  const uint32_t most = s_most;  // keys in the fullest bin, or 4
+  if (most <= FINISH_BIN_MAX) {
+    const uint16_t* s_start = reinterpret_cast<const uint16_t*>(s_bin);
+    each_round([&](int r, uint32_t) {
+      const uint32_t b = code_of(e[r]) >> bin_shift;
+      slot[r] = ((b & 1u) ? slot[r] >> 16 : slot[r] & 0xffffu) + s_start[b];
+      forget(e[r]);
+    });
+    each_round([&](int r, uint32_t p) {
+      if (p < count) {
+        s_code[slot[r]] = code_of(e[r]);
+        if constexpr (HAS_IDX) s_idx[slot[r]] = (uint16_t)p;
+      }
+    });
+    if (tid < SIDE) {  // what lies outside belongs outside
+      s_code[-1 - (int)tid] = 0;
+      s_code[count + tid] = ~0u;
+    }
+    __syncthreads();
+    if constexpr (HAS_VALUES && !BIG) load_values();  // not earlier: the registers hold the keys until here
+    // ---- inside the bins: keys of lower bins are smaller and lie in front, so a lane counts the keys on the wrong
+    // side of its own, without asking for their bins, as far as the fullest bin can reach.  4-byte keys leave
+    // straight for their places: a wave's lie next to each other but for those steps.
+    uint32_t move[HAS_IDX ? ITEMS : 1];  // place now, and in the workgroup before << 16
+    auto settle = [&](auto side, bool by_place) {
+      auto place = [&](uint32_t p, uint32_t& packed) {
+        const uint32_t mine = s_code[p];
+        const uint32_t my_idx = HAS_IDX ? s_idx[p] : 0u;
+        uint32_t q = p;
+        bool equal = false;
+#pragma unroll
+        for (int j = 1; j <= side(); ++j) {
+          const uint32_t left = s_code[(int)p - j], right = s_code[(int)p + j];
+          q -= left > mine ? 1u : 0u;
+          q += right < mine ? 1u : 0u;
+          if constexpr (HAS_IDX) equal = equal || left == mine || right == mine;
+        }
+        if (p < count) {
+          if (by_place || equal) {
+            // equal codes: by the whole key where the code is not all of it, and then in the order before
+            auto in_front = [&](uint32_t j) {  // does place j's key belong in front of this one
+              const uint32_t x = s_code[j];
+              if (x != mine || !HAS_IDX) return x < mine || (x == mine && j < p);
+              const uint32_t i = s_idx[j];
+              if constexpr (KEYS_MOVE) {
+                const K a = keys_in[i], b = keys_in[my_idx];
+                if (a != b) return a < b;
+              }
+              return i < my_idx;
+            };
+            const uint32_t from = p > most ? p - most : 0, to = p + most < count ? p + most : count;
+            q = from;
+            for (uint32_t j = from; j < to; ++j) q += j != p && in_front(j) ? 1u : 0u;
+          }
+          if constexpr (!KEYS_MOVE) keys_out[q] = decoded((K)(lo + mine));
+        }
+        packed = q | my_idx << 16;
+      };
+      if constexpr (HAS_IDX) {
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+          if (r < rounds) place((uint32_t)r * BLOCK + tid, move[r]);
+        }
+      } else {
+        uint32_t unused;
+#pragma unroll 2
+        for (int r = 0; r < rounds; ++r) place((uint32_t)r * BLOCK + tid, unused);
+      }
+    };
+    if (most <= 4) settle(std::integral_constant<int, 3>{}, false);
+    else if (most <= 6) settle(std::integral_constant<int, 5>{}, false);
+    else if (most <= SIDE + 1) settle(std::integral_constant<int, SIDE>{}, false);
+    else settle(std::integral_constant<int, 0>{}, true);
+    if constexpr (KEYS_MOVE) {
+      __syncthreads();  // the codes have been read out of the room the keys take now
+      each_round([&](int r, uint32_t p) { s_keys[p] = e[r]; });
+      __syncthreads();
+      each_round([&](int r, uint32_t p) {
+        if (p < count) keys_out[move[r] & 0xffffu] = decoded(s_keys[move[r] >> 16]);
+      });
+    }
+    if constexpr (HAS_VALUES) {
+      __syncthreads();
+      each_round([&](int r, uint32_t p) { s_vals[p] = v[r]; });
+      __syncthreads();
+      each_round([&](int r, uint32_t p) {
+        if (p < count) vals_out[move[r] & 0xffffu] = s_vals[move[r] >> 16];
+      });
+    }
+    continue;
+  }
+
+  // ---- stable passes over the digits that vary.  A lane's keys are 64 places apart now (loaded again), slots past
+  // the end sort last.  The keys move through LDS with their 16-bit place in the workgroup, by which the values
+  // are picked up at the end.
+  const uint32_t span = (uint32_t)wave * (WAVE * rounds) + lane;  // + r * WAVE
+  uint32_t* s_cnt = s_bin;                                        // [WAVES][RADIX_SIZE]
+  uint32_t* my_cnt = s_cnt + wave * RADIX_SIZE;
+  K differ = 0;
+  uint32_t idx_rank[ITEMS];  // place before, and the rank in a pass << 16
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const uint32_t p = span + r * WAVE;
+    idx_rank[r] = p;
+    if (r < rounds) {
+      const K x = keys_in[p < count ? p : count - 1];
+      differ |= x ^ lo;
+      e[r] = p < count ? x : (K)~(K)0;
+    }
+  }
+  struct Or {
+    TA_DEVICE K operator()(K a, K b) const { return a | b; }
+  };
+  differ = wave_reduce(differ, Or{});
+  __syncthreads();
+  if (lane == 0) s_differ[wave] = differ;
+  for (int i = tid; i < WAVES * RADIX_SIZE; i += BLOCK) s_cnt[i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) differ |= s_differ[w];
+  const uint64_t vary = wave_uniform((uint64_t)differ);
+  for (int at = 0; at < (int)sizeof(K) * 8; at += RADIX_BITS) {
+    if (((vary >> at) & (RADIX_SIZE - 1)) == 0) continue;
+    auto digit_of = [&](K x) { return (uint32_t)(x >> at) & (RADIX_SIZE - 1u); };
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+      if (r < rounds) {
+        idx_rank[r] |= wave_rank_round(digit_of(e[r]), my_cnt) << 16;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();
+    uint32_t sum = 0, incl = 0;
+    if (tid < RADIX_SIZE) {
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        const uint32_t c = s_cnt[w * RADIX_SIZE + tid];
+        s_cnt[w * RADIX_SIZE + tid] = sum;
+        sum += c;
+      }
+      incl = wave_inclusive_scan(sum, OpPlus{});
+      if (lane == WAVE - 1) s_digit_wave[wave] = incl;
+    }
+    __syncthreads();
+    if (tid < RADIX_SIZE) {
+      uint32_t base = incl - sum;
+      for (int w = 0; w < wave; ++w) base += s_digit_wave[w];
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) s_cnt[w * RADIX_SIZE + tid] += base;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+      if (r < rounds) {
+        const uint32_t p = my_cnt[digit_of(e[r])] + (idx_rank[r] >> 16);
+        s_keys[p] = e[r];
+        if constexpr (HAS_VALUES) s_idx[p] = (uint16_t)idx_rank[r];
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < WAVES * RADIX_SIZE; i += BLOCK) s_cnt[i] = 0;
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+      if (r < rounds) {
+        e[r] = s_keys[span + r * WAVE];
+        idx_rank[r] = HAS_VALUES ? s_idx[span + r * WAVE] : 0u;
+      }
+    }
+    __syncthreads();
+  }
+  if constexpr (HAS_VALUES) {
+    __syncthreads();
+    for (uint32_t p = tid; p < count; p += BLOCK) s_vals[p] = vals_in[p];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const uint32_t p = span + r * WAVE;
+    if (r < rounds && p < count) {
+      keys_out[p] = codec.decode(e[r]);
+      if constexpr (HAS_VALUES) vals_out[p] = s_vals[idx_rank[r] & 0xffffu];
+    }
+  }
+  }
+}
+
+}  // namespace ta

@@ -3,10 +3,12 @@
 //
 //   init       zeroes the digit histograms, the per-pass tile descriptors and tickets
 //   histogram  one read of the keys builds the 256-bin histogram of EVERY 8-bit digit
-//   scan       exclusive scan of each histogram -> global digit offsets; a digit whose one
+//   plan       exclusive scan of each histogram -> global digit offsets; a digit whose one
 //              bin holds all n keys is marked "skip" (the reference's sequential radix
 //              sort does the same, thrust/system/detail/sequential/stable_radix_sort.inl:
-//              264-283), and the ping-pong source of every pass is derived from that
+//              264-283), and the ping-pong source of every pass is derived from that.  Where the
+//              top one or two digits leave short stretches of equal prefixes, only their passes run
+//              and radix_finish.hpp orders the stretches
 //   pass x P   chained digit-binning pass ("onesweep"): a tile ranks its keys by digit,
 //              learns the global offset of each of its 256 digit runs by decoupled
 //              look-back over the tiles before it, and scatters keys (and values)
@@ -30,6 +32,7 @@
 #include "common.hpp"
 #include "dispatch.hpp"
 #include "launch.hpp"
+#include "radix_finish.hpp"
 #include "radix_rank.hpp"
 #include "small_sort.hpp"
 #include "sort_codec.hpp"
@@ -37,7 +40,6 @@
 
 namespace ta {
 
-constexpr int MAX_PASSES = 8;
 constexpr uint64_t SORT_MAX_N = (1ull << 32) - 1;       // positions and counts are 32-bit
 constexpr uint64_t SORT_MAX_N_NARROW = (1ull << 30) - 1;  // ... and fit 30 bits up to here
 
@@ -51,14 +53,7 @@ struct Descriptor {
   static constexpr D INCLUSIVE = (D)2 << SHIFT;
 };
 
-struct SortCtl {
-  uint32_t skip[MAX_PASSES];     // pass moves nothing
-  uint32_t src_alt[MAX_PASSES];  // pass reads the alternate buffer
-  uint32_t final_in_alt;         // result sits in the alternate buffer after the last pass
-  uint32_t gave_up;              // a tile stopped waiting for its predecessors (see LOOKBACK_SPIN_LIMIT)
-};
-
-constexpr uint32_t TICKET_WORDS = MAX_PASSES * TICKET_CLASSES * TICKET_STRIDE;
+constexpr uint32_t TICKET_WORDS = MAX_SLOTS * TICKET_CLASSES * TICKET_STRIDE;
 
 // A tile waits for its predecessors' counts in a loop.  Every predecessor is taken by a running
 // workgroup as long as every class keeps receiving its workgroups while slots are free -- which
@@ -93,12 +88,28 @@ __global__ __launch_bounds__(256) void sort_init_kernel(uint32_t* __restrict__ w
 // extract at a constant position.
 constexpr int HIST_BLOCK = 1024;
 constexpr int HIST_UNROLL = 4;  // 16-byte vectors in flight per lane
+constexpr uint32_t SAMPLES = 16384;  // keys the plan looks at, at most
+
+// Keys taken from all over the array, one from each stretch of `step` at a place that follows no pattern.
+// The workgroups of the histogram kernel fetch them on the side: 16384 loads from as many pages take one
+// workgroup 40 us.
+template <typename K>
+struct Sampling {
+  K* out;              // [count], encoded
+  uint32_t per_block;  // taken by each workgroup, <= HIST_BLOCK (0: none)
+  uint32_t count;
+  uint32_t step;
+  TA_DEVICE uint32_t position(uint32_t j) const {
+    return j * step + (uint32_t)(((uint64_t)(j * 2654435769u) * step) >> 32);
+  }
+};
 
 template <typename K, int NP, bool WHOLE_BYTES>
 __global__ __launch_bounds__(HIST_BLOCK) void sort_histogram_kernel(const K* __restrict__ keys,
                                                                      uint64_t n, KeyCodec<K> codec,
                                                                      SortGeometry geo,
-                                                                     uint32_t* __restrict__ hist) {
+                                                                     uint32_t* __restrict__ hist,
+                                                                     Sampling<K> sampling) {
   constexpr int COPIES = NP <= 4 ? 32 : 16;
   constexpr int BINS = NP * RADIX_SIZE;
   constexpr int VEC = Vec16<K>::N;
@@ -106,6 +117,10 @@ __global__ __launch_bounds__(HIST_BLOCK) void sort_histogram_kernel(const K* __r
   for (int i = threadIdx.x; i < BINS * COPIES; i += HIST_BLOCK) s_hist[i] = 0;
   __syncthreads();
   uint32_t* my_copy = s_hist + (threadIdx.x % COPIES);
+  // its address says nothing yet about what is counted below: the load is on its way meanwhile
+  const bool takes_sample = threadIdx.x < sampling.per_block;
+  K sample = 0;
+  if (takes_sample) sample = keys[sampling.position(blockIdx.x * sampling.per_block + threadIdx.x)];
 
   auto count = [&](K k) {
     const K e = (WHOLE_BYTES || codec.plain) ? k : codec.encode(k);
@@ -177,6 +192,7 @@ __global__ __launch_bounds__(HIST_BLOCK) void sort_histogram_kernel(const K* __r
       }
     }
   }
+  if (takes_sample) sampling.out[blockIdx.x * sampling.per_block + threadIdx.x] = codec.encode(sample);
   __syncthreads();
   // fold the copies; thread t starts at copy t so that a wave spreads over all banks
   for (int bin = threadIdx.x; bin < BINS; bin += HIST_BLOCK) {
@@ -190,16 +206,16 @@ __global__ __launch_bounds__(HIST_BLOCK) void sort_histogram_kernel(const K* __r
 template <typename K>
 static void launch_histogram(int passes, uint32_t blocks, hipStream_t stream, const K* keys,
                              uint64_t n, const KeyCodec<K>& codec, const SortGeometry& geo,
-                             uint32_t* hist) {
+                             uint32_t* hist, const Sampling<K>& sampling) {
   const bool whole = codec.plain && geo.begin_bit == 0 && geo.end_bit == passes * RADIX_BITS;
 #define TA_HIST_CASE(NP)                                                                       \
   case NP:                                                                                     \
     if (whole)                                                                                 \
       TA_LAUNCH("sort_histogram", stream, (sort_histogram_kernel<K, NP, true>), dim3(blocks),  \
-                dim3(HIST_BLOCK), keys, n, codec, geo, hist);                                  \
+                dim3(HIST_BLOCK), keys, n, codec, geo, hist, sampling);                                 \
     else                                                                                       \
       TA_LAUNCH("sort_histogram", stream, (sort_histogram_kernel<K, NP, false>), dim3(blocks), \
-                dim3(HIST_BLOCK), keys, n, codec, geo, hist);                                  \
+                dim3(HIST_BLOCK), keys, n, codec, geo, hist, sampling);                                 \
     break;
   switch (passes) {
     TA_HIST_CASE(1) TA_HIST_CASE(2) TA_HIST_CASE(3) TA_HIST_CASE(4)
@@ -209,39 +225,146 @@ static void launch_histogram(int passes, uint32_t blocks, hipStream_t stream, co
 #undef TA_HIST_CASE
 }
 
-// ------------------------------------------------------------------ scan of the histograms
-// One workgroup of 256 threads; thread d owns bin d.  hist[p][d] becomes the exclusive
-// prefix (the global offset of digit d in pass p).
-__global__ __launch_bounds__(RADIX_SIZE) void sort_scan_kernel(uint32_t* __restrict__ hist,
-                                                               uint32_t n, SortGeometry geo,
+// ------------------------------------------------------------------ scan of the histograms, and the plan
+// One workgroup; a group of 256 threads takes every fourth digit, a thread owns a bin.  hist[p][d] becomes the
+// exclusive prefix (the global offset of digit d in pass p), and ctl says what each of the launches behind this
+// one does (SortCtl).
+//
+// The short way (TOP_SLOTS launches over the top digits, then radix_finish.hpp) is taken when the stretches of equal
+// top digits can be expected to fit a workgroup, stretch_max keys:
+//   one digit   its largest bin, known exactly
+//   two digits  the product of the two largest bins' shares (exact for independent digits), and, as digits need not be
+//               independent, SAMPLES keys: the pairs among them that share both digits give the mean size of the stretch
+//               a key finds itself in, and no stretch may hold many more samples than the longest one allowed would
+// A wrong guess costs the TOP_SLOTS passes: the bounds kernel sees every stretch.
+constexpr int PLAN_BLOCK = 1024;
+
+template <typename K>
+__global__ __launch_bounds__(PLAN_BLOCK) void sort_plan_kernel(uint32_t n, Sampling<K> sampling, uint32_t* __restrict__ hist,
+                                                               SortGeometry geo, int top_slots, uint32_t cap,
+                                                               uint32_t stretch_max,  // 0: the short way is not open
                                                                SortCtl* __restrict__ ctl) {
-  __shared__ uint32_t s_wave[RADIX_SIZE / WAVE];
-  __shared__ uint32_t s_full;
-  const int d = threadIdx.x;
-  uint32_t parity = 0;
-  for (int p = 0; p < geo.passes; ++p) {
-    if (d == 0) s_full = 0;
-    __syncthreads();
-    const uint32_t c = hist[p * RADIX_SIZE + d];
-    if (c == n) s_full = 1;
-    const uint32_t incl = wave_inclusive_scan(c, OpPlus{});
-    if ((d % WAVE) == WAVE - 1) s_wave[d / WAVE] = incl;
-    __syncthreads();
-    uint32_t base = 0;
-    for (int w = 0; w < d / WAVE; ++w) base += s_wave[w];
-    hist[p * RADIX_SIZE + d] = base + incl - c;
-    const uint32_t skip = s_full;
-    if (d == 0) {
-      ctl->skip[p] = skip;
-      ctl->src_alt[p] = parity;
+  constexpr int GROUPS = PLAN_BLOCK / RADIX_SIZE;
+  constexpr int PER_THREAD = SAMPLES / PLAN_BLOCK;
+  __shared__ uint32_t s_wave[MAX_PASSES][RADIX_SIZE / WAVE];
+  __shared__ uint32_t s_most[MAX_PASSES];
+  __shared__ uint32_t s_bins[1 << (2 * RADIX_BITS - 1)];  // 16-bit counts, two to a word
+  __shared__ uint32_t s_pairs, s_peak;
+  const int group = threadIdx.x / RADIX_SIZE, d = threadIdx.x % RADIX_SIZE;
+  const int wave = d / WAVE, lane = d % WAVE;
+  if (threadIdx.x < MAX_PASSES) s_most[threadIdx.x] = 0;
+  if (threadIdx.x == 0) s_pairs = s_peak = 0;
+  __syncthreads();
+  uint32_t excl[MAX_PASSES / GROUPS];
+#pragma unroll
+  for (int i = 0; i < MAX_PASSES / GROUPS; ++i) {
+    const int p = i * GROUPS + group;
+    if (p < geo.passes) {
+      const uint32_t c = hist[p * RADIX_SIZE + d];
+      const uint32_t incl = wave_inclusive_scan(c, OpPlus{});
+      const uint32_t most = wave_reduce(c, OpMax{});
+      excl[i] = incl - c;
+      if (lane == WAVE - 1) {
+        s_wave[p][wave] = incl;
+        atomicMax(&s_most[p], most);
+      }
     }
-    parity ^= (skip ? 0u : 1u);
-    __syncthreads();
   }
-  if (d == 0) {
-    ctl->final_in_alt = parity;
-    ctl->gave_up = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < MAX_PASSES / GROUPS; ++i) {
+    const int p = i * GROUPS + group;
+    if (p < geo.passes) {
+      for (int w = 0; w < wave; ++w) excl[i] += s_wave[p][w];
+      hist[p * RADIX_SIZE + d] = excl[i];
+    }
   }
+  int moving = 0, top = 0;  // digits whose pass moves something, and the highest of them
+  for (int p = 0; p < geo.passes; ++p) {
+    if (s_most[p] != n) {
+      ++moving;
+      top = p;
+    }
+  }
+  uint32_t fast = 0;
+  float longest = 0;  // stretch expected
+  if (stretch_max != 0) {
+    if (moving >= 3 && s_most[top] <= stretch_max) {
+      fast = 1;
+      longest = (float)s_most[top];
+    } else if (top_slots == 2 && moving >= 4) {
+      const float share = (float)s_most[top] / (float)n * ((float)s_most[top - 1] / (float)n);
+      longest = share * (float)n;
+      if (longest <= 0.92f * (float)stretch_max) {  // (uniform for the workgroup)
+        for (uint32_t i = threadIdx.x; i < (1u << (2 * RADIX_BITS - 1)); i += PLAN_BLOCK) s_bins[i] = 0;
+        const int bit = (top - 1) * RADIX_BITS;
+        const uint32_t samples = sampling.count;
+        uint32_t bin[PER_THREAD];
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+          const uint32_t j = (uint32_t)i * PLAN_BLOCK + threadIdx.x;
+          bin[i] = j < samples ? (uint32_t)(sampling.out[j] >> bit) & 0xffffu : 0u;
+        }
+        __syncthreads();
+        uint32_t pairs = 0, peak = 0;
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+          if ((uint32_t)i * PLAN_BLOCK + threadIdx.x < samples) {
+            const uint32_t half = (bin[i] & 1u) * 16;
+            const uint32_t old = (__hip_atomic_fetch_add(&s_bins[bin[i] >> 1], 1u << half, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >> half) & 0xffffu;
+            pairs += old;
+            peak = old + 1 > peak ? old + 1 : peak;
+          }
+        }
+        pairs = wave_reduce(pairs, OpPlus{});
+        peak = wave_reduce(peak, OpMax{});
+        if (lane == 0) {
+          atomicAdd(&s_pairs, pairs);
+          atomicMax(&s_peak, peak);
+        }
+        __syncthreads();
+        const float mean = 2.0f * (float)s_pairs / ((float)samples * (float)samples) * (float)n;
+        longest = mean > longest ? mean : longest;
+        const float allowed = (float)stretch_max / (float)n * (float)samples;  // samples the longest stretch would hold
+        if (longest <= 0.92f * (float)stretch_max && (float)s_peak <= allowed + 4.0f * __builtin_sqrtf(allowed) + 8.0f) fast = 2;
+      }
+    }
+  }
+  if (threadIdx.x != 0) return;
+  uint32_t parity = 0;
+  int slot = 0;
+  bool first = true;
+  auto put = [&](uint32_t action, int p, bool last) {
+    ctl->slot[slot++] = SortCtl::pack(action, (uint32_t)p, parity, first, last);
+    if (action != SortCtl::SKIP) {
+      parity ^= 1u;
+      first = false;
+    }
+  };
+  if (fast) {
+    for (int i = (int)fast; i < top_slots; ++i) put(SortCtl::SKIP, 0, false);
+    for (int p = top + 1 - (int)fast; p <= top; ++p) put(s_most[p] == n ? SortCtl::SKIP : SortCtl::RUN, p, false);
+    ctl->fast_src_alt = parity;
+    ctl->final_in_alt = 0;
+    // a window and the longest stretch that may cross its end fill a workgroup: leave room beyond the stretch expected
+    const float room = longest + 6.0f * __builtin_sqrtf(longest) + 0.05f * longest;
+    uint32_t reach = (uint32_t)room + 1;
+    reach = reach < cap / 8 ? cap / 8 : reach > stretch_max ? stretch_max : reach;
+    // ... and take smaller windows than that where they would leave CUs without work
+    const uint32_t even = n / (4 * NUM_CU) > cap - stretch_max ? n / (4 * NUM_CU) : cap - stretch_max;
+    ctl->window = even < cap - reach ? even : cap - reach;
+    ctl->prefix_bit = (uint32_t)((top + 1 - (int)fast) * RADIX_BITS);
+  }
+  if (fast != 1) {  // (one digit: nothing can fail)
+    for (int p = 0; p < geo.passes; ++p)
+      put(s_most[p] == n ? SortCtl::SKIP : fast ? SortCtl::IF_FAILED : SortCtl::RUN, p, p == top);
+  }
+  while (slot < MAX_SLOTS) put(SortCtl::SKIP, 0, false);
+  ctl->fast = fast;
+  ctl->failed = 0;
+  ctl->gave_up = 0;
+  if (fast) ctl->final_in_alt_failed = parity;
+  else ctl->final_in_alt = parity;
 }
 
 // ------------------------------------------------------------------ onesweep pass
@@ -261,11 +384,12 @@ constexpr int LOOKBACK_WINDOW = 4;
 // OFF32: every key and value of the call lies within 4 GiB of its array's start, so that
 // global addresses are a scalar base plus a 32-bit byte offset (one vector instruction per
 // access less than with 64-bit address arithmetic).
-template <typename K, typename V, bool HAS_VALUES, int BLOCK, int ITEMS, typename D, bool OFF32>
-__global__ __launch_bounds__(BLOCK) void onesweep_pass_kernel(
+// CROWDED: registers are held to what two workgroups per CU leave each, at the cost of some spills.
+template <typename K, typename V, bool HAS_VALUES, int BLOCK, int ITEMS, typename D, bool OFF32, bool CROWDED>
+__global__ __launch_bounds__(BLOCK, CROWDED ? 2 * BLOCK / WAVE / 4 : 1) void onesweep_pass_kernel(
     K* __restrict__ keys_a, K* __restrict__ keys_b, V* __restrict__ vals_a, V* __restrict__ vals_b,
-    uint32_t n, int pass, SortGeometry geo, KeyCodec<K> codec,
-    const uint32_t* __restrict__ bin_base,  // [RADIX_SIZE] global digit offsets of this pass
+    uint32_t n, int slot, SortGeometry geo, KeyCodec<K> codec,
+    const uint32_t* __restrict__ hist,      // [passes][RADIX_SIZE] global digit offsets
     D* __restrict__ status,                 // [tiles][RADIX_SIZE]
     uint32_t* __restrict__ ticket,          // [TICKET_CLASSES] counters of this pass, TICKET_STRIDE words apart
     const SortCtl* __restrict__ ctl,
@@ -276,8 +400,11 @@ __global__ __launch_bounds__(BLOCK) void onesweep_pass_kernel(
   constexpr int TILE = Shape::TILE;
   static_assert(BLOCK >= RADIX_SIZE, "one thread per digit is required");
 
-  if (ctl->skip[pass]) return;
-  const bool from_alt = ctl->src_alt[pass] != 0;
+  const uint32_t todo = ctl->slot[slot];
+  if (!SortCtl::runs(todo, ctl->failed)) return;
+  const int pass = (int)SortCtl::digit(todo);
+  const uint32_t* __restrict__ bin_base = hist + pass * RADIX_SIZE;
+  const bool from_alt = SortCtl::src_alt(todo);
   const K* __restrict__ keys_in = from_alt ? keys_b : keys_a;
   K* __restrict__ keys_out = from_alt ? keys_a : keys_b;
   const V* __restrict__ vals_in = from_alt ? vals_b : vals_a;
@@ -324,14 +451,8 @@ __global__ __launch_bounds__(BLOCK) void onesweep_pass_kernel(
 
   // Keys travel between the passes in their encoded form: the first pass that runs encodes them as
   // it loads, the last one decodes them as it stores (unsigned ascending keys need no transform).
-  bool encodes = false, decodes = false;  // uniform
-  if (!codec.plain) {
-    encodes = decodes = true;
-    for (int p = 0; p < pass; ++p)
-      if (!ctl->skip[p]) encodes = false;
-    for (int p = pass + 1; p < geo.passes; ++p)
-      if (!ctl->skip[p]) decodes = false;
-  }
+  const bool encodes = !codec.plain && SortCtl::encodes(todo);  // uniform
+  const bool decodes = !codec.plain && SortCtl::decodes(todo);
 
   // ---- load (wave-striped); slots past the end sort last inside the tile
   K e[ITEMS];
@@ -557,7 +678,7 @@ __global__ __launch_bounds__(256) void sort_copy_back_kernel(K* __restrict__ key
                                                              const V* __restrict__ vals_alt,
                                                              uint64_t n,
                                                              const SortCtl* __restrict__ ctl) {
-  if (!ctl->final_in_alt) return;
+  if (!(ctl->failed ? ctl->final_in_alt_failed : ctl->final_in_alt)) return;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     keys[i] = keys_alt[i];
@@ -576,6 +697,16 @@ struct SortPlan {
                                : (sizeof(K) == 4 && !HAS_VALUES)                 ? 18
                                                                                  : 16;
   static constexpr int TILE = BLOCK * ITEMS;
+  // Where tiles of this size are fewer than the CUs: a third or half of it.  The time is that of one or two tiles
+  // then, and shorter with smaller ones (copy and sort of 1e6 float32 75 -> 65 us, 2.1e6 90 -> 84; 4e6 106 -> 110).
+  static constexpr int FINE_ITEMS = ITEMS == 8 ? 4 : 6;
+  static constexpr uint64_t FINE_MAX = (uint64_t)TILE * NUM_CU * 5 / 8;
+  // 4-byte keys with values need 74 registers, a workgroup per CU.  Two with 64 and 36 bytes of spills each win while
+  // there are a few tiles per CU (8e6 pairs 194 -> 177 us) and lose with one or with many (4e6 115 -> 126, 16e6
+  // 352 -> 353, 32e6 695 -> 718).
+  static constexpr bool TIGHT = sizeof(K) == 4 && HAS_VALUES && ITEMS == 16;
+  static constexpr uint64_t TIGHT_MIN = (uint64_t)TILE * NUM_CU, TIGHT_MAX = 1u << 24;
+  static constexpr int FINE_TILE = BLOCK * FINE_ITEMS;
 };
 
 template <typename K, typename V, bool HAS_VALUES>
@@ -589,7 +720,10 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   geo.begin_bit = begin_bit;
   geo.end_bit = end_bit;
   geo.passes = (end_bit - begin_bit + RADIX_BITS - 1) / RADIX_BITS;
-  const uint64_t tiles = (n + Plan::TILE - 1) / Plan::TILE;
+  const bool fine = n <= Plan::FINE_MAX;
+  const bool crowded = Plan::TIGHT && n > Plan::TIGHT_MIN && n < Plan::TIGHT_MAX;
+  const uint64_t tile = fine ? Plan::FINE_TILE : Plan::TILE;
+  const uint64_t tiles = (n + tile - 1) / tile;
 
   TempLayout lay;
   const size_t off_ctl = lay.add(sizeof(SortCtl));
@@ -597,9 +731,30 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   const bool wide = n > SORT_MAX_N_NARROW;  // prefixes need more than 30 bits: 64-bit descriptors
   // every key and value within 4 GiB of its array's start: 32-bit byte offsets
   const bool off32 = !wide && n * (uint64_t)((HAS_VALUES && sizeof(V) > sizeof(K)) ? sizeof(V) : sizeof(K)) <= (1ull << 32);
-  const size_t zero_words = (size_t)TICKET_WORDS + (size_t)MAX_PASSES * RADIX_SIZE +
-                            (size_t)geo.passes * tiles * RADIX_SIZE * (wide ? 2 : 1);
-  const size_t off_zero = lay.add(zero_words * sizeof(uint32_t));
+  // The short way, over whole keys only.  Against all digits' passes, copy and sort of random keys back to back:
+  //   8-byte keys      9001 keys 80 -> 51 us, 1e6 135 -> 85, 8e6 315 -> 189, 1.28e8 4330 -> 2226; with 4-byte values
+  //                    89 -> 63, 159 -> 91, 398 -> 239, 6188 -> 3033 us
+  //   4-byte integers  by one digit (as long as its bins can fit at all) 9001 keys 58 -> 41 us, 1.5e6 83 -> 62; with
+  //                    values 64 -> 46, 99 -> 72.  By two digits it saves two passes and costs the last step: from 2^25
+  //                    keys without values on 1.06 times as fast (2^28: 1.04), below 0.95-1.02, with values 0.89-1.04.
+  //   floats           share few exponents: 4-byte ones outgrow a workgroup at some 20000 keys, 8-byte ones (four
+  //                    bits of mantissa in two digits) at a few 100000.
+  using Finish = FinishShape<K, V, HAS_VALUES>;
+  const bool is_float = dtype == THRUST_AMD_F32 || dtype == THRUST_AMD_F64;
+  const bool two_digits = sizeof(K) == 8 ? !is_float || n <= (1u << 19) : !HAS_VALUES && !is_float && n >= (1u << 25);
+  const bool one_digit = n <= (is_float ? 8 : 256) * (uint64_t)Finish::STRETCH_MAX;
+  const bool hybrid = sizeof(K) >= 4 && begin_bit == 0 && end_bit == key_bits && n > SMALL_SORT_MAX &&
+                      n / 65536 <= Finish::STRETCH_MAX * 9 / 10 && (one_digit || two_digits);
+  const int top_slots = !hybrid ? 0 : two_digits ? TOP_SLOTS : 1;
+  const int slots = geo.passes + (hybrid && two_digits ? TOP_SLOTS : 0);
+  const uint64_t max_windows = (n + Finish::WINDOW_MIN - 1) / Finish::WINDOW_MIN;
+  // descriptor words of a slot; the first kernel clears those of `cleared_slots` slots, the finish kernel the others
+  const size_t slot_words = (size_t)tiles * RADIX_SIZE * (wide ? 2 : 1);
+  const int cleared_slots = hybrid ? top_slots : slots;
+  const size_t zero_words = (size_t)TICKET_WORDS + (size_t)MAX_PASSES * RADIX_SIZE + (size_t)cleared_slots * slot_words;
+  const size_t off_zero = lay.add((zero_words + (size_t)(slots - cleared_slots) * slot_words) * sizeof(uint32_t));
+  const size_t off_bounds = lay.add(hybrid ? (max_windows + 1) * sizeof(uint32_t) : 0);
+  const size_t off_samples = lay.add(top_slots == 2 ? SAMPLES * sizeof(K) : 0);
   const size_t off_keys = lay.add((size_t)n * sizeof(K));
   const size_t off_vals = lay.add(HAS_VALUES ? (size_t)n * sizeof(V) : 0);
   if (temp == nullptr) {
@@ -630,24 +785,45 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
     TA_LAUNCH("sort_init", stream, sort_init_kernel, dim3((uint32_t)blocks), dim3(256), zero, (uint64_t)zero_words);
     TA_CHECK_LAUNCH();
   }
+  Sampling<K> sampling{};
   {
     constexpr uint64_t HT = (uint64_t)HIST_BLOCK * HIST_UNROLL * Vec16<K>::N;
     uint64_t blocks = (n + HT - 1) / HT;
     if (blocks > (uint64_t)NUM_CU) blocks = NUM_CU;
-    launch_histogram<K>(geo.passes, (uint32_t)blocks, stream, (const K*)keys_a, n, codec, geo, hist);
+    if (top_slots == 2) {
+      sampling.out = reinterpret_cast<K*>(base + off_samples);
+      const uint64_t wanted = n / 256 < SAMPLES ? n / 256 : SAMPLES;
+      const uint64_t each = wanted / blocks < (uint64_t)HIST_BLOCK ? wanted / blocks : (uint64_t)HIST_BLOCK;
+      sampling.per_block = (uint32_t)(each > 0 ? each : 1);
+      sampling.count = sampling.per_block * (uint32_t)blocks;
+      sampling.step = (uint32_t)(n / sampling.count);
+    }
+    launch_histogram<K>(geo.passes, (uint32_t)blocks, stream, (const K*)keys_a, n, codec, geo, hist, sampling);
     TA_CHECK_LAUNCH();
   }
-  TA_LAUNCH("sort_scan", stream, sort_scan_kernel, dim3(1), dim3(RADIX_SIZE), hist, (uint32_t)n, geo, ctl);
+  TA_LAUNCH("sort_plan", stream, sort_plan_kernel<K>, dim3(1), dim3(PLAN_BLOCK), (uint32_t)n, sampling, hist, geo, top_slots, (uint32_t)Finish::CAP, hybrid ? Finish::STRETCH_MAX : 0u, ctl);
   TA_CHECK_LAUNCH();
-  for (int p = 0; p < geo.passes; ++p) {
-    const size_t status_off = (size_t)p * tiles * RADIX_SIZE;  // in descriptor words
-    if (off32) {
-      TA_LAUNCH("onesweep_pass", stream, (onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, true>), dim3((uint32_t)tiles), dim3(Plan::BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, p, geo, codec, hist + p * RADIX_SIZE, status + status_off, tickets + (size_t)p * TICKET_CLASSES * TICKET_STRIDE, (const SortCtl*)ctl, &ctl->gave_up);
-    } else if (wide) {
-      TA_LAUNCH("onesweep_pass", stream, (onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint64_t, false>), dim3((uint32_t)tiles), dim3(Plan::BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, p, geo, codec, hist + p * RADIX_SIZE, reinterpret_cast<uint64_t*>(status) + status_off, tickets + (size_t)p * TICKET_CLASSES * TICKET_STRIDE, (const SortCtl*)ctl, &ctl->gave_up);
-    } else {
-      TA_LAUNCH("onesweep_pass", stream, (onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, false>), dim3((uint32_t)tiles), dim3(Plan::BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, p, geo, codec, hist + p * RADIX_SIZE, status + status_off, tickets + (size_t)p * TICKET_CLASSES * TICKET_STRIDE, (const SortCtl*)ctl, &ctl->gave_up);
+  for (int slot = 0; slot < slots; ++slot) {
+    if constexpr (sizeof(K) >= 4) {
+      if (hybrid && slot == top_slots) {
+        uint32_t* bounds = reinterpret_cast<uint32_t*>(base + off_bounds);
+        TA_LAUNCH("sort_bounds", stream, sort_bounds_kernel<K>, dim3((uint32_t)(max_windows / 256 + 1)), dim3(256), (const K*)keys_a, (const K*)keys_b, (uint32_t)n, (uint32_t)Finish::CAP, bounds, (const SortCtl*)ctl, &ctl->failed);
+        TA_CHECK_LAUNCH();
+        TA_LAUNCH("sort_finish", stream, (sort_finish_kernel<K, V, HAS_VALUES>), dim3((uint32_t)(Finish::LOOPS && max_windows > FINISH_BLOCKS_MAX ? FINISH_BLOCKS_MAX : max_windows)), dim3(Finish::BLOCK), keys_a, (const K*)keys_b, vals_a, (const V*)vals_b, (uint32_t)n, codec, (const uint32_t*)bounds, (const SortCtl*)ctl, status + (size_t)top_slots * slot_words, (uint64_t)((slots - top_slots) * slot_words));
+        TA_CHECK_LAUNCH();
+      }
     }
+    const char* label = hybrid && slot >= top_slots ? "onesweep_rest" : "onesweep_pass";
+    uint32_t* slot_status = status + (size_t)slot * slot_words;
+    uint32_t* slot_tickets = tickets + (size_t)slot * TICKET_CLASSES * TICKET_STRIDE;
+    auto launch = [&](auto kernel, auto* descriptors) {
+      TA_LAUNCH(label, stream, kernel, dim3((uint32_t)tiles), dim3(Plan::BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, slot, geo, codec, (const uint32_t*)hist, descriptors, slot_tickets, (const SortCtl*)ctl, &ctl->gave_up);
+    };
+    if (fine) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::FINE_ITEMS, uint32_t, true, false>, slot_status);
+    else if (off32 && crowded) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, true, Plan::TIGHT>, slot_status);
+    else if (off32) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, true, false>, slot_status);
+    else if (wide) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint64_t, false, false>, reinterpret_cast<uint64_t*>(slot_status));
+    else launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, false, false>, slot_status);
     TA_CHECK_LAUNCH();
   }
   {
