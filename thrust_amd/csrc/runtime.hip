@@ -2,6 +2,7 @@
 // fill, and the temporary-storage arena.  These are the only entry points that
 // allocate or block; every compute entry point works on caller-owned memory.
 #include "common.hpp"
+#include "copy_rule.hpp"
 #include "dispatch.hpp"
 #include "launch.hpp"
 
@@ -71,12 +72,12 @@ namespace ta {
 // this device (256 threads, one 16-byte vector each, 4 KiB per workgroup: many workgroups that live
 // for one load and one store keep the memory system busier than few that loop).  1 GiB: 0.347 ms =
 // 6.2 TB/s; the runtime's own copy, whose 256 workgroups loop, 0.428 ms = 5.0 TB/s.
-__global__ __launch_bounds__(256) void copy_kernel(char* __restrict__ dst, const char* __restrict__ src, uint64_t bytes) {
+__global__ __launch_bounds__(COPY_BLOCK) void copy_kernel(char* __restrict__ dst, const char* __restrict__ src, uint64_t bytes) {
   // dst and src are equally misaligned: the same number of bytes before the first boundary of both
   const uint64_t lead = (16 - (reinterpret_cast<uintptr_t>(dst) & 15)) & 15;
   const uint64_t head = lead < bytes ? lead : bytes;
   const uint64_t vecs = (bytes - head) / 16;
-  const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  const uint64_t i = (uint64_t)blockIdx.x * COPY_BLOCK + threadIdx.x;
   if (i < vecs) reinterpret_cast<uint4*>(dst + head)[i] = reinterpret_cast<const uint4*>(src + head)[i];
   if (blockIdx.x == 0 && threadIdx.x < 16) {
     const uint64_t tail = head + vecs * 16 + threadIdx.x;
@@ -84,10 +85,6 @@ __global__ __launch_bounds__(256) void copy_kernel(char* __restrict__ dst, const
     if (tail < bytes) dst[tail] = src[tail];
   }
 }
-
-// Below this the copy lives in the caches and the runtime's kernel is as fast (64 MiB: 19.7 us here,
-// 19.5 us there; 256 MiB: 88.8 against 98.9 us), without the two pointer lookups.
-constexpr size_t COPY_KERNEL_MIN_BYTES = (size_t)128 << 20;
 
 // True for memory of the given device (not of another device, nor host memory, which the runtime
 // copies in its own way).
@@ -102,14 +99,11 @@ static bool is_own_device_memory(const void* p, int device) {
 
 static int copy_on_device(void* dst, const void* src, size_t bytes, hipStream_t stream) {
   int device = 0;
-  if (bytes >= COPY_KERNEL_MIN_BYTES && ((reinterpret_cast<uintptr_t>(dst) ^ reinterpret_cast<uintptr_t>(src)) & 15) == 0 &&
+  if (copy_kernel_takes(reinterpret_cast<uintptr_t>(dst), reinterpret_cast<uintptr_t>(src), bytes) &&
       hipGetDevice(&device) == hipSuccess && is_own_device_memory(dst, device) && is_own_device_memory(src, device)) {
-    const uint64_t blocks = bytes / 16 / 256 + 1;
-    if (blocks <= 0x7fffffffull) {
-      TA_LAUNCH("copy", stream, copy_kernel, dim3((uint32_t)blocks), dim3(256), static_cast<char*>(dst), static_cast<const char*>(src), (uint64_t)bytes);
-      TA_CHECK_LAUNCH();
-      return 0;
-    }
+    TA_LAUNCH("copy", stream, copy_kernel, dim3((uint32_t)copy_blocks(bytes)), dim3(COPY_BLOCK), static_cast<char*>(dst), static_cast<const char*>(src), (uint64_t)bytes);
+    TA_CHECK_LAUNCH();
+    return 0;
   }
   return (int)hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, stream);
 }
