@@ -1,6 +1,7 @@
 // Host-side check of the rule by which device-to-device copies go to the library's copy kernel
 // (thrust_amd/csrc/copy_rule.hpp, the functions runtime.hip calls): every copy it takes is a legal launch
-// whose threads cover all its vectors, and the larger ones are left to the runtime.
+// whose threads cover all its vectors, the larger ones are left to the runtime, and so are ranges that
+// reach beyond the allocation they begin in.
 #include <cstdint>
 #include <cstdio>
 
@@ -31,6 +32,13 @@ int main() {
   expect(copy_kernel_takes(A + 5, 2 * A + 21, GIB), "equally misaligned buffers");
   expect(!copy_kernel_takes(A, 2 * A + 1, GIB), "differently misaligned buffers");
   expect(!copy_kernel_takes(A, 2 * A, COPY_KERNEL_MIN_BYTES - 1), "small copies");
+  expect(copy_range_known(A, GIB, A, GIB), "a whole allocation");
+  expect(copy_range_known(A + 16, GIB - 16, A, GIB), "the end of an allocation");
+  expect(!copy_range_known(A, GIB + 1, A, GIB), "a byte past the end");
+  expect(!copy_range_known(A + 16, GIB, A, GIB), "past the end from inside");
+  expect(!copy_range_known(A + GIB + 1, 1, A, GIB), "behind the allocation");
+  expect(!copy_range_known(A - 1, 1, A, GIB), "in front of the allocation");
+  expect(!copy_range_known(A + 16, ~(uint64_t)0, A, GIB), "a size that wraps round");
   if (failures == 0) std::printf("PASSED\n");
   return failures != 0;
 }

@@ -18,6 +18,12 @@ constexpr uint64_t COPY_BLOCKS_MAX = 0xffffffffull / COPY_BLOCK;
 
 inline uint64_t copy_blocks(uint64_t bytes) { return bytes / 16 / COPY_BLOCK + 1; }
 
+// [p, p + bytes) lies inside the allocation [base, base + size).  The runtime's copy refuses a range that does not
+// (the caller's mistake, which the kernel would carry out); it also knows buffers mapped from several allocations.
+inline bool copy_range_known(uintptr_t p, uint64_t bytes, uintptr_t base, uint64_t size) {
+  return p >= base && p - base <= size && bytes <= size - (p - base);
+}
+
 inline bool copy_kernel_takes(uintptr_t dst, uintptr_t src, uint64_t bytes) {
   return bytes >= COPY_KERNEL_MIN_BYTES && ((dst ^ src) & 15) == 0 && copy_blocks(bytes) <= COPY_BLOCKS_MAX;
 }

@@ -86,21 +86,25 @@ __global__ __launch_bounds__(COPY_BLOCK) void copy_kernel(char* __restrict__ dst
   }
 }
 
-// True for memory of the given device (not of another device, nor host memory, which the runtime
-// copies in its own way).
-static bool is_own_device_memory(const void* p, int device) {
+// True for a range inside one allocation of the given device (not of another device, nor host memory, which the
+// runtime copies in its own way).
+static bool is_own_device_memory(const void* p, size_t bytes, int device) {
   hipPointerAttribute_t attr;
-  if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess ||
+      hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  return attr.type == hipMemoryTypeDevice && attr.device == device;
+  return attr.type == hipMemoryTypeDevice && attr.device == device &&
+         copy_range_known(reinterpret_cast<uintptr_t>(p), bytes, reinterpret_cast<uintptr_t>(base), size);
 }
 
 static int copy_on_device(void* dst, const void* src, size_t bytes, hipStream_t stream) {
   int device = 0;
   if (copy_kernel_takes(reinterpret_cast<uintptr_t>(dst), reinterpret_cast<uintptr_t>(src), bytes) &&
-      hipGetDevice(&device) == hipSuccess && is_own_device_memory(dst, device) && is_own_device_memory(src, device)) {
+      hipGetDevice(&device) == hipSuccess && is_own_device_memory(dst, bytes, device) && is_own_device_memory(src, bytes, device)) {
     TA_LAUNCH("copy", stream, copy_kernel, dim3((uint32_t)copy_blocks(bytes)), dim3(COPY_BLOCK), static_cast<char*>(dst), static_cast<const char*>(src), (uint64_t)bytes);
     TA_CHECK_LAUNCH();
     return 0;
