@@ -25,37 +25,9 @@
 #include "launch.hpp"
 #include "radix_rank.hpp"
 #include "sort_codec.hpp"
+#include "sort_ctl.hpp"
 
 namespace ta {
-
-constexpr int MAX_PASSES = 8;
-constexpr int TOP_SLOTS = 2;                       // passes in front of the last step, at most
-constexpr int MAX_SLOTS = TOP_SLOTS + MAX_PASSES;  // pass launches of a sort
-
-// What the launches of a sort do, decided on the device from the histograms.  A sort through all digits uses as
-// many slots as it has digits, whatever their number; one that takes the short way its first TOP_SLOTS, and the
-// others only if the bounds kernel finds a stretch that does not fit.
-struct SortCtl {
-  enum : uint32_t { SKIP, RUN, IF_FAILED };
-  uint32_t slot[MAX_SLOTS];      // action, digit, source buffer, whether it encodes / decodes the keys
-  uint32_t final_in_alt;         // result sits in the alternate buffer after the last slot,
-  uint32_t final_in_alt_failed;  // ... if the short way failed
-  uint32_t gave_up;              // a tile stopped waiting for its predecessors (see LOOKBACK_SPIN_LIMIT)
-  uint32_t fast;                 // the short way is taken, with this many digits
-  uint32_t failed;               // ... and was given up
-  uint32_t fast_src_alt;         // the last step reads the alternate buffer
-  uint32_t prefix_bit;           // lowest bit of the digits the array is ordered by then
-  uint32_t window;               // positions per workgroup of the last step
-
-  static TA_DEVICE uint32_t pack(uint32_t action, uint32_t digit, uint32_t src_alt, bool encodes, bool decodes) {
-    return action | digit << 4 | src_alt << 8 | (encodes ? 1u << 9 : 0u) | (decodes ? 1u << 10 : 0u);
-  }
-  static TA_DEVICE bool runs(uint32_t s, uint32_t failed) { return (s & 15u) == RUN || ((s & 15u) == IF_FAILED && failed != 0); }
-  static TA_DEVICE uint32_t digit(uint32_t s) { return s >> 4 & 15u; }
-  static TA_DEVICE bool src_alt(uint32_t s) { return (s >> 8 & 1u) != 0; }
-  static TA_DEVICE bool encodes(uint32_t s) { return (s >> 9 & 1u) != 0; }
-  static TA_DEVICE bool decodes(uint32_t s) { return (s >> 10 & 1u) != 0; }
-};
 
 constexpr uint32_t FINISH_BIN_MAX = 24;
 constexpr uint64_t FINISH_BLOCKS_MAX = NUM_CU * 4;  // workgroups without a window cost their dispatch
@@ -77,7 +49,7 @@ template <typename K>
 __global__ __launch_bounds__(256) void sort_bounds_kernel(const K* __restrict__ keys_a, const K* __restrict__ keys_b, uint32_t n,
                                                           uint32_t cap, uint32_t* __restrict__ bounds, const SortCtl* __restrict__ ctl,
                                                           uint32_t* __restrict__ failed) {
-  if (!ctl->fast) return;
+  if (!ctl->finds_bounds()) return;
   const uint32_t window = ctl->window;
   const uint32_t windows = (n + window - 1) / window;
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -139,7 +111,7 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   static_assert(ITEMS % GROUP == 0, "groups");
   static_assert(WAVES * RADIX_SIZE <= BIN_WORDS, "the passes' counters lie over the bins");
 
-  if (!ctl->fast || ctl->failed) {
+  if (!ctl->finishes()) {
     // the chained passes do the sort: their tile descriptors are cleared here, not by every call's first kernel
     const uint64_t stride = (uint64_t)gridDim.x * BLOCK;
     for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < status_words; i += stride) status[i] = 0;

@@ -61,7 +61,8 @@ constexpr uint32_t TICKET_WORDS = MAX_SLOTS * TICKET_CLASSES * TICKET_STRIDE;
 // least 64 slots.  Should neither hold, a tile that has polled this often stops waiting: it
 // uses what it has summed so far (its positions stay inside the array: a prefix can only be too
 // small), sets SortCtl::gave_up, and every tile that sees the flag does the same, so the
-// kernel ends -- with keys out of order -- instead of hanging.
+// kernel ends instead of hanging.  The launches behind it do nothing then (SortCtl::strike_out): the
+// call ends with an unfinished sort, keys out of order and in their encoded form.
 constexpr uint32_t LOOKBACK_SPIN_LIMIT = 1u << 21;
 
 struct SortGeometry {
@@ -393,7 +394,7 @@ __global__ __launch_bounds__(BLOCK, CROWDED ? 2 * BLOCK / WAVE / 4 : 1) void one
     D* __restrict__ status,                 // [tiles][RADIX_SIZE]
     uint32_t* __restrict__ ticket,          // [TICKET_CLASSES] counters of this pass, TICKET_STRIDE words apart
     const SortCtl* __restrict__ ctl,
-    uint32_t* __restrict__ gave_up) {       // &SortCtl::gave_up, the one field the passes write
+    SortCtl* __restrict__ ctl_out) {        // the same block: fields that only a pass that gives up writes
   using Shape = PassShape<K, V, HAS_VALUES, BLOCK, ITEMS>;
   using Desc = Descriptor<D>;
   constexpr int WAVES = Shape::WAVES;
@@ -605,8 +606,10 @@ __global__ __launch_bounds__(BLOCK, CROWDED ? 2 * BLOCK / WAVE / 4 : 1) void one
           ++spins;
           if (spins >= LOOKBACK_SPIN_LIMIT ||
               (spins % 1024u == 0 &&
-               __hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-            __hip_atomic_store(gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+               __hip_atomic_load(&ctl_out->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+            ctl_out->strike_out(slot, [](uint32_t* p, uint32_t x) {
+              __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            });
             break;
           }
         }
@@ -678,7 +681,7 @@ __global__ __launch_bounds__(256) void sort_copy_back_kernel(K* __restrict__ key
                                                              const V* __restrict__ vals_alt,
                                                              uint64_t n,
                                                              const SortCtl* __restrict__ ctl) {
-  if (!(ctl->failed ? ctl->final_in_alt_failed : ctl->final_in_alt)) return;
+  if (!ctl->copies_back()) return;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     keys[i] = keys_alt[i];
@@ -817,7 +820,7 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
     uint32_t* slot_status = status + (size_t)slot * slot_words;
     uint32_t* slot_tickets = tickets + (size_t)slot * TICKET_CLASSES * TICKET_STRIDE;
     auto launch = [&](auto kernel, auto* descriptors) {
-      TA_LAUNCH(label, stream, kernel, dim3((uint32_t)tiles), dim3(Plan::BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, slot, geo, codec, (const uint32_t*)hist, descriptors, slot_tickets, (const SortCtl*)ctl, &ctl->gave_up);
+      TA_LAUNCH(label, stream, kernel, dim3((uint32_t)tiles), dim3(Plan::BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, slot, geo, codec, (const uint32_t*)hist, descriptors, slot_tickets, (const SortCtl*)ctl, ctl);
     };
     if (fine) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::FINE_ITEMS, uint32_t, true, false>, slot_status);
     else if (off32 && crowded) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, true, Plan::TIGHT>, slot_status);
