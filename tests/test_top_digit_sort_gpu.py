@@ -51,6 +51,25 @@ def _order(x, descending):
     return np.argsort(~u if descending else u, kind="stable")
 
 
+def _control(temp):
+    """The control block of the last sort (thrust_amd/csrc/sort_ctl.hpp), the first thing in its temporary storage."""
+    words = temp.buf[:18 * 4].cpu().numpy().view(np.uint32)
+    return {"gave_up": int(words[12]), "fast": int(words[13]), "failed": int(words[14])}
+
+
+@pytest.mark.parametrize("n", [1 << 25, (1 << 25) + 4097])
+@pytest.mark.parametrize("repeats", [1, 100])
+def test_four_byte_keys_never_take_two_digits(dev, n, repeats):
+    """With two digits, stretches of keys that repeat outgrow a workgroup after the passes over them have run."""
+    temp = dev.Temp()
+    values = datagen.splitmix64(3, n // repeats).astype(np.uint32)
+    x = values[(datagen.splitmix64(4, n) % np.uint64(len(values))).astype(np.int64)]
+    k = dev.DeviceArray.from_numpy(x)
+    dev.sort_keys(k, temp=temp)
+    assert _control(temp)["fast"] == 0
+    assert np.array_equal(k.numpy(), np.sort(x))
+
+
 @pytest.mark.parametrize("dtype", [np.uint32, np.int32, np.float32, np.uint64, np.float64])
 @pytest.mark.parametrize("kind", ["uniform", "normal", "repeated", "clusters", "long_stretch", "equal", "skewed", "ids", "sorted"])
 def test_sorts_by_top_digits(dev, dtype, kind):

@@ -13,11 +13,9 @@
 // turns counts into starts, the keys are laid out by bin, and each key counts the keys of its bin that belong in front
 // of it -- the smaller ones and, among equal ones, those that stood in front -- so the atomics' order does not show.
 // What bounds it: vector instructions (90 per key and lane) and, for 2000 keys a workgroup, the latency of its ten
-// steps; LDS is busy 40 % of the time.  2^28 uint32: 0.93 ms (2.3 TB/s) in place of two passes of 0.50; 2^27 (uint64,
-// uint32): 0.85 ms (3.8 TB/s) in place of six of 0.65.  Measured on the way: comparing inside the bins place by place 1.39
-// ms, with lanes that hold neighbouring places 1.98 (bank conflicts), 512 threads with 16 keys each and spilled
-// registers 1.30.  Workgroups that loop over windows save their dispatch where the chained passes do the sort (112 us for
-// 2^28 keys), but cost 8-byte keys registers (0.85 -> 1.19 ms).
+// steps; LDS is busy 40 % of the time.  2^27 (uint64, uint32): 0.85 ms (3.8 TB/s) in place of six passes of 0.65.
+// Workgroups that loop over windows save their dispatch where the chained passes do the sort, but cost
+// registers (0.85 -> 1.19 ms).
 // A bin of more than FINISH_BIN_MAX keys (many equal keys, values in clusters) makes the workgroup run stable passes
 // over the digits that vary instead.
 #pragma once
@@ -30,7 +28,6 @@
 namespace ta {
 
 constexpr uint32_t FINISH_BIN_MAX = 24;
-constexpr uint64_t FINISH_BLOCKS_MAX = NUM_CU * 4;  // workgroups without a window cost their dispatch
 
 template <typename K, typename V, bool HAS_VALUES>
 struct FinishShape {
@@ -39,7 +36,6 @@ struct FinishShape {
   static constexpr int ITEMS = 8;
   static constexpr int CAP = BLOCK * ITEMS;
   static constexpr int WAVES_PER_SIMD = (BIG ? 3 : 2) * BLOCK / WAVE / 4;
-  static constexpr bool LOOPS = !BIG;  // a workgroup takes one window after the other
   static constexpr uint32_t WINDOW_MIN = BIG ? 1536 : 2048;
   static constexpr uint32_t STRETCH_MAX = CAP - WINDOW_MIN;  // longest stretch of one prefix that can be promised a place
 };
@@ -130,13 +126,12 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   K* s_keys = reinterpret_cast<K*>(s_items);
   V* s_vals = reinterpret_cast<V*>(s_items);
 
-  for (uint32_t w = blockIdx.x; w < windows; w = Shape::LOOPS ? w + gridDim.x : windows) {
+  const uint32_t w = blockIdx.x;
+  if (w >= windows) return;
   const uint32_t first = bounds[w];
   const uint32_t count = bounds[w + 1] - first;
-  if (count == 0 || count > (uint32_t)CAP) continue;
-  if (Shape::LOOPS) __syncthreads();  // the window before is done with the LDS
-  uint32_t tid = threadIdx.x;
-  if (Shape::LOOPS) asm volatile("" : "+v"(tid));  // nothing derived from it is kept from window to window
+  if (count == 0 || count > (uint32_t)CAP) return;
+  const uint32_t tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int rounds = (int)((count + BLOCK - 1) / BLOCK);
   const K* __restrict__ keys_in = (ctl->fast_src_alt ? keys_b : keys_a) + first;
@@ -314,7 +309,7 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
         if (p < count) vals_out[move[r] & 0xffffu] = s_vals[move[r] >> 16];
       });
     }
-    continue;
+    return;
   }
 
   // ---- stable passes over the digits that vary.  A lane's keys are 64 places apart now (loaded again), slots past
@@ -407,7 +402,6 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
       keys_out[p] = codec.decode(e[r]);
       if constexpr (HAS_VALUES) vals_out[p] = s_vals[idx_rank[r] & 0xffffu];
     }
-  }
   }
 }
 

@@ -738,13 +738,14 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   //   8-byte keys      9001 keys 80 -> 51 us, 1e6 135 -> 85, 8e6 315 -> 189, 1.28e8 4330 -> 2226; with 4-byte values
   //                    89 -> 63, 159 -> 91, 398 -> 239, 6188 -> 3033 us
   //   4-byte integers  by one digit (as long as its bins can fit at all) 9001 keys 58 -> 41 us, 1.5e6 83 -> 62; with
-  //                    values 64 -> 46, 99 -> 72.  By two digits it saves two passes and costs the last step: from 2^25
-  //                    keys without values on 1.06 times as fast (2^28: 1.04), below 0.95-1.02, with values 0.89-1.04.
+  //                    values 64 -> 46, 99 -> 72.  Never by two digits: that saves two passes and costs the last step,
+  //                    0.95-1.06 times as fast for random keys of 2^25 and more, and where keys repeat (ten times or a
+  //                    thousand) their stretches outgrow a workgroup after the passes have run: 2^28 keys 2170 -> 3220 us.
   //   floats           share few exponents: 4-byte ones outgrow a workgroup at some 20000 keys, 8-byte ones (four
   //                    bits of mantissa in two digits) at a few 100000.
   using Finish = FinishShape<K, V, HAS_VALUES>;
   const bool is_float = dtype == THRUST_AMD_F32 || dtype == THRUST_AMD_F64;
-  const bool two_digits = sizeof(K) == 8 ? !is_float || n <= (1u << 19) : !HAS_VALUES && !is_float && n >= (1u << 25);
+  const bool two_digits = sizeof(K) == 8 && (!is_float || n <= (1u << 19));
   const bool one_digit = n <= (is_float ? 8 : 256) * (uint64_t)Finish::STRETCH_MAX;
   const bool hybrid = sizeof(K) >= 4 && begin_bit == 0 && end_bit == key_bits && n > SMALL_SORT_MAX &&
                       n / 65536 <= Finish::STRETCH_MAX * 9 / 10 && (one_digit || two_digits);
@@ -812,7 +813,7 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
         uint32_t* bounds = reinterpret_cast<uint32_t*>(base + off_bounds);
         TA_LAUNCH("sort_bounds", stream, sort_bounds_kernel<K>, dim3((uint32_t)(max_windows / 256 + 1)), dim3(256), (const K*)keys_a, (const K*)keys_b, (uint32_t)n, (uint32_t)Finish::CAP, bounds, (const SortCtl*)ctl, &ctl->failed);
         TA_CHECK_LAUNCH();
-        TA_LAUNCH("sort_finish", stream, (sort_finish_kernel<K, V, HAS_VALUES>), dim3((uint32_t)(Finish::LOOPS && max_windows > FINISH_BLOCKS_MAX ? FINISH_BLOCKS_MAX : max_windows)), dim3(Finish::BLOCK), keys_a, (const K*)keys_b, vals_a, (const V*)vals_b, (uint32_t)n, codec, (const uint32_t*)bounds, (const SortCtl*)ctl, status + (size_t)top_slots * slot_words, (uint64_t)((slots - top_slots) * slot_words));
+        TA_LAUNCH("sort_finish", stream, (sort_finish_kernel<K, V, HAS_VALUES>), dim3((uint32_t)max_windows), dim3(Finish::BLOCK), keys_a, (const K*)keys_b, vals_a, (const V*)vals_b, (uint32_t)n, codec, (const uint32_t*)bounds, (const SortCtl*)ctl, status + (size_t)top_slots * slot_words, (uint64_t)((slots - top_slots) * slot_words));
         TA_CHECK_LAUNCH();
       }
     }
