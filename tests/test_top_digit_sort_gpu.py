@@ -53,8 +53,57 @@ def _order(x, descending):
 
 def _control(temp):
     """The control block of the last sort (thrust_amd/csrc/sort_ctl.hpp), the first thing in its temporary storage."""
-    words = temp.buf[:18 * 4].cpu().numpy().view(np.uint32)
-    return {"gave_up": int(words[12]), "fast": int(words[13]), "failed": int(words[14])}
+    words = temp.buf[:15 * 4].cpu().numpy().view(np.uint32)
+    return {"gave_up": int(words[9]), "fast": int(words[10]), "long_windows": int(words[14])}
+
+
+def _sampled(n):
+    """Places the plan of a two-digit sort looks at (Sampling in thrust_amd/csrc/radix_sort.hip)."""
+    blocks = min(-(-n // 8192), 256)
+    each = max(1, min(min(n // 64, 16384) // blocks, 1024))
+    count = each * blocks
+    step = n // count
+    j = np.arange(count, dtype=np.uint64)
+    return j * np.uint64(step) + (((j * np.uint64(2654435769) & np.uint64(0xFFFFFFFF)) * np.uint64(step)) >> np.uint64(32))
+
+
+# (how many keys, what they are): more than a workgroup of the last step takes, and of one tile, some, and many of the tail's
+LONG = [(150_001, "hot", 4100), (150_001, "prefix", 5000), (150_001, "both", 8193), (1_000_003, "hot", 9001),
+        (1_000_003, "prefix", 30_001)]
+
+
+@pytest.mark.parametrize("dtype", [np.uint64, np.int64])
+@pytest.mark.parametrize("n,kind,many", LONG)
+def test_stretches_too_long_for_the_last_step(dev, dtype, n, kind, many):
+    """Stretches of equal top digits that the samples do not see are sorted by the tail."""
+    unseen = np.ones(n, dtype=bool)
+    unseen[_sampled(n)] = False
+    at = np.flatnonzero(unseen)[::3]
+    assert len(at) >= 2 * many
+    x = datagen.splitmix64(5, n)
+    spread = len(at) // (2 * many)
+    for i, where in enumerate((at[:many * spread:spread], at[many * spread:2 * many * spread:spread])):
+        high = np.uint64(0x1234 + 0x7000 * i) << np.uint64(48)
+        if kind == "hot" or (kind == "both" and i == 0):
+            x[where] = high | np.uint64(77)
+        else:
+            x[where] = high | (x[where] & np.uint64((1 << 48) - 1))
+    x = x.view(dtype)
+    temp = dev.Temp()
+    for descending in (False, True):
+        order = _order(x, descending)
+        k = dev.DeviceArray.from_numpy(x)
+        dev.sort_keys(k, descending=descending, temp=temp)
+        control = _control(temp)
+        assert control["fast"] == 2 and control["long_windows"] >= 2, control
+        assert np.array_equal(k.numpy(), x[order]), descending
+        for vdtype in (np.uint8, np.uint32, np.uint64):
+            v = np.arange(n).astype(vdtype)
+            k, w = dev.DeviceArray.from_numpy(x), dev.DeviceArray.from_numpy(v)
+            dev.sort_pairs(k, w, descending=descending, temp=temp)
+            assert _control(temp)["long_windows"] >= 2
+            assert np.array_equal(k.numpy(), x[order]), (vdtype, descending)
+            assert np.array_equal(w.numpy(), v[order]), (vdtype, descending)
 
 
 @pytest.mark.parametrize("n", [1 << 25, (1 << 25) + 4097])

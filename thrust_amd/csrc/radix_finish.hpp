@@ -1,12 +1,11 @@
 // The last step of a radix sort whose passes covered the top digits only: the array is in stable order of a
 // prefix of the keys, and every stretch of equal prefixes is short enough to be ordered in one workgroup.
 //
-//   bounds  for every window of `window` positions the first place at or behind its start where a new prefix
-//           begins.  A stretch that reaches further than CAP - window past the edge it crosses raises
-//           SortCtl::failed, and the chained passes sort the array as if nothing had happened (it holds the same
-//           keys, equal ones in their original order).
-//   finish  a workgroup takes the stretches that begin inside its window (at most CAP keys), orders them by the
-//           whole key in registers and LDS and writes them to their place in the caller's array.
+//   bounds  for every window of `window` positions the first place at or behind its start where a new prefix begins
+//   finish  a workgroup takes the stretches that begin inside its window, orders them by the whole key in registers
+//           and LDS and writes them to their place in the caller's array.  More than CAP keys (a stretch that the plan
+//           did not expect) are left to the
+//   tail    where a workgroup sorts such a window with stable passes through memory
 //
 // Inside a workgroup the keys go to as many bins as there are places (key minus smallest key, shifted so that the
 // largest falls into the last bins): one LDS atomic per key counts a bin and tells the key its place in it, a scan
@@ -43,9 +42,8 @@ struct FinishShape {
 // window: see above; sorted: the array in order of its keys' bits from prefix_bit on; bounds[ceil(n / window) + 1]
 template <typename K>
 __global__ __launch_bounds__(256) void sort_bounds_kernel(const K* __restrict__ keys_a, const K* __restrict__ keys_b, uint32_t n,
-                                                          uint32_t cap, uint32_t* __restrict__ bounds, const SortCtl* __restrict__ ctl,
-                                                          uint32_t* __restrict__ failed) {
-  if (!ctl->finds_bounds()) return;
+                                                          uint32_t cap, uint32_t* __restrict__ bounds, const SortCtl* __restrict__ ctl) {
+  if (!ctl->finishes()) return;
   const uint32_t window = ctl->window;
   const uint32_t windows = (n + window - 1) / window;
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -57,13 +55,12 @@ __global__ __launch_bounds__(256) void sort_bounds_kernel(const K* __restrict__ 
   const K* __restrict__ x = ctl->fast_src_alt ? keys_b : keys_a;
   const int bit = (int)ctl->prefix_bit;
   const uint32_t edge = i * window;
-  const uint32_t reach = cap - window;  // a new prefix has to begin at edge + reach at the latest
+  const uint32_t reach = cap - window;  // a new prefix is expected at edge + reach at the latest
   const K here = x[edge - 1] >> bit;
   uint32_t lo = edge, hi = n - edge < reach ? n : edge + reach;  // the answer lies in [lo, hi]
   if (hi < n && (x[hi] >> bit) == here) {
-    __hip_atomic_store(failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    bounds[i] = edge;
-    return;
+    lo = hi + 1;
+    hi = n;
   }
   while (lo < hi) {
     const uint32_t mid = lo + (hi - lo) / 2;
@@ -85,8 +82,9 @@ TA_DEVICE uint32_t row_inclusive_scan(uint32_t x) {
 template <typename K, typename V, bool HAS_VALUES>
 __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShape<K, V, HAS_VALUES>::WAVES_PER_SIMD)) void sort_finish_kernel(
     K* __restrict__ keys_a, const K* __restrict__ keys_b, V* __restrict__ vals_a, const V* __restrict__ vals_b, uint32_t n,
-    KeyCodec<K> codec, const uint32_t* __restrict__ bounds, const SortCtl* __restrict__ ctl, uint32_t* __restrict__ status,
-    uint64_t status_words) {
+    KeyCodec<K> codec, const uint32_t* __restrict__ bounds, const SortCtl* __restrict__ ctl, uint32_t* __restrict__ long_windows,
+    uint32_t* __restrict__ long_list,  // windows for the tail, *long_windows of them
+    uint32_t* __restrict__ status, uint64_t status_words) {
   using Shape = FinishShape<K, V, HAS_VALUES>;
   constexpr int BLOCK = Shape::BLOCK, ITEMS = Shape::ITEMS, CAP = Shape::CAP, WAVES = BLOCK / WAVE;
   constexpr bool BIG = Shape::BIG;
@@ -130,8 +128,12 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   if (w >= windows) return;
   const uint32_t first = bounds[w];
   const uint32_t count = bounds[w + 1] - first;
-  if (count == 0 || count > (uint32_t)CAP) return;
+  if (count == 0) return;
   const uint32_t tid = threadIdx.x;
+  if (count > (uint32_t)CAP) {
+    if (tid == 0) long_list[atomicAdd(long_windows, 1u)] = w;
+    return;
+  }
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int rounds = (int)((count + BLOCK - 1) / BLOCK);
   const K* __restrict__ keys_in = (ctl->fast_src_alt ? keys_b : keys_a) + first;
@@ -401,6 +403,140 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
     if (r < rounds && p < count) {
       keys_out[p] = codec.decode(e[r]);
       if constexpr (HAS_VALUES) vals_out[p] = s_vals[idx_rank[r] & 0xffffu];
+    }
+  }
+}
+
+// The windows that do not fit a workgroup of the last step: stable passes over the digits that vary in the window,
+// between the place of the window in the two buffers (its own in either, so nobody else reads or writes them).
+// Tiles of TAIL_BLOCK * TAIL_ITEMS keys are ranked as in a chained pass, one after the other, so the order of the tiles
+// needs no look-back.  Bound by latency: one workgroup has nothing else to do meanwhile.
+// Where no window is left over it copies the result back if it sits in the alternate buffer, or does nothing.
+constexpr int TAIL_BLOCK = 1024;
+constexpr int TAIL_ITEMS = 8;
+
+template <typename K, typename V, bool HAS_VALUES>
+__global__ __launch_bounds__(TAIL_BLOCK) void sort_tail_kernel(K* keys_a, K* keys_b, V* vals_a, V* vals_b, uint32_t n,
+                                                               KeyCodec<K> codec, const uint32_t* __restrict__ bounds,
+                                                               const uint32_t* __restrict__ long_list,
+                                                               const SortCtl* __restrict__ ctl) {
+  constexpr int WAVES = TAIL_BLOCK / WAVE;
+  constexpr int DIGITS = (int)sizeof(K);
+  constexpr uint32_t TILE = TAIL_BLOCK * TAIL_ITEMS;
+  __shared__ uint32_t s_hist[DIGITS][RADIX_SIZE];
+  __shared__ uint32_t s_cnt[WAVES * RADIX_SIZE];
+  __shared__ uint32_t s_base[RADIX_SIZE];  // where the next key of a digit goes
+  __shared__ uint32_t s_digit_wave[RADIX_SIZE / WAVE];
+  __shared__ uint32_t s_constant;          // digits that all keys share, one bit each
+  const uint32_t tid = threadIdx.x;
+  if (ctl->copies_back()) {
+    for (uint64_t i = (uint64_t)blockIdx.x * TAIL_BLOCK + tid; i < n; i += (uint64_t)gridDim.x * TAIL_BLOCK) {
+      keys_a[i] = keys_b[i];
+      if constexpr (HAS_VALUES) vals_a[i] = vals_b[i];
+    }
+    return;
+  }
+  if (!ctl->finishes()) return;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+  uint32_t* my_cnt = s_cnt + wave * RADIX_SIZE;
+  for (uint32_t item = blockIdx.x; item < ctl->long_windows; item += gridDim.x) {
+    const uint32_t w = long_list[item];
+    const uint32_t first = bounds[w], count = bounds[w + 1] - first;
+    bool in_alt = ctl->fast_src_alt != 0;  // where the keys are now
+    __syncthreads();                       // the window before is done with the LDS
+    for (uint32_t i = tid; i < (uint32_t)(DIGITS * RADIX_SIZE); i += TAIL_BLOCK) (&s_hist[0][0])[i] = 0;
+    for (uint32_t i = tid; i < (uint32_t)(WAVES * RADIX_SIZE); i += TAIL_BLOCK) s_cnt[i] = 0;
+    if (tid == 0) s_constant = 0;
+    __syncthreads();
+    {
+      const K* x = (in_alt ? keys_b : keys_a) + first;
+#pragma unroll 4
+      for (uint32_t p = tid; p < count; p += TAIL_BLOCK) {
+        const K k = x[p];
+#pragma unroll
+        for (int d = 0; d < DIGITS; ++d)
+          __hip_atomic_fetch_add(&s_hist[d][(uint32_t)(k >> (d * RADIX_BITS)) & (RADIX_SIZE - 1u)], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
+    __syncthreads();
+    if (tid < RADIX_SIZE) {
+#pragma unroll
+      for (int d = 0; d < DIGITS; ++d)
+        if (s_hist[d][tid] == count) atomicOr(&s_constant, 1u << d);
+    }
+    __syncthreads();
+    const uint32_t constant = __builtin_amdgcn_readfirstlane(s_constant);
+    for (int d = 0; d < DIGITS; ++d) {
+      if (constant >> d & 1u) continue;
+      const int at = d * RADIX_BITS;
+      auto digit_of = [&](K x) { return (uint32_t)(x >> at) & (RADIX_SIZE - 1u); };
+      const K* keys_in = (in_alt ? keys_b : keys_a) + first;
+      K* keys_out = (in_alt ? keys_a : keys_b) + first;
+      const V* vals_in = HAS_VALUES ? (in_alt ? vals_b : vals_a) + first : nullptr;
+      V* vals_out = HAS_VALUES ? (in_alt ? vals_a : vals_b) + first : nullptr;
+      uint32_t c = 0, incl = 0;
+      if (tid < RADIX_SIZE) {
+        c = s_hist[d][tid];
+        incl = wave_inclusive_scan(c, OpPlus{});
+        if (lane == WAVE - 1) s_digit_wave[wave] = incl;
+      }
+      __syncthreads();
+      if (tid < RADIX_SIZE) {
+        uint32_t base = incl - c;
+        for (int v = 0; v < wave; ++v) base += s_digit_wave[v];
+        s_base[tid] = base;
+      }
+      for (uint32_t tile = 0; tile < count; tile += TILE) {
+        K e[TAIL_ITEMS];
+        V v[HAS_VALUES ? TAIL_ITEMS : 1];
+        uint32_t rank[TAIL_ITEMS];
+        const uint32_t span = tile + (uint32_t)wave * (WAVE * TAIL_ITEMS) + lane;
+        // slots past the end (of the last tile) repeat the last key and count as all ones: they come last
+#pragma unroll
+        for (int r = 0; r < TAIL_ITEMS; ++r) {
+          const uint32_t p = span + r * WAVE, q = p < count ? p : count - 1;
+          e[r] = keys_in[q];
+          if constexpr (HAS_VALUES) v[r] = vals_in[q];
+        }
+#pragma unroll
+        for (int r = 0; r < TAIL_ITEMS; ++r) {
+          rank[r] = wave_rank_round(span + r * WAVE < count ? digit_of(e[r]) : RADIX_SIZE - 1u, my_cnt);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+        if (tid < RADIX_SIZE) {
+          uint32_t sum = s_base[tid];
+#pragma unroll
+          for (int k = 0; k < WAVES; ++k) {
+            const uint32_t t = s_cnt[k * RADIX_SIZE + tid];
+            s_cnt[k * RADIX_SIZE + tid] = sum;
+            sum += t;
+          }
+          s_base[tid] = sum;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < TAIL_ITEMS; ++r) {
+          if (span + r * WAVE < count) {
+            const uint32_t q = my_cnt[digit_of(e[r])] + rank[r];
+            keys_out[q] = e[r];
+            if constexpr (HAS_VALUES) vals_out[q] = v[r];
+          }
+        }
+        // a wave's counters are its own until the next barrier
+#pragma unroll
+        for (int i = 0; i < RADIX_SIZE / WAVE; ++i) my_cnt[i * WAVE + lane] = 0;
+      }
+      __syncthreads();  // the next pass reads what this one has written
+      in_alt = !in_alt;
+    }
+    if (in_alt || !codec.plain) {
+      for (uint32_t p = tid; p < count; p += TAIL_BLOCK) {
+        const uint32_t i = first + p;
+        keys_a[i] = codec.decode(in_alt ? keys_b[i] : keys_a[i]);
+        if constexpr (HAS_VALUES)
+          if (in_alt) vals_a[i] = vals_b[i];
+      }
     }
   }
 }

@@ -37,6 +37,7 @@
 #include "small_sort.hpp"
 #include "sort_codec.hpp"
 #include "sort_tickets.hpp"
+#include "top_digits.hpp"
 
 namespace ta {
 
@@ -53,7 +54,7 @@ struct Descriptor {
   static constexpr D INCLUSIVE = (D)2 << SHIFT;
 };
 
-constexpr uint32_t TICKET_WORDS = MAX_SLOTS * TICKET_CLASSES * TICKET_STRIDE;
+constexpr uint32_t TICKET_WORDS = MAX_PASSES * TICKET_CLASSES * TICKET_STRIDE;
 
 // A tile waits for its predecessors' counts in a loop.  Every predecessor is taken by a running
 // workgroup as long as every class keeps receiving its workgroups while slots are free -- which
@@ -231,13 +232,12 @@ static void launch_histogram(int passes, uint32_t blocks, hipStream_t stream, co
 // exclusive prefix (the global offset of digit d in pass p), and ctl says what each of the launches behind this
 // one does (SortCtl).
 //
-// The short way (TOP_SLOTS launches over the top digits, then radix_finish.hpp) is taken when the stretches of equal
+// The short way (one or two launches over the top digits, then radix_finish.hpp) is taken when the stretches of equal
 // top digits can be expected to fit a workgroup, stretch_max keys:
 //   one digit   its largest bin, known exactly
-//   two digits  the product of the two largest bins' shares (exact for independent digits), and, as digits need not be
-//               independent, SAMPLES keys: the pairs among them that share both digits give the mean size of the stretch
-//               a key finds itself in, and no stretch may hold many more samples than the longest one allowed would
-// A wrong guess costs the TOP_SLOTS passes: the bounds kernel sees every stretch.
+//   two digits  (8-byte keys) by the product of the two largest bins' shares, exact for independent digits, and, as digits
+//               need not be independent and keys may repeat, by SAMPLES keys: see top_two_digits
+// A stretch that is longer all the same costs its own sort by one workgroup (sort_tail_kernel), not the array's.
 constexpr int PLAN_BLOCK = 1024;
 
 template <typename K>
@@ -249,12 +249,14 @@ __global__ __launch_bounds__(PLAN_BLOCK) void sort_plan_kernel(uint32_t n, Sampl
   constexpr int PER_THREAD = SAMPLES / PLAN_BLOCK;
   __shared__ uint32_t s_wave[MAX_PASSES][RADIX_SIZE / WAVE];
   __shared__ uint32_t s_most[MAX_PASSES];
-  __shared__ uint32_t s_bins[1 << (2 * RADIX_BITS - 1)];  // 16-bit counts, two to a word
-  __shared__ uint32_t s_pairs, s_peak;
+  constexpr uint32_t PLAN_WORDS = sizeof(K) == 8 ? 1u << (2 * RADIX_BITS - 1) : 1u;
+  static_assert(PLAN_WORDS == 1 || PLAN_WORDS * 32 == TWIN_PLACES, "a bit for every place");
+  __shared__ uint32_t s_bins[PLAN_WORDS];  // 16-bit counts, two to a word; then bits
+  __shared__ uint32_t s_pairs, s_peak, s_twins;
   const int group = threadIdx.x / RADIX_SIZE, d = threadIdx.x % RADIX_SIZE;
   const int wave = d / WAVE, lane = d % WAVE;
   if (threadIdx.x < MAX_PASSES) s_most[threadIdx.x] = 0;
-  if (threadIdx.x == 0) s_pairs = s_peak = 0;
+  if (threadIdx.x == 0) s_pairs = s_peak = s_twins = 0;
   __syncthreads();
   uint32_t excl[MAX_PASSES / GROUPS];
 #pragma unroll
@@ -289,46 +291,62 @@ __global__ __launch_bounds__(PLAN_BLOCK) void sort_plan_kernel(uint32_t n, Sampl
   }
   uint32_t fast = 0;
   float longest = 0;  // stretch expected
-  if (stretch_max != 0) {
-    if (moving >= 3 && s_most[top] <= stretch_max) {
-      fast = 1;
-      longest = (float)s_most[top];
-    } else if (top_slots == 2 && moving >= 4) {
-      const float share = (float)s_most[top] / (float)n * ((float)s_most[top - 1] / (float)n);
-      longest = share * (float)n;
-      if (longest <= 0.92f * (float)stretch_max) {  // (uniform for the workgroup)
-        for (uint32_t i = threadIdx.x; i < (1u << (2 * RADIX_BITS - 1)); i += PLAN_BLOCK) s_bins[i] = 0;
-        const int bit = (top - 1) * RADIX_BITS;
-        const uint32_t samples = sampling.count;
-        uint32_t bin[PER_THREAD];
+  if (stretch_max != 0 && moving >= 3 && s_most[top] <= stretch_max) {
+    fast = 1;
+    longest = (float)s_most[top];
+  }
+  if constexpr (sizeof(K) == 8) {
+    const float even = (float)s_most[top] / (float)n * (float)s_most[top > 0 ? top - 1 : 0];
+    if (!fast && top_slots == 2 && moving >= 4 && even <= (float)stretch_max) {  // (uniform for the workgroup)
+      const uint32_t samples = sampling.count;
+      K sample[PER_THREAD];
 #pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
-          const uint32_t j = (uint32_t)i * PLAN_BLOCK + threadIdx.x;
-          bin[i] = j < samples ? (uint32_t)(sampling.out[j] >> bit) & 0xffffu : 0u;
-        }
+      for (int i = 0; i < PER_THREAD; ++i) {
+        const uint32_t j = (uint32_t)i * PLAN_BLOCK + threadIdx.x;
+        sample[i] = j < samples ? sampling.out[j] : (K)0;
+      }
+      auto clear = [&] {
+        for (uint32_t i = threadIdx.x; i < PLAN_WORDS; i += PLAN_BLOCK) s_bins[i] = 0;
         __syncthreads();
-        uint32_t pairs = 0, peak = 0;
+      };
+      clear();
+      const int bit = (top - 1) * RADIX_BITS;
+      uint32_t pairs = 0, peak = 0, twins = 0;
+#pragma unroll
+      for (int i = 0; i < PER_THREAD; ++i) {
+        if ((uint32_t)i * PLAN_BLOCK + threadIdx.x < samples) {
+          const uint32_t bin = (uint32_t)(sample[i] >> bit) & 0xffffu;
+          const uint32_t half = (bin & 1u) * 16;
+          const uint32_t old = (__hip_atomic_fetch_add(&s_bins[bin >> 1], 1u << half, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >> half) & 0xffffu;
+          pairs += old;
+          peak = old + 1 > peak ? old + 1 : peak;
+        }
+      }
+      if (even > (float)stretch_max / 4) {
+        // samples whose bit, one of TWIN_PLACES by a hash of the key, another one has set before
+        __syncthreads();
+        clear();
 #pragma unroll
         for (int i = 0; i < PER_THREAD; ++i) {
           if ((uint32_t)i * PLAN_BLOCK + threadIdx.x < samples) {
-            const uint32_t half = (bin[i] & 1u) * 16;
-            const uint32_t old = (__hip_atomic_fetch_add(&s_bins[bin[i] >> 1], 1u << half, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >> half) & 0xffffu;
-            pairs += old;
-            peak = old + 1 > peak ? old + 1 : peak;
+            const uint64_t h = ((uint64_t)sample[i] ^ (uint64_t)sample[i] >> 29) * 0x9e3779b97f4a7c15ull;
+            const uint32_t place = (uint32_t)(h >> 40) % TWIN_PLACES, bit_of = 1u << place % 32;
+            const uint32_t old = __hip_atomic_fetch_or(&s_bins[place / 32], bit_of, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            twins += (old & bit_of) != 0 ? 1u : 0u;
           }
         }
-        pairs = wave_reduce(pairs, OpPlus{});
-        peak = wave_reduce(peak, OpMax{});
-        if (lane == 0) {
-          atomicAdd(&s_pairs, pairs);
-          atomicMax(&s_peak, peak);
-        }
-        __syncthreads();
-        const float mean = 2.0f * (float)s_pairs / ((float)samples * (float)samples) * (float)n;
-        longest = mean > longest ? mean : longest;
-        const float allowed = (float)stretch_max / (float)n * (float)samples;  // samples the longest stretch would hold
-        if (longest <= 0.92f * (float)stretch_max && (float)s_peak <= allowed + 4.0f * __builtin_sqrtf(allowed) + 8.0f) fast = 2;
       }
+      pairs = wave_reduce(pairs, OpPlus{});
+      peak = wave_reduce(peak, OpMax{});
+      twins = wave_reduce(twins, OpPlus{});
+      if (lane == 0) {
+        atomicAdd(&s_pairs, pairs);
+        atomicMax(&s_peak, peak);
+        atomicAdd(&s_twins, twins);
+      }
+      __syncthreads();
+      longest = top_two_digits((float)n, (float)samples, even, (float)s_pairs, (float)s_twins, (float)s_peak, (float)stretch_max);
+      if (longest > 0) fast = 2;
     }
   }
   if (threadIdx.x != 0) return;
@@ -342,30 +360,26 @@ __global__ __launch_bounds__(PLAN_BLOCK) void sort_plan_kernel(uint32_t n, Sampl
       first = false;
     }
   };
+  ctl->fast = fast;
+  ctl->gave_up = 0;
+  ctl->long_windows = 0;
   if (fast) {
-    for (int i = (int)fast; i < top_slots; ++i) put(SortCtl::SKIP, 0, false);
     for (int p = top + 1 - (int)fast; p <= top; ++p) put(s_most[p] == n ? SortCtl::SKIP : SortCtl::RUN, p, false);
     ctl->fast_src_alt = parity;
-    ctl->final_in_alt = 0;
+    parity = 0;  // the last step writes the caller's array
     // a window and the longest stretch that may cross its end fill a workgroup: leave room beyond the stretch expected
-    const float room = longest + 6.0f * __builtin_sqrtf(longest) + 0.05f * longest;
+    const float room = fast == 1 ? longest : longest + __builtin_sqrtf(longest) + 0.02f * longest;
     uint32_t reach = (uint32_t)room + 1;
     reach = reach < cap / 8 ? cap / 8 : reach > stretch_max ? stretch_max : reach;
     // ... and take smaller windows than that where they would leave CUs without work
     const uint32_t even = n / (4 * NUM_CU) > cap - stretch_max ? n / (4 * NUM_CU) : cap - stretch_max;
     ctl->window = even < cap - reach ? even : cap - reach;
     ctl->prefix_bit = (uint32_t)((top + 1 - (int)fast) * RADIX_BITS);
+  } else {
+    for (int p = 0; p < geo.passes; ++p) put(s_most[p] == n ? SortCtl::SKIP : SortCtl::RUN, p, p == top);
   }
-  if (fast != 1) {  // (one digit: nothing can fail)
-    for (int p = 0; p < geo.passes; ++p)
-      put(s_most[p] == n ? SortCtl::SKIP : fast ? SortCtl::IF_FAILED : SortCtl::RUN, p, p == top);
-  }
-  while (slot < MAX_SLOTS) put(SortCtl::SKIP, 0, false);
-  ctl->fast = fast;
-  ctl->failed = 0;
-  ctl->gave_up = 0;
-  if (fast) ctl->final_in_alt_failed = parity;
-  else ctl->final_in_alt = parity;
+  while (slot < MAX_PASSES) put(SortCtl::SKIP, 0, false);
+  ctl->final_in_alt = parity;
 }
 
 // ------------------------------------------------------------------ onesweep pass
@@ -402,7 +416,7 @@ __global__ __launch_bounds__(BLOCK, CROWDED ? 2 * BLOCK / WAVE / 4 : 1) void one
   static_assert(BLOCK >= RADIX_SIZE, "one thread per digit is required");
 
   const uint32_t todo = ctl->slot[slot];
-  if (!SortCtl::runs(todo, ctl->failed)) return;
+  if (!SortCtl::runs(todo)) return;
   const int pass = (int)SortCtl::digit(todo);
   const uint32_t* __restrict__ bin_base = hist + pass * RADIX_SIZE;
   const bool from_alt = SortCtl::src_alt(todo);
@@ -750,7 +764,7 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   const bool hybrid = sizeof(K) >= 4 && begin_bit == 0 && end_bit == key_bits && n > SMALL_SORT_MAX &&
                       n / 65536 <= Finish::STRETCH_MAX * 9 / 10 && (one_digit || two_digits);
   const int top_slots = !hybrid ? 0 : two_digits ? TOP_SLOTS : 1;
-  const int slots = geo.passes + (hybrid && two_digits ? TOP_SLOTS : 0);
+  const int slots = geo.passes;
   const uint64_t max_windows = (n + Finish::WINDOW_MIN - 1) / Finish::WINDOW_MIN;
   // descriptor words of a slot; the first kernel clears those of `cleared_slots` slots, the finish kernel the others
   const size_t slot_words = (size_t)tiles * RADIX_SIZE * (wide ? 2 : 1);
@@ -758,6 +772,7 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   const size_t zero_words = (size_t)TICKET_WORDS + (size_t)MAX_PASSES * RADIX_SIZE + (size_t)cleared_slots * slot_words;
   const size_t off_zero = lay.add((zero_words + (size_t)(slots - cleared_slots) * slot_words) * sizeof(uint32_t));
   const size_t off_bounds = lay.add(hybrid ? (max_windows + 1) * sizeof(uint32_t) : 0);
+  const size_t off_long = lay.add(hybrid ? (n / Finish::CAP + 1) * sizeof(uint32_t) : 0);
   const size_t off_samples = lay.add(top_slots == 2 ? SAMPLES * sizeof(K) : 0);
   const size_t off_keys = lay.add((size_t)n * sizeof(K));
   const size_t off_vals = lay.add(HAS_VALUES ? (size_t)n * sizeof(V) : 0);
@@ -796,7 +811,7 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
     if (blocks > (uint64_t)NUM_CU) blocks = NUM_CU;
     if (top_slots == 2) {
       sampling.out = reinterpret_cast<K*>(base + off_samples);
-      const uint64_t wanted = n / 256 < SAMPLES ? n / 256 : SAMPLES;
+      const uint64_t wanted = n / 64 < SAMPLES ? n / 64 : SAMPLES;
       const uint64_t each = wanted / blocks < (uint64_t)HIST_BLOCK ? wanted / blocks : (uint64_t)HIST_BLOCK;
       sampling.per_block = (uint32_t)(each > 0 ? each : 1);
       sampling.count = sampling.per_block * (uint32_t)blocks;
@@ -807,13 +822,14 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   }
   TA_LAUNCH("sort_plan", stream, sort_plan_kernel<K>, dim3(1), dim3(PLAN_BLOCK), (uint32_t)n, sampling, hist, geo, top_slots, (uint32_t)Finish::CAP, hybrid ? Finish::STRETCH_MAX : 0u, ctl);
   TA_CHECK_LAUNCH();
+  uint32_t* bounds = reinterpret_cast<uint32_t*>(base + off_bounds);
+  uint32_t* long_list = reinterpret_cast<uint32_t*>(base + off_long);
   for (int slot = 0; slot < slots; ++slot) {
     if constexpr (sizeof(K) >= 4) {
       if (hybrid && slot == top_slots) {
-        uint32_t* bounds = reinterpret_cast<uint32_t*>(base + off_bounds);
-        TA_LAUNCH("sort_bounds", stream, sort_bounds_kernel<K>, dim3((uint32_t)(max_windows / 256 + 1)), dim3(256), (const K*)keys_a, (const K*)keys_b, (uint32_t)n, (uint32_t)Finish::CAP, bounds, (const SortCtl*)ctl, &ctl->failed);
+        TA_LAUNCH("sort_bounds", stream, sort_bounds_kernel<K>, dim3((uint32_t)(max_windows / 256 + 1)), dim3(256), (const K*)keys_a, (const K*)keys_b, (uint32_t)n, (uint32_t)Finish::CAP, bounds, (const SortCtl*)ctl);
         TA_CHECK_LAUNCH();
-        TA_LAUNCH("sort_finish", stream, (sort_finish_kernel<K, V, HAS_VALUES>), dim3((uint32_t)max_windows), dim3(Finish::BLOCK), keys_a, (const K*)keys_b, vals_a, (const V*)vals_b, (uint32_t)n, codec, (const uint32_t*)bounds, (const SortCtl*)ctl, status + (size_t)top_slots * slot_words, (uint64_t)((slots - top_slots) * slot_words));
+        TA_LAUNCH("sort_finish", stream, (sort_finish_kernel<K, V, HAS_VALUES>), dim3((uint32_t)max_windows), dim3(Finish::BLOCK), keys_a, (const K*)keys_b, vals_a, (const V*)vals_b, (uint32_t)n, codec, (const uint32_t*)bounds, (const SortCtl*)ctl, &ctl->long_windows, long_list, status + (size_t)top_slots * slot_words, (uint64_t)((slots - top_slots) * slot_words));
         TA_CHECK_LAUNCH();
       }
     }
@@ -829,6 +845,15 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
     else if (wide) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint64_t, false, false>, reinterpret_cast<uint64_t*>(slot_status));
     else launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, false, false>, slot_status);
     TA_CHECK_LAUNCH();
+  }
+  if constexpr (sizeof(K) == 8) {
+    if (top_slots == 2) {
+      uint64_t blocks = (n + TAIL_BLOCK - 1) / TAIL_BLOCK;
+      if (blocks > (uint64_t)NUM_CU * 2) blocks = (uint64_t)NUM_CU * 2;
+      TA_LAUNCH("sort_tail", stream, (sort_tail_kernel<K, V, HAS_VALUES>), dim3((uint32_t)blocks), dim3(TAIL_BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, codec, (const uint32_t*)bounds, (const uint32_t*)long_list, (const SortCtl*)ctl);
+      TA_CHECK_LAUNCH();
+      return 0;
+    }
   }
   {
     uint64_t blocks = (n + 255) / 256;
