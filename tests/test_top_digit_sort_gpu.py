@@ -1,6 +1,7 @@
 """The sort that runs its passes over the top digits only and orders the stretches of equal prefixes in
-one workgroup each: inputs that take it with one digit and with two, whose bins are too full for counting,
-that make it give up (a stretch too long for a workgroup), and that never take it."""
+one workgroup each: inputs that take it with one digit and with two, whose bins are full or too full for counting,
+with stretches too long for a workgroup that the samples see (long_stretch: all digits get their pass) or do not see (the
+tail sorts them), and that never take it."""
 import numpy as np
 import pytest
 
@@ -28,6 +29,11 @@ def _keys(kind, dtype, n):
         k = np.full(n, 12345, dtype=np.uint64)
     elif kind == "skewed":        # nine in ten equal
         k = np.where(r % u(10) != 0, u(1 << 20), r)
+    elif kind in ("tens", "near"):  # about ten keys are equal, or share all but their low bits: bins of 9 to 24
+        k = (r >> u(64 - bits))[:max(n // 10, 1)][(datagen.splitmix64(98, n) % u(max(n // 10, 1))).astype(np.int64)]
+        if kind == "near":
+            low = u((1 << (bits // 3)) - 1)
+            k = (k & ~low) | (r & low)
     elif kind == "ids":           # 0 .. n-1 shuffled: constant top digits
         k = np.argsort(r).astype(np.uint64)
     elif kind == "sorted":
@@ -120,7 +126,7 @@ def test_four_byte_keys_never_take_two_digits(dev, n, repeats):
 
 
 @pytest.mark.parametrize("dtype", [np.uint32, np.int32, np.float32, np.uint64, np.float64])
-@pytest.mark.parametrize("kind", ["uniform", "normal", "repeated", "clusters", "long_stretch", "equal", "skewed", "ids", "sorted"])
+@pytest.mark.parametrize("kind", ["uniform", "normal", "repeated", "clusters", "long_stretch", "equal", "skewed", "tens", "near", "ids", "sorted"])
 def test_sorts_by_top_digits(dev, dtype, kind):
     temp = dev.Temp()
     for n in SIZES:

@@ -100,7 +100,8 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   constexpr bool HAS_IDX = KEYS_MOVE || HAS_VALUES;
   constexpr size_t ITEM = (HAS_VALUES && sizeof(V) > sizeof(K)) ? sizeof(V) : sizeof(K);
   constexpr size_t CODE_BYTES = (CAP + 2 * (SIDE + 1)) * sizeof(uint32_t);
-  constexpr size_t FRONT_BYTES = CODE_BYTES > CAP * ITEM ? CODE_BYTES : CAP * ITEM;
+  constexpr size_t REST_BYTES = KEYS_MOVE ? CAP * sizeof(uint32_t) : 0;  // what the codes leave out of a key
+  constexpr size_t FRONT_BYTES = CODE_BYTES + REST_BYTES > CAP * ITEM ? CODE_BYTES + REST_BYTES : CAP * ITEM;
   static_assert(BLOCK >= RADIX_SIZE && (CAP & (CAP - 1)) == 0 && CAP <= 8192 && MY_WORDS % 4 == 0, "shape");
   static_assert(ITEMS % GROUP == 0, "groups");
   static_assert(WAVES * RADIX_SIZE <= BIN_WORDS, "the passes' counters lie over the bins");
@@ -121,6 +122,7 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   __shared__ K s_differ[WAVES];
   __shared__ uint32_t s_most;
   uint32_t* s_code = reinterpret_cast<uint32_t*>(s_items) + SIDE + 1;
+  uint32_t* s_rest = reinterpret_cast<uint32_t*>(s_items + CODE_BYTES);
   K* s_keys = reinterpret_cast<K*>(s_items);
   V* s_vals = reinterpret_cast<V*>(s_items);
 
@@ -223,6 +225,7 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   __syncthreads();
 
   const uint32_t most = s_most;  // keys in the fullest bin, or 4
+  const bool place_by_place = most > (uint32_t)SIDE + 1;
   if (most <= FINISH_BIN_MAX) {
     const uint16_t* s_start = reinterpret_cast<const uint16_t*>(s_bin);
     each_round([&](int r, uint32_t) {
@@ -235,7 +238,15 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
         s_code[slot[r]] = code_of(e[r]);
         if constexpr (HAS_IDX) s_idx[slot[r]] = (uint16_t)p;
       }
+      forget(e[r]);
     });
+    if constexpr (KEYS_MOVE) {
+      if (place_by_place) {
+        each_round([&](int r, uint32_t p) {
+          if (p < count) s_rest[slot[r]] = (uint32_t)e[r] - (uint32_t)lo;
+        });
+      }
+    }
     if (tid < SIDE) {  // what lies outside belongs outside
       s_code[-1 - (int)tid] = 0;
       s_code[count + tid] = ~0u;
@@ -246,7 +257,7 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
     // side of its own, without asking for their bins, as far as the fullest bin can reach.  4-byte keys leave
     // straight for their places: a wave's lie next to each other but for those steps.
     uint32_t move[HAS_IDX ? ITEMS : 1];  // place now, and in the workgroup before << 16
-    auto settle = [&](auto side, bool by_place) {
+    auto settle = [&](auto side, auto by_place) {
       auto place = [&](uint32_t p, uint32_t& packed) {
         const uint32_t mine = s_code[p];
         const uint32_t my_idx = HAS_IDX ? s_idx[p] : 0u;
@@ -260,21 +271,28 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
           if constexpr (HAS_IDX) equal = equal || left == mine || right == mine;
         }
         if (p < count) {
-          if (by_place || equal) {
-            // equal codes: by the whole key where the code is not all of it, and then in the order before
-            auto in_front = [&](uint32_t j) {  // does place j's key belong in front of this one
-              const uint32_t x = s_code[j];
-              if (x != mine || !HAS_IDX) return x < mine || (x == mine && j < p);
-              const uint32_t i = s_idx[j];
-              if constexpr (KEYS_MOVE) {
-                const K a = keys_in[i], b = keys_in[my_idx];
-                if (a != b) return a < b;
-              }
-              return i < my_idx;
-            };
-            const uint32_t from = p > most ? p - most : 0, to = p + most < count ? p + most : count;
+          if (by_place() || equal) {
+            // place by place in the key's own bin: equal codes by what they leave out of the key (from LDS where many
+            // are asked for it) and then in the order before
+            const uint32_t b = mine >> bin_shift;
+            const uint32_t from = s_start[b], to = b + 1 < (uint32_t)BINS ? s_start[b + 1] : count;
+            const uint32_t my_rest = KEYS_MOVE && by_place() ? s_rest[p] : 0u;
             q = from;
-            for (uint32_t j = from; j < to; ++j) q += j != p && in_front(j) ? 1u : 0u;
+            for (uint32_t j = from; j < to; ++j) {
+              const uint32_t x = s_code[j];
+              const uint32_t i = HAS_IDX ? s_idx[j] : j;
+              bool front = i < (HAS_IDX ? my_idx : p);
+              if constexpr (KEYS_MOVE && by_place()) {
+                const uint32_t rest = s_rest[j];
+                front = rest < my_rest || (rest == my_rest && front);
+              } else if constexpr (KEYS_MOVE) {
+                if (x == mine && code_shift != 0) {
+                  const K a = keys_in[i], whole = keys_in[my_idx];
+                  front = a < whole || (a == whole && front);
+                }
+              }
+              q += x < mine || (x == mine && front) ? 1u : 0u;
+            }
           }
           if constexpr (!KEYS_MOVE) keys_out[q] = decoded((K)(lo + mine));
         }
@@ -291,10 +309,10 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
         for (int r = 0; r < rounds; ++r) place((uint32_t)r * BLOCK + tid, unused);
       }
     };
-    if (most <= 4) settle(std::integral_constant<int, 3>{}, false);
-    else if (most <= 6) settle(std::integral_constant<int, 5>{}, false);
-    else if (most <= SIDE + 1) settle(std::integral_constant<int, SIDE>{}, false);
-    else settle(std::integral_constant<int, 0>{}, true);
+    if (most <= 4) settle(std::integral_constant<int, 3>{}, std::false_type{});
+    else if (most <= 6) settle(std::integral_constant<int, 5>{}, std::false_type{});
+    else if (most <= SIDE + 1) settle(std::integral_constant<int, SIDE>{}, std::false_type{});
+    else settle(std::integral_constant<int, 0>{}, std::true_type{});
     if constexpr (KEYS_MOVE) {
       __syncthreads();  // the codes have been read out of the room the keys take now
       each_round([&](int r, uint32_t p) { s_keys[p] = e[r]; });
