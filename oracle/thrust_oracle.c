@@ -77,6 +77,13 @@ static void reverse_sz(size_t* x, size_t n) {
   }
 }
 
+/* Shape of the reductions: nprocs == 1 is the sequential system, nprocs <= 0 the OpenMP system with
+ * omp_get_num_procs() processors (which may be one), as the reference does. */
+#define SEQUENTIAL 0L
+static long reduce_procs(int nprocs) {
+  return nprocs == 1 ? SEQUENTIAL : nprocs > 0 ? nprocs : omp_get_num_procs();
+}
+
 #define T int8_t
 #define U uint8_t
 #define S i8
@@ -189,10 +196,10 @@ static size_t dtype_size(int dtype) {
   return (dtype >= 0 && dtype < 10) ? sz[dtype] : 0;
 }
 
-/* nprocs <= 0: omp_get_num_procs(), as the reference does. */
+/* nprocs: see reduce_procs */
 ORACLE_API int oracle_reduce(const void* in, uint64_t n, int dtype, int op, const void* init,
                              void* out, int nprocs) {
-  const long P = nprocs > 0 ? nprocs : omp_get_num_procs();
+  const long P = reduce_procs(nprocs);
 #define BODY(S, T) *(T*)out = reduce_##S((const T*)in, (size_t)n, *(const T*)init, op, P);
   DISPATCH(dtype, BODY)
 #undef BODY
@@ -459,7 +466,7 @@ ORACLE_API int oracle_reduce_by_key(const void* keys_in, const void* values_in, 
  * iterator's difference type with plus; the transform is the same 0/1 map copy_if uses. */
 ORACLE_API int oracle_count_if(const void* in, uint64_t n, int dtype, int cmp, const void* threshold,
                                uint64_t* count, int nprocs) {
-  const long P = nprocs > 0 ? nprocs : omp_get_num_procs();
+  const long P = reduce_procs(nprocs);
   unsigned* flags = (unsigned*)malloc((n ? n : 1) * sizeof(unsigned));
 #define BODY(S, T) \
   pred_flags_##S((const T*)in, (size_t)n, cmp, threshold ? *(const T*)threshold : (T)0, flags);
@@ -532,7 +539,7 @@ ORACLE_API int oracle_set_operation_by_key(int op, const void* ka, uint64_t na, 
  * (generic/transform_scan.inl:37-97): the system's scans over it. */
 ORACLE_API int oracle_transform_reduce(const void* in, uint64_t n, int dtype, int unary, int op,
                                        const void* init, void* out, int nprocs) {
-  const long P = nprocs > 0 ? nprocs : omp_get_num_procs();
+  const long P = reduce_procs(nprocs);
 #define BODY(S, T)                                                     \
   T* f = transformed_##S((const T*)in, (size_t)n, unary);              \
   *(T*)out = reduce_##S(f, (size_t)n, *(const T*)init, op, P);         \
@@ -566,7 +573,7 @@ ORACLE_API int oracle_transform_exclusive_scan(const void* in, void* out, uint64
 
 ORACLE_API int oracle_inner_product(const void* a, const void* b, uint64_t n, int dtype,
                                     const void* init, void* out, int nprocs) {
-  const long P = nprocs > 0 ? nprocs : omp_get_num_procs();
+  const long P = reduce_procs(nprocs);
 #define BODY(S, T) \
   *(T*)out = inner_product_##S((const T*)a, (const T*)b, (size_t)n, *(const T*)init, P);
   DISPATCH(dtype, BODY)

@@ -346,6 +346,33 @@ def test_reduce_and_scan_are_sums_modulo_2k(oracle):
         assert int(ex[0]) == 9 and (int(ex[-1]) - (9 + total - exact[-1])) % (1 << bits) == 0
 
 
+def test_openmp_reduce_with_one_processor_is_not_the_sequential_fold():
+    """With one processor OpenMP still adds init to the finished sum (omp/detail/reduce.inl:37-65); the sequential
+    system folds from init (sequential/reduce.h)."""
+    import subprocess
+    import sys
+    code = """
+import os
+os.sched_setaffinity(0, {min(os.sched_getaffinity(0))})
+import numpy as np
+from oracle import cpu
+x, init = (np.arange(2000) % 7 + 0.1).astype(np.float32), np.float32(1e6)
+total = x[0]
+for v in x[1:]:
+    total = np.float32(total + v)
+fold = init
+for v in x:
+    fold = np.float32(fold + v)
+openmp = np.float32(init + total)
+assert openmp != fold
+assert cpu.Oracle().reduce(x, init=init) == openmp
+assert cpu.Oracle(nthreads=1).reduce(x, init=init) == fold
+"""
+    res = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                         capture_output=True, text=True, timeout=120)
+    assert res.returncode == 0, res.stderr
+
+
 def test_reduce_is_independent_of_chunk_count_for_integers():
     x = datagen.c1_int32(100000)
     vals = {cpu.Oracle(nthreads=p).reduce(x) for p in (1, 2, 3, 7, 8, 64)}
