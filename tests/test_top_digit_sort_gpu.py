@@ -144,3 +144,48 @@ def test_sorts_by_top_digits(dev, dtype, kind):
                 dev.sort_pairs(k, w, descending=descending, temp=temp)
                 assert np.array_equal(k.numpy().view(np.uint8), x[order].view(np.uint8)), (n, vdtype, descending)
                 assert np.array_equal(w.numpy(), v[order]), (n, vdtype, descending)
+
+
+# Sizes up to which the last step fits one digit, tiles are small, and pairs of 4-byte keys run two workgroups per CU
+# (SortPlan and sort_impl in thrust_amd/csrc/radix_sort.hip), and where the two-digit way ends.
+EDGES = [(np.uint32, None, 256 * 6144), (np.int32, np.uint16, 256 * 6144), (np.float32, np.uint32, 8 * 6144),
+         (np.int32, np.uint64, 256 * 2560), (np.float64, None, 1 << 19),
+         (np.uint8, None, 16384 * 160), (np.uint16, np.uint64, 8192 * 160), (np.uint32, None, 18432 * 160),
+         (np.int32, np.uint8, 16384 * 160), (np.uint64, np.uint32, 8192 * 160),
+         (np.uint32, np.uint8, 1 << 22), (np.int32, np.uint16, 1 << 22), (np.float32, np.uint32, 1 << 22),
+         (np.uint32, np.uint16, (1 << 24) - 1)]
+
+
+@pytest.mark.parametrize("dtype,vdtype,edge", EDGES)
+def test_sizes_where_the_kernels_change(dev, dtype, vdtype, edge):
+    for n in (edge, edge + 1):
+        bits = np.dtype(dtype).itemsize * 8
+        x = (datagen.splitmix64(7, n) >> np.uint64(64 - bits)).astype(f"u{bits // 8}").view(dtype)
+        if np.dtype(dtype).kind == "f":
+            x = np.where(np.isnan(x), dtype(1), x)
+        for descending in (False, True):
+            order = _order(x, descending)
+            k = dev.DeviceArray.from_numpy(x)
+            if vdtype is None:
+                dev.sort_keys(k, descending=descending)
+            else:
+                v = np.arange(n).astype(vdtype)
+                w = dev.DeviceArray.from_numpy(v)
+                dev.sort_pairs(k, w, descending=descending)
+                assert np.array_equal(w.numpy(), v[order]), (n, descending)
+            assert np.array_equal(k.numpy().view(np.uint8), x[order].view(np.uint8)), (n, descending)
+
+
+def test_long_stretches_among_many_keys(dev):
+    """2^25 eight-byte keys, four values 7000 times: the plan takes two digits, the tail sorts the windows that hold them."""
+    n = 1 << 25
+    x = datagen.splitmix64(8, n)
+    where = (datagen.splitmix64(9, 28_000) % np.uint64(n)).astype(np.int64)
+    x[where] = np.repeat(datagen.splitmix64(10, 4), 7000)
+    temp = dev.Temp()
+    k, w = dev.DeviceArray.from_numpy(x), dev.DeviceArray.from_numpy(np.arange(n, dtype=np.uint32))
+    dev.sort_pairs(k, w, temp=temp)
+    order = _order(x, False)
+    assert np.array_equal(k.numpy(), x[order]) and np.array_equal(w.numpy(), order.astype(np.uint32))
+    control = _control(temp)
+    assert control["fast"] == 2 and control["long_windows"] >= 4, control
