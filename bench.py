@@ -323,7 +323,7 @@ def main():
                                                    "storage, kept clean by the kernel itself, one launch per call"},
         # before and after the sort, each the mean of >= 50 back-to-back calls; "ms" above is the mean of the two
         "reduce_scan_passes": c1_passes,
-        "roofline": {"bound": "hbm", "kernel": "onesweep_pass (one of 2 per sort of these keys)",
+        "roofline": {"bound": "hbm", "kernel": "onesweep_pass (one of 4 per sort)",
                      "achieved": round(pass_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(pass_gbs / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": traffic_source,
                      "launch_ms": round(pass_ms, 4)},

@@ -89,6 +89,13 @@ def run_c2_float(torch, capi, reps):
     return {"c2_sort_f32_2p28": _row(med, mn, 36 * n, Gkeys_per_s=round(n / med / 1e6, 2), model="36 B/key")}
 
 
+def _launches_of_last_sort(temp):
+    """(digit passes that ran, 1 if the last step of the short way did) of the radix sort that used `temp` last: its
+    control block (csrc/sort_ctl.hpp) lies at the start."""
+    words = temp.buf[:11 * 4].cpu().numpy().view("uint32")
+    return int(((words[:8] & 15) == 1).sum()), int(words[10] != 0)
+
+
 def run_c3(torch, capi, reps):
     m = 1 << 27
     rows = {}
@@ -111,12 +118,13 @@ def run_c3(torch, capi, reps):
         if not ok:
             _fail(f"C3 sort_by_key {kind}")
         # passes over a digit that is the same in every key move nothing (the reference's sequential radix
-        # sort skips them too): the bytes of the call are the histogram read and the passes that run
-        passes_run = sum(1 for p in range(8) if int(((keys >> (8 * p)) & 0xFF).min().item())
-                         != int(((keys >> (8 * p)) & 0xFF).max().item()))
+        # sort skips them too), and random keys need two passes and the last step: the bytes of the call are the
+        # histogram read and what runs
+        passes_run, last_step = _launches_of_last_sort(t)
         rows[f"c3_sort_by_key_u64_u32_2p27_{kind}"] = _row(
-            med, mn, (8 + 24 * passes_run) * m, Gpairs_per_s=round(m / med / 1e6, 2), passes_run=passes_run,
-            model="8 B/pair histogram read + 24 B/pair per pass that runs (all 8: 200 B/pair)")
+            med, mn, (8 + 24 * (passes_run + last_step)) * m, Gpairs_per_s=round(m / med / 1e6, 2), passes_run=passes_run,
+            last_step_run=bool(last_step),
+            model="8 B/pair histogram read + 24 B/pair per pass that runs and for the last step, if it runs")
         del keys, vals, sk, sv, wk, wv, t, ko, vo, o, same
     return rows
 
