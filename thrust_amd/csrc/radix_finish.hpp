@@ -11,12 +11,13 @@
 // largest falls into the last bins): one LDS atomic per key counts a bin and tells the key its place in it, a scan
 // turns counts into starts, the keys are laid out by bin, and each key counts the keys of its bin that belong in front
 // of it -- the smaller ones and, among equal ones, those that stood in front -- so the atomics' order does not show.
-// What bounds it: vector instructions (90 per key and lane) and, for 2000 keys a workgroup, the latency of its ten
-// steps; LDS is busy 40 % of the time.  2^27 (uint64, uint32): 0.85 ms (3.8 TB/s) in place of six passes of 0.65.
-// Workgroups that loop over windows save their dispatch where the chained passes do the sort, but cost
-// registers (0.85 -> 1.19 ms).
+// What bounds it: the latency of its ten steps for the 2000 keys of a workgroup, three workgroups to a CU, and vector
+// instructions: 142 per pair of (uint64, uint32) keep the SIMDs half busy; LDS is busy 28 % of the time.  2^27 pairs: 0.97 ms
+// (3.3 TB/s) in place of six passes of 0.69; keys alone 0.65 in place of six of 0.48.  Workgroups that loop over windows
+// save their dispatch where the chained passes do the sort (40 us for 2^27 keys), but cost registers (0.85 -> 1.19 ms).
 // A bin of more than FINISH_BIN_MAX keys (many equal keys, values in clusters) makes the workgroup run stable passes
-// over the digits that vary instead.
+// over the digits that vary instead: three times as long for 2^27 uint64 that repeat 30 times (the sort still takes 0.8
+// of the time of all passes).
 #pragma once
 #include "common.hpp"
 #include "launch.hpp"
@@ -428,7 +429,9 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
 // The windows that do not fit a workgroup of the last step: stable passes over the digits that vary in the window,
 // between the place of the window in the two buffers (its own in either, so nobody else reads or writes them).
 // Tiles of TAIL_BLOCK * TAIL_ITEMS keys are ranked as in a chained pass, one after the other, so the order of the tiles
-// needs no look-back.  Bound by latency: one workgroup has nothing else to do meanwhile.
+// needs no look-back.  Bound by latency: one workgroup has nothing else to do meanwhile.  A sort of 2^27 uint64 with one
+// value 1e4 times takes 2.09 ms, 1.96 without it, 4.14 with all digits' passes.  The plan bounds a window's keys: c equal
+// prefixes weigh c / n in both digits, and the product of the heaviest shares times n fits a workgroup.
 // Where no window is left over it copies the result back if it sits in the alternate buffer, or does nothing.
 constexpr int TAIL_BLOCK = 1024;
 constexpr int TAIL_ITEMS = 8;

@@ -1,7 +1,8 @@
 // thrust_amd_sort_keys / thrust_amd_sort_pairs: onesweep least-significant-digit radix sort (up to 8192
 // keys: one workgroup, small_sort.hpp).
 //
-//   init       zeroes the digit histograms, the per-pass tile descriptors and tickets
+//   init       zeroes the digit histograms, the tickets and the tile descriptors of the passes (of the first one or two,
+//              where the short way is open: the last step clears the others if they are needed)
 //   histogram  one read of the keys builds the 256-bin histogram of EVERY 8-bit digit
 //   plan       exclusive scan of each histogram -> global digit offsets; a digit whose one
 //              bin holds all n keys is marked "skip" (the reference's sequential radix
@@ -12,7 +13,7 @@
 //   pass x P   chained digit-binning pass ("onesweep"): a tile ranks its keys by digit,
 //              learns the global offset of each of its 256 digit runs by decoupled
 //              look-back over the tiles before it, and scatters keys (and values)
-//   copy-back  only if an odd number of passes ran
+//   copy-back  only if an odd number of passes ran (8-byte keys: in the launch of the short way's tail)
 //
 // Ranking inside a tile uses the wave64 match pattern (radix_rank.hpp): rank = wave-private LDS counter
 // + number of peers in lower lanes.  Lanes hold keys wave-striped (lane l of wave w holds
@@ -26,8 +27,8 @@
 // 32-bit words for n < 2^30 keys and 64-bit words up to the limit of 2^32 - 1 keys per call
 // (positions and histogram counts are 32-bit).
 //
-// Algorithmic HBM traffic for K-byte keys, V-byte values, P = K passes:
-// K*n (histogram) + P * 2*(K+V)*n.  Replaces cub::DeviceRadixSort as called from
+// Algorithmic HBM traffic for K-byte keys, V-byte values and P digits that vary: K*n (histogram) + P * 2*(K+V)*n;
+// by the short way with one or two digits D: K*n + (D + 1) * 2*(K+V)*n.  Replaces cub::DeviceRadixSort as called from
 // thrust/system/cuda/detail/sort.h:1326-1508.
 #include "common.hpp"
 #include "dispatch.hpp"
@@ -715,7 +716,9 @@ struct SortPlan {
                                                                                  : 16;
   static constexpr int TILE = BLOCK * ITEMS;
   // Where tiles of this size are fewer than the CUs: a third or half of it.  The time is that of one or two tiles
-  // then, and shorter with smaller ones (copy and sort of 1e6 float32 75 -> 65 us, 2.1e6 90 -> 84; 4e6 106 -> 110).
+  // then, and shorter with smaller ones.  Sort of 1e6 and 2.6e6 random keys, large tiles against small ones: float32 76 -> 65,
+  // 97 -> 93 us; with uint32 values 86 -> 75, 102 -> 94; uint8 29.4 -> 27.5, 34.3 -> 34.3; uint16 42.6 -> 38.8, 50.6 -> 50.5;
+  // (uint16, uint64) 47 -> 45, and 51.5 -> 51.7 at 1.6e6; float64 137 -> 130 at 1e6.  Float32 at 4e6: 106 -> 110.
   static constexpr int FINE_ITEMS = ITEMS == 8 ? 4 : 6;
   static constexpr uint64_t FINE_MAX = (uint64_t)TILE * NUM_CU * 5 / 8;
   // 4-byte keys with values need 74 registers, a workgroup per CU.  Two with 64 and 36 bytes of spills each win while
@@ -748,15 +751,18 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   const bool wide = n > SORT_MAX_N_NARROW;  // prefixes need more than 30 bits: 64-bit descriptors
   // every key and value within 4 GiB of its array's start: 32-bit byte offsets
   const bool off32 = !wide && n * (uint64_t)((HAS_VALUES && sizeof(V) > sizeof(K)) ? sizeof(V) : sizeof(K)) <= (1ull << 32);
-  // The short way, over whole keys only.  Against all digits' passes, copy and sort of random keys back to back:
-  //   8-byte keys      9001 keys 80 -> 51 us, 1e6 135 -> 85, 8e6 315 -> 189, 1.28e8 4330 -> 2226; with 4-byte values
-  //                    89 -> 63, 159 -> 91, 398 -> 239, 6188 -> 3033 us
-  //   4-byte integers  by one digit (as long as its bins can fit at all) 9001 keys 58 -> 41 us, 1.5e6 83 -> 62; with
-  //                    values 64 -> 46, 99 -> 72.  Never by two digits: that saves two passes and costs the last step,
+  // The short way, over whole keys only.  Against all digits' passes, sort of random keys:
+  //   8-byte keys      1e4 keys 84 -> 48 us, 1e6 135 -> 79, 8e6 309 -> 166, 1.34e8 4130 -> 1960; with 4-byte values
+  //                    92 -> 49, 157 -> 86, 363 -> 197, 5790 -> 2700 us; where keys repeat 10 to 30 times 0.66-0.85 of the
+  //                    time, where the plan declines 1.00-1.05 (5 to 10 us up to 8e6 keys, 1 % at 1.34e8; 1.04-1.09 where
+  //                    one digit varies): two launches that do nothing, one of them of a workgroup per window
+  //   4-byte integers  by one digit (as long as its bins can fit at all) 1e4 keys 68 -> 40 us, 1e6 75 -> 49; with
+  //                    values 70 -> 41, 85 -> 55.  Never by two digits: that saves two passes and costs the last step,
   //                    0.95-1.06 times as fast for random keys of 2^25 and more, and where keys repeat (ten times or a
-  //                    thousand) their stretches outgrow a workgroup after the passes have run: 2^28 keys 2170 -> 3220 us.
+  //                    thousand) the stretches outgrow a workgroup: 2^28 keys 2170 -> 3220 us when all passes follow.
   //   floats           share few exponents: 4-byte ones outgrow a workgroup at some 20000 keys, 8-byte ones (four
   //                    bits of mantissa in two digits) at a few 100000.
+  // It ends where random keys' stretches of two digits come near STRETCH_MAX (1.5e8 keys); a third digit would carry on.
   using Finish = FinishShape<K, V, HAS_VALUES>;
   const bool is_float = dtype == THRUST_AMD_F32 || dtype == THRUST_AMD_F64;
   const bool two_digits = sizeof(K) == 8 && (!is_float || n <= (1u << 19));
