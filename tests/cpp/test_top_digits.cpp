@@ -14,7 +14,7 @@
 constexpr float STRETCH_MAX = 2560;
 
 // Keys are drawn by draw(rnd); as the plan kernel counts them.  hot_share: share of one key among them.
-static float verdict(double n, uint32_t bins, double values, double hot_share, uint32_t seed) {
+static float longest_stretch(double n, uint32_t bins, double values, double hot_share, uint32_t seed) {
   std::mt19937_64 rnd(seed);
   const uint32_t samples = (uint32_t)std::min(n / 64, 16384.0);
   std::vector<uint32_t> count(bins, 0);
@@ -46,7 +46,7 @@ int main() {
   for (double n : {9e3, 3e4, 1e5, 1e6, 4e6, 1.6e7, 3.3e7, 6.7e7, 1.34e8, 1.5e8}) {
     int declined = 0;
     for (uint32_t seed = 1; seed <= 40; ++seed) {
-      const float longest = verdict(n, 65536, random_values, 0, seed);
+      const float longest = longest_stretch(n, 65536, random_values, 0, seed);
       const double expected = n / 65536 + 3.5 * std::sqrt(n / 65536);
       if (longest == 0) ++declined;
       else if (longest < expected) {
@@ -67,7 +67,7 @@ int main() {
                         Case{6.7e7, 6.7e4, 0, "1000 copies of each key"}, Case{1e6, random_values, 0.05, "a key that is one in twenty"},
                         Case{1e6, random_values, 0.005, "a key that is one in 200"}, Case{1.34e8, random_values, 0.01, "a key that is one in 100"}}) {
     int taken = 0;
-    for (uint32_t seed = 1; seed <= 40; ++seed) taken += verdict(c.n, 65536, c.values, c.hot, seed) > 0 ? 1 : 0;
+    for (uint32_t seed = 1; seed <= 40; ++seed) taken += longest_stretch(c.n, 65536, c.values, c.hot, seed) > 0 ? 1 : 0;
     if (taken > 2) {
       std::printf("FAILED: %g keys, %s: taken %d times of 40\n", c.n, c.what, taken);
       ++failures;
