@@ -72,6 +72,29 @@ def test_scans_int_bit_exact(dev, oracle, dtype):
         assert np.array_equal(dev.exclusive_scan(d, 5).numpy(), oracle.exclusive_scan(x, 5)), (dtype, n)
 
 
+def _edges(dtype):
+    """Sizes around the ends of one workgroup's tile, of the tiles of two launches and of their range, and of the reduction by one workgroup."""
+    size = np.dtype(dtype).itemsize
+    one, two = (128 << 10) // size, (16 << 10) // size
+    most_two, most_reduce = (64 << 20) // size, (512 << 10) // size
+    for edge in (one, one + two, 3 * one, most_reduce, most_two):
+        yield from (edge - 1, edge, edge + 1)
+
+
+@pytest.mark.parametrize("dtype", [np.int8, np.uint16, np.int32, np.uint64])
+def test_scan_and_reduce_at_the_edges_of_their_shapes(dev, dtype):
+    for n in _edges(dtype):
+        x = _ints(n, dtype, 57)
+        for skip in (0, 1):  # the second call's array does not begin on 16 bytes
+            d = dev.DeviceArray(n - skip, dev.DTYPE_OF_NP[np.dtype(dtype)], dev.DeviceArray.from_numpy(x).storage[skip * x.itemsize:])
+            sums = np.cumsum(x[skip:], dtype=dtype)
+            assert np.array_equal(dev.inclusive_scan(d).numpy(), sums), (dtype, n, skip)
+            shifted = np.concatenate([np.zeros(1, dtype), sums[:-1]]) + dtype(3)
+            assert np.array_equal(dev.exclusive_scan(d, 3).numpy(), shifted), (dtype, n, skip)
+            assert dev.reduce(d, dev.PLUS, 0).numpy()[0] == sums[-1], (dtype, n, skip)
+            assert dev.reduce(d, dev.MIN, 127).numpy()[0] == min(x[skip:].min(), 127), (dtype, n, skip)
+
+
 def test_scan_in_place_and_unaligned(dev, oracle):
     x = _ints(70001, np.int32, 23)
     d = dev.DeviceArray.from_numpy(x)

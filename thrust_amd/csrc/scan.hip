@@ -63,12 +63,17 @@ static int scan_static_setup(ScanStaticDevice& dev) {
   return 0;
 }
 
+struct ScanStaticSize {  // bytes of descriptors
+  template <typename T, typename Op>
+  static int run(size_t* need, uint64_t n) {
+    return ScanLaunch<false, UnIdentity>::run_kept_clean<T, Op>(nullptr, need, nullptr, nullptr, n, nullptr);
+  }
+};
 struct ScanStaticLaunch {
   template <typename T, typename Op>
   static int run(void* scratch, const void* in, void* out, uint64_t n, hipStream_t stream) {
     size_t bytes = SCAN_STATIC_SCRATCH_BYTES;
-    return ScanLaunch<false, UnIdentity>::run<T, Op>(scratch, &bytes, in, out, n, nullptr, stream,
-                                                     /*kept_clean=*/true);
+    return ScanLaunch<false, UnIdentity>::run_kept_clean<T, Op>(scratch, &bytes, in, out, n, stream);
   }
 };
 
@@ -78,7 +83,8 @@ TA_EXPORT int thrust_amd_inclusive_scan_static(const void* in, void* out, uint64
                                                int op, void* stream) {
   using namespace ta;
   size_t need = 0;
-  const int rc = thrust_amd_inclusive_scan(nullptr, &need, in, out, n, dtype, op, stream);
+  if (!valid_dtype(dtype) || !valid_binop(op)) return (int)hipErrorInvalidValue;
+  const int rc = dispatch_dtype_op<ScanStaticSize>(dtype, op, &need, n);
   if (rc) return rc;
   if (need > SCAN_STATIC_SCRATCH_BYTES) return (int)hipErrorInvalidValue;  // n beyond the fixed scratch
   if (n == 0) return 0;

@@ -11,7 +11,8 @@
 // chained by the wave total, then one cross-wave step through LDS.
 //
 // HBM traffic: n*sizeof(T) read + n*sizeof(T) written; tile descriptors add
-// 8*W bytes per tile (W = 32-bit words of T).
+// 8*W bytes per tile (W = 32-bit words of T).  Short arrays take one or two launches without
+// look-back instead (below); what they read twice comes from the caches the second time.
 #pragma once
 #include "common.hpp"
 #include "dispatch.hpp"
@@ -19,12 +20,24 @@
 
 namespace ta {
 
-// Tile shapes (threads x 16-byte vectors per lane).  The per-tile cost of the ticket
-// (a same-address atomic retires every ~12 ns on MI355X) and of the look-back makes large
-// tiles win once there are enough of them to fill 256 CUs; small inputs use small tiles.
+// Tile shapes (threads x 16-byte vectors per lane) of the single-pass kernel.  The per-tile cost of
+// the ticket (a same-address atomic retires every ~12 ns on MI355X) and of the look-back makes
+// large tiles win; the small ones are left to short arrays in storage that is kept clean.
 struct ScanShapeLarge { static constexpr int BLOCK = 1024, CHUNKS = 12; };
 struct ScanShapeSmall { static constexpr int BLOCK = 256, CHUNKS = 4; };
 constexpr uint64_t SCAN_LARGE_MIN_BYTES = (uint64_t)32 << 20;
+
+// Arrays below SCAN_TWO_MAX_BYTES are scanned by two launches that wait for nothing (scan_partials_kernel,
+// scan_apply_kernel): their second read of the input meets the caches, and no tile queues at the ticket.
+// Whole call in us, single pass with its better shape against two launches: 4 MB of int32 10.4 -> 9.7,
+// 16 MB 15.6 (27 with the shape it took) -> 11.3, 32 MB 26 (46) -> 17, 64 MB 35.8 -> 31.7, 128 MB 51 -> 58;
+// int64 8 MB 12 (17) -> 9.7, 32 MB 18 (48) -> 17.7, 64 MB 31.8 -> 32.2, 128 MB 54 -> 60.
+// Tiles of 64 KiB instead of 16: 64 MB 32.5, the others alike.
+struct ScanShapeTwo { static constexpr int BLOCK = 256, CHUNKS = 4; };
+constexpr uint64_t SCAN_TWO_MAX_BYTES = (uint64_t)64 << 20;
+// An array that fits one workgroup of this shape (128 KiB) takes the second launch alone: 32768 int32
+// 9.7 -> 6.8 us with its host call, which is what both figures are made of.
+struct ScanShapeOne { static constexpr int BLOCK = 1024, CHUNKS = 8; };
 
 static __global__ void tile_state_init_kernel(uint64_t* __restrict__ words, uint64_t count,
                                        uint32_t* __restrict__ counters, uint32_t num_counters) {
@@ -202,56 +215,249 @@ __global__ __launch_bounds__(Shape::BLOCK) void scan_kernel(const T* in, T* out,
   }
 }
 
+// ------------------------------------------------------------------ two launches
+// Vector j of a lane in a tile of which `valid` elements exist (its last tile): a whole vector where the
+// wave's vectors j exist altogether, else elements, none past the last one; what does not exist becomes id.
+template <bool ALIGNED, typename T, typename Pre>
+TA_DEVICE Vec16<T> scan_load_ragged(const T* tile, uint32_t first, uint32_t wave_first, uint32_t valid, T id, Pre pre) {
+  constexpr int VEC = Vec16<T>::N;
+  Vec16<T> x;
+  if (wave_first + WAVE * VEC <= valid) {
+    x = load_vec<ALIGNED>(tile + first);
+  } else {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) x.v[i] = tile[first + i < valid ? first + i : valid - 1];
+  }
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) x.v[i] = (first + i < valid) ? pre(x.v[i]) : id;
+  return x;
+}
+
+// First launch: the fold of every tile but the last one.
+template <typename T, typename Op, typename Pre, bool ALIGNED, typename Shape>
+__global__ __launch_bounds__(Shape::BLOCK) void scan_partials_kernel(const T* __restrict__ in, T* __restrict__ partials) {
+  constexpr int VEC = Vec16<T>::N;
+  const Op op;
+  const Pre pre;
+  const T* tile = in + (uint64_t)blockIdx.x * (Shape::BLOCK * Shape::CHUNKS * VEC);
+  Vec16<T> x[Shape::CHUNKS];
+#pragma unroll
+  for (int j = 0; j < Shape::CHUNKS; ++j) x[j] = load_vec<ALIGNED>(tile + (j * Shape::BLOCK + threadIdx.x) * VEC);
+  T acc[VEC];
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) acc[i] = pre(x[0].v[i]);
+#pragma unroll
+  for (int j = 1; j < Shape::CHUNKS; ++j) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) acc[i] = op(acc[i], pre(x[j].v[i]));
+  }
+#pragma unroll
+  for (int i = 1; i < VEC; ++i) acc[0] = op(acc[0], acc[i]);
+  __shared__ T s_wave[Shape::BLOCK / WAVE];
+  const T wave_total = wave_reduce(acc[0], op);
+  if (threadIdx.x % WAVE == 0) s_wave[threadIdx.x / WAVE] = wave_total;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    T total = s_wave[0];
+#pragma unroll
+    for (int w = 1; w < Shape::BLOCK / WAVE; ++w) total = op(total, s_wave[w]);
+    partials[blockIdx.x] = total;
+  }
+}
+
+// Second launch: every tile folds the partials of the tiles before it (they fit the caches, and arrive
+// while its own elements do) and scans its elements.  A call of one tile needs nothing but this launch.
+template <typename T, typename Op, typename Pre, bool EXCLUSIVE, bool ALIGNED, typename Shape>
+__global__ __launch_bounds__(Shape::BLOCK) void scan_apply_kernel(const T* in, T* out, uint64_t n, T init,
+                                                                  const T* __restrict__ partials) {
+  constexpr int SCAN_BLOCK = Shape::BLOCK;
+  constexpr int SCAN_CHUNKS = Shape::CHUNKS;
+  constexpr int VEC = Vec16<T>::N;
+  constexpr int WAVES = SCAN_BLOCK / WAVE;
+  constexpr uint32_t WAVE_SPAN = WAVE * SCAN_CHUNKS * VEC;
+  constexpr uint32_t TILE = WAVES * WAVE_SPAN;
+  const Op op;
+  const Pre pre;
+  const T id = Op::template identity<T>();
+  __shared__ T s_wave_agg[WAVES];
+  __shared__ T s_before[WAVES];
+
+  const uint32_t tile = blockIdx.x;
+  const uint64_t tile_base = (uint64_t)tile * TILE;
+  const uint32_t valid = (uint32_t)((n - tile_base < TILE) ? (n - tile_base) : TILE);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+  const int lane = threadIdx.x % WAVE;
+  const uint32_t lane_off = wave * WAVE_SPAN + lane * VEC;
+
+  Vec16<T> x[SCAN_CHUNKS];
+  if (valid == TILE) {
+#pragma unroll
+    for (int j = 0; j < SCAN_CHUNKS; ++j) x[j] = load_vec<ALIGNED>(in + tile_base + lane_off + j * (WAVE * VEC));
+  } else {
+#pragma unroll
+    for (int j = 0; j < SCAN_CHUNKS; ++j) {
+      const uint32_t wave_first = wave * WAVE_SPAN + j * (WAVE * VEC);
+      if (wave_first < valid) {
+        x[j] = scan_load_ragged<ALIGNED>(in + tile_base, lane_off + j * (WAVE * VEC), wave_first, valid, id, pre);
+      } else {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) x[j].v[i] = id;
+      }
+    }
+  }
+  T before = id;
+  for (uint32_t t = threadIdx.x; t < tile; t += SCAN_BLOCK) before = op(before, partials[t]);
+  if (valid == TILE) {
+#pragma unroll
+    for (int j = 0; j < SCAN_CHUNKS; ++j) {
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) x[j].v[i] = pre(x[j].v[i]);
+    }
+  }
+
+  // ---- wave-local scan in place, as in scan_kernel
+  T carry = id;
+#pragma unroll
+  for (int j = 0; j < SCAN_CHUNKS; ++j) {
+    T s = x[j].v[0];
+#pragma unroll
+    for (int i = 1; i < VEC; ++i) s = op(s, x[j].v[i]);
+    const T incl = wave_inclusive_scan(s, op, id);
+    T run = op(carry, wave_shift_up(incl, id));
+    carry = op(carry, readlane(incl, WAVE - 1));
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      const T next = op(run, x[j].v[i]);
+      x[j].v[i] = EXCLUSIVE ? run : next;
+      run = next;
+    }
+  }
+  before = wave_reduce(before, op);
+  if (lane == 0) {
+    s_wave_agg[wave] = carry;
+    s_before[wave] = before;
+  }
+  __syncthreads();
+  T wave_prefix = id;
+  T prefix = id;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    if (w < wave) wave_prefix = op(wave_prefix, s_wave_agg[w]);
+    prefix = op(prefix, s_before[w]);
+  }
+  if constexpr (EXCLUSIVE) prefix = (tile == 0) ? init : op(init, prefix);
+  prefix = op(prefix, wave_prefix);
+#pragma unroll
+  for (int j = 0; j < SCAN_CHUNKS; ++j) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) x[j].v[i] = op(prefix, x[j].v[i]);
+    const uint32_t wave_first = wave * WAVE_SPAN + j * (WAVE * VEC);
+    T* dst = out + tile_base + lane_off + j * (WAVE * VEC);
+    if (wave_first + WAVE * VEC <= valid) {
+      store_vec<ALIGNED>(dst, x[j]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        if (lane_off + j * (WAVE * VEC) + i < valid) dst[i] = x[j].v[i];
+      }
+    }
+  }
+}
+
 template <bool EXCLUSIVE, typename Pre>
 struct ScanLaunch {
-  // kept_clean: `temp` is storage of the library's own that only this function uses and that was all
-  // zero to begin with; the kernel then clears up after itself and no clearing launch precedes it.
-  template <typename T, typename Op, typename Shape>
-  static int run_shape(void* temp, size_t* temp_bytes, const void* in, void* out, uint64_t n,
-                       const void* init, hipStream_t stream, bool kept_clean = false) {
+  template <typename Shape, typename T>
+  static constexpr uint64_t tile_of() { return (uint64_t)Shape::BLOCK * Shape::CHUNKS * Vec16<T>::N; }
+
+  // The single-pass kernel.  KEPT_CLEAN: `temp` is storage of the library's own that only this function uses
+  // and that was all zero to begin with; the kernel then clears up after itself and no clearing launch precedes it.
+  template <typename T, typename Op, typename Shape, bool KEPT_CLEAN>
+  static int run_single_pass(void* temp, size_t* temp_bytes, const T* in, T* out, uint64_t n, const void* init,
+                             hipStream_t stream) {
     constexpr int W = TileWords<T>::W;
-    constexpr uint64_t TILE = (uint64_t)Shape::BLOCK * Shape::CHUNKS * Vec16<T>::N;
-    const uint64_t tiles = (n + TILE - 1) / TILE;
+    const uint64_t tiles = (n + tile_of<Shape, T>() - 1) / tile_of<Shape, T>();
     if (tiles > 0xffffffffull) return (int)hipErrorInvalidValue;
     TempLayout lay;
     const size_t off_ticket = lay.add(2 * sizeof(uint32_t));  // the ticket and the count of finished tiles
     const size_t off_status = lay.add((size_t)tiles * W * sizeof(uint64_t));
-    if (temp == nullptr) {
-      *temp_bytes = lay.total;
-      return 0;
-    }
-    if (*temp_bytes < lay.total) return (int)hipErrorInvalidValue;
-    if (n == 0) return 0;
-    if (!in || !out) return (int)hipErrorInvalidValue;
-    T init_v = Op::template identity<T>();
-    if (EXCLUSIVE) {
-      if (!init) return (int)hipErrorInvalidValue;
-      __builtin_memcpy(&init_v, init, sizeof(T));
-    }
+    T init_v;
+    const int rc = check_args<T, Op>(temp, temp_bytes, lay.total, in, out, n, init, init_v);
+    if (rc != 0 || temp == nullptr || n == 0) return rc;
     uint32_t* ticket = reinterpret_cast<uint32_t*>(static_cast<char*>(temp) + off_ticket);
     uint64_t* status = reinterpret_cast<uint64_t*>(static_cast<char*>(temp) + off_status);
     const uint64_t words = tiles * W;
-    uint32_t* finished = kept_clean ? ticket + 1 : nullptr;
-    if (!kept_clean) {
+    uint32_t* finished = KEPT_CLEAN ? ticket + 1 : nullptr;
+    if (!KEPT_CLEAN) {
       TA_LAUNCH("tile_state_init", stream, tile_state_init_kernel, dim3((uint32_t)((words + 255) / 256)), dim3(256), status, words, ticket, 2u);
       TA_CHECK_LAUNCH();
     }
-    const T* src = static_cast<const T*>(in);
-    T* dst = static_cast<T*>(out);
     if (is_aligned16(in) && is_aligned16(out))
-      TA_LAUNCH("scan", stream, (scan_kernel<T, Op, Pre, EXCLUSIVE, true, Shape>), dim3((uint32_t)tiles), dim3(Shape::BLOCK), src, dst, n, init_v, status, ticket, finished);
+      TA_LAUNCH("scan", stream, (scan_kernel<T, Op, Pre, EXCLUSIVE, true, Shape>), dim3((uint32_t)tiles), dim3(Shape::BLOCK), in, out, n, init_v, status, ticket, finished);
     else
-      TA_LAUNCH("scan", stream, (scan_kernel<T, Op, Pre, EXCLUSIVE, false, Shape>), dim3((uint32_t)tiles), dim3(Shape::BLOCK), src, dst, n, init_v, status, ticket, finished);
+      TA_LAUNCH("scan", stream, (scan_kernel<T, Op, Pre, EXCLUSIVE, false, Shape>), dim3((uint32_t)tiles), dim3(Shape::BLOCK), in, out, n, init_v, status, ticket, finished);
     TA_CHECK_LAUNCH();
     return 0;
   }
 
+  // One launch where the array is one tile, else two; `temp` holds the partials of the tiles.
+  template <typename T, typename Op, typename Shape>
+  static int run_two_launches(void* temp, size_t* temp_bytes, const T* in, T* out, uint64_t n, const void* init,
+                              hipStream_t stream) {
+    const uint32_t tiles = (uint32_t)((n + tile_of<Shape, T>() - 1) / tile_of<Shape, T>());
+    TempLayout lay;
+    const size_t off_partials = lay.add((size_t)tiles * sizeof(T));
+    T init_v;
+    const int rc = check_args<T, Op>(temp, temp_bytes, lay.total, in, out, n, init, init_v);
+    if (rc != 0 || temp == nullptr || n == 0) return rc;
+    T* partials = reinterpret_cast<T*>(static_cast<char*>(temp) + off_partials);
+    if (tiles > 1) {
+      if (is_aligned16(in))
+        TA_LAUNCH("scan_partials", stream, (scan_partials_kernel<T, Op, Pre, true, Shape>), dim3(tiles - 1), dim3(Shape::BLOCK), in, partials);
+      else
+        TA_LAUNCH("scan_partials", stream, (scan_partials_kernel<T, Op, Pre, false, Shape>), dim3(tiles - 1), dim3(Shape::BLOCK), in, partials);
+      TA_CHECK_LAUNCH();
+    }
+    if (is_aligned16(in) && is_aligned16(out))
+      TA_LAUNCH("scan", stream, (scan_apply_kernel<T, Op, Pre, EXCLUSIVE, true, Shape>), dim3(tiles), dim3(Shape::BLOCK), in, out, n, init_v, (const T*)partials);
+    else
+      TA_LAUNCH("scan", stream, (scan_apply_kernel<T, Op, Pre, EXCLUSIVE, false, Shape>), dim3(tiles), dim3(Shape::BLOCK), in, out, n, init_v, (const T*)partials);
+    TA_CHECK_LAUNCH();
+    return 0;
+  }
+
+  // Answers the size query (temp null) and checks the arguments; reads the initial value where there is one.
   template <typename T, typename Op>
-  static int run(void* temp, size_t* temp_bytes, const void* in, void* out, uint64_t n,
-                 const void* init, hipStream_t stream, bool kept_clean = false) {
+  static int check_args(void* temp, size_t* temp_bytes, size_t need, const T* in, T* out, uint64_t n, const void* init, T& init_v) {
+    init_v = Op::template identity<T>();
+    if (temp == nullptr) {
+      *temp_bytes = need;
+      return 0;
+    }
+    if (*temp_bytes < need) return (int)hipErrorInvalidValue;
+    if (n == 0) return 0;
+    if (!in || !out || (EXCLUSIVE && !init)) return (int)hipErrorInvalidValue;
+    if (EXCLUSIVE) __builtin_memcpy(&init_v, init, sizeof(T));
+    return 0;
+  }
+
+  template <typename T, typename Op>
+  static int run(void* temp, size_t* temp_bytes, const void* in_, void* out_, uint64_t n, const void* init, hipStream_t stream) {
+    const T* in = static_cast<const T*>(in_);
+    T* out = static_cast<T*>(out_);
+    if (n > SCAN_TWO_MAX_BYTES / sizeof(T))
+      return run_single_pass<T, Op, ScanShapeLarge, false>(temp, temp_bytes, in, out, n, init, stream);
+    if (n <= tile_of<ScanShapeOne, T>())
+      return run_two_launches<T, Op, ScanShapeOne>(temp, temp_bytes, in, out, n, init, stream);
+    return run_two_launches<T, Op, ScanShapeTwo>(temp, temp_bytes, in, out, n, init, stream);
+  }
+
+  template <typename T, typename Op>
+  static int run_kept_clean(void* temp, size_t* temp_bytes, const void* in_, void* out_, uint64_t n, hipStream_t stream) {
+    const T* in = static_cast<const T*>(in_);
+    T* out = static_cast<T*>(out_);
     if (n * sizeof(T) >= SCAN_LARGE_MIN_BYTES)
-      return run_shape<T, Op, ScanShapeLarge>(temp, temp_bytes, in, out, n, init, stream, kept_clean);
-    return run_shape<T, Op, ScanShapeSmall>(temp, temp_bytes, in, out, n, init, stream, kept_clean);
+      return run_single_pass<T, Op, ScanShapeLarge, true>(temp, temp_bytes, in, out, n, nullptr, stream);
+    return run_single_pass<T, Op, ScanShapeSmall, true>(temp, temp_bytes, in, out, n, nullptr, stream);
   }
 };
 
