@@ -194,7 +194,8 @@ __global__ __launch_bounds__((RbkItems<K, V>::block), 4) void rbk_kernel(RbkArgs
   K* s_keys_out = reinterpret_cast<K*>(sh.keys_out);
   V* s_values_out = reinterpret_cast<V*>(sh.values_out);
 
-  if (threadIdx.x == 0) sh.tile = atomicAdd(a.ticket, 1u);
+  // (the ticket of a call of one tile has not been cleared)
+  if (threadIdx.x == 0) sh.tile = a.n > TILE ? atomicAdd(a.ticket, 1u) : 0u;
   __syncthreads();
   const uint32_t tile = sh.tile;
   const uint64_t tile_base = (uint64_t)tile * TILE;
@@ -370,11 +371,15 @@ inline int rbk_launch(char* temp, RbkArgs<K, V, Eq, Op> a, hipStream_t stream) {
               (reinterpret_cast<uintptr_t>(a.values) % alignof(RbkValueVec<V, RbkTemp<K, V>::VEC>)) == 0;
   const uint64_t words = lay.tiles * RbkTemp<K, V>::W;
   const uint64_t init_threads = words ? words : 1;
-  THRUST_AMD_KERNEL_LAUNCH("rbk_init", stream, rbk_init_kernel<0>, dim3((uint32_t)((init_threads + 255) / 256)), dim3(256),
-                           a.status, words, a.ticket, a.d_num_runs);
-  hipError_t e = hipPeekAtLastError();
-  if (e != hipSuccess) return (int)e;
-  if (a.n == 0) return 0;
+  // a call of one tile waits for no other tile: no descriptors to clear, one launch instead of two
+  // (4097 pairs, whole call: 15.7 -> 11.8 us)
+  if (lay.tiles != 1) {
+    THRUST_AMD_KERNEL_LAUNCH("rbk_init", stream, rbk_init_kernel<0>, dim3((uint32_t)((init_threads + 255) / 256)), dim3(256),
+                             a.status, words, a.ticket, a.d_num_runs);
+    const hipError_t e = hipPeekAtLastError();
+    if (e != hipSuccess) return (int)e;
+    if (a.n == 0) return 0;
+  }
   THRUST_AMD_KERNEL_LAUNCH("reduce_by_key", stream, (rbk_kernel<K, V, Eq, Op>), dim3((uint32_t)lay.tiles),
                            dim3(RbkTemp<K, V>::BLOCK), a);
   return (int)hipPeekAtLastError();

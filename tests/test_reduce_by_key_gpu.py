@@ -36,6 +36,22 @@ def test_integer_values_exact(dev, oracle, kdtype, vdtype):
         assert np.array_equal(ko.numpy(runs), rk) and np.array_equal(vo.numpy(runs), rv), (kdtype, vdtype, n)
 
 
+@pytest.mark.parametrize("vdtype", [np.int32, np.uint64])
+def test_calls_of_one_tile_and_their_neighbours(dev, oracle, vdtype):
+    """Up to one tile a call is a single launch on descriptors that nobody has cleared (filled with ones here)."""
+    import torch
+    temp = dev.Temp()
+    temp.buf = torch.full((1 << 16,), 255, dtype=torch.uint8, device="cuda")
+    for edge in (28, 64 * 28, 14336, 16384, 28672):
+        for n in (edge - 1, edge, edge + 1):
+            k = _keys(n, np.int32, 13, 5)
+            v = (datagen.splitmix64(15, n) >> np.uint64(20)).astype(vdtype)
+            dk, dv = dev.DeviceArray.from_numpy(k), dev.DeviceArray.from_numpy(v)
+            ko, vo, runs = dev.reduce_by_key(dk, dv, temp=temp)
+            rk, rv = oracle.reduce_by_key(k, v)
+            assert runs == rk.size and np.array_equal(ko.numpy(runs), rk) and np.array_equal(vo.numpy(runs), rv), (vdtype, n)
+
+
 @pytest.mark.parametrize("op", [1, 2])
 def test_min_max(dev, oracle, op):
     n = 70001
