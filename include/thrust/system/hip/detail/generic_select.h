@@ -86,14 +86,6 @@ inline carved_temp carve(temp_storage& temp, uint64_t n, std::size_t extra_bytes
   c.d_num = reinterpret_cast<uint64_t*>(c.base + c.lay.total);
   return c;
 }
-template <typename U>
-inline int move_parked_back(const carved_temp& c, U* data, uint64_t n, hipStream_t stream) {
-  THRUST_AMD_KERNEL_LAUNCH("partition_tail", stream, (sel::partition_tail_kernel<U>), dim3(sel::tail_grid<U>(n)),
-                           dim3(sel::TAIL_BLOCK), data, (const U*)(c.base + c.lay.off_extra), n,
-                           (const uint64_t*)c.d_num,
-                           (const uint32_t*)(reinterpret_cast<uint32_t*>(c.base + c.lay.off_ticket) + 16));
-  return (int)hipPeekAtLastError();
-}
 }  // namespace select_detail
 
 // The selection by a predicate in all its shapes; returns how many elements it selected.
@@ -125,8 +117,7 @@ uint64_t generic_selection(void* stream, const temp_source& source, const T* ite
     a.tested_true = reinterpret_cast<Tested*>(out_true);
     a.tested_false = in_place ? reinterpret_cast<Tested*>(c.base + c.lay.off_extra) : reinterpret_cast<Tested*>(out_false);
     if (in_place) {
-      rc = sel::select_launch<Tested, U, sel::FLAG_PRED, false, true, true>(c.base, c.lay, a, s);
-      if (rc == 0) rc = select_detail::move_parked_back<Tested>(c, reinterpret_cast<Tested*>(out_true), n, s);
+      rc = sel::partition_in_place_launch<Tested, Tested, U, false>(c.base, c.lay, a, reinterpret_cast<Tested*>(out_true), s);
     } else if (out_false) {
       rc = sel::select_launch<Tested, U, sel::FLAG_PRED, false, true>(c.base, c.lay, a, s);
     } else {
@@ -138,8 +129,7 @@ uint64_t generic_selection(void* stream, const temp_source& source, const T* ite
     a.payload_true = reinterpret_cast<U*>(out_true);
     a.payload_false = in_place ? reinterpret_cast<U*>(c.base + c.lay.off_extra) : reinterpret_cast<U*>(out_false);
     if (in_place) {
-      rc = sel::select_launch<Tested, U, sel::FLAG_PRED, true, true, true>(c.base, c.lay, a, s);
-      if (rc == 0) rc = select_detail::move_parked_back<U>(c, reinterpret_cast<U*>(out_true), n, s);
+      rc = sel::partition_in_place_launch<U, Tested, U, true>(c.base, c.lay, a, reinterpret_cast<U*>(out_true), s);
     } else if (out_false) {
       rc = sel::select_launch<Tested, U, sel::FLAG_PRED, true, true>(c.base, c.lay, a, s);
     } else {

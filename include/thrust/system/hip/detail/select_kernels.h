@@ -19,8 +19,8 @@
 // compacts them in its own piece of LDS first, so that its store instructions cover
 // contiguous addresses.
 //
-// The in-place partition parks one side in temp storage and copies it back afterwards.  Its
-// init kernel samples the input and picks the direction of the sweep so that the parked side
+// The in-place partition parks one side in temp storage and copies it back afterwards (unless the array
+// is one tile).  From 32 MiB on its init kernel samples the input and picks the direction of the sweep so that the parked side
 // is the smaller one: forwards, the selected elements are written in place (each lands at or
 // before its source) and the rejected ones are parked; from the back, the rejected elements
 // are written in place (each lands at or behind its source) and the selected ones are parked.
@@ -76,6 +76,11 @@ constexpr int SELECT_LEAN_ITEMS = 64;
 constexpr int SELECT_LEAN_HEAD_ITEMS = 56;
 constexpr int SELECT_LEAN_TWO_ITEMS = 48;
 constexpr int SELECT_LANE_BYTES = 256;
+// In-place partitions of up to so many bytes sweep forwards without asking which side is the smaller: the sample's
+// loads and a launch cost more than parking the larger side.  Whole call with its copy, us, either way against
+// forwards: int32 with 50 % selected 1e6 32.6 -> 21.7, 4e6 44 -> 34, 16e6 81 -> 71; with 5 % (95 % parked) 4e6
+// 40 -> 36, 12e6 63.7 -> 61.6, 16e6 78 -> 80; float64 with 5 % 4e6 47 -> 42, 8e6 73 -> 74, 16e6 117 -> 141.
+constexpr uint64_t SELECT_ONE_WAY_MAX_BYTES = (uint64_t)32 << 20;
 constexpr int SELECT_MIN_ITEMS = 8;   // sizes the descriptor array
 constexpr int SELECT_MAX_ITEMS = 32;
 
@@ -191,13 +196,14 @@ struct SelectArgs {
   uint32_t* ticket;
   uint32_t aligned;     // tested (and payload) pointers allow whole-vector loads
   const uint32_t* reverse;  // in-place partition only: *reverse != 0 sweeps from the back (else nullptr)
+  uint32_t one_tile;    // in-place partition of a single tile: rejected elements go behind the selected ones
 };
 
 // Arguments with every pointer null and the given flagger (which need not be default-constructible).
 template <typename T, typename U, typename Flagger>
 inline SelectArgs<T, U, Flagger> make_select_args(const Flagger& flag) {
   return SelectArgs<T, U, Flagger>{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
-                                   flag,    nullptr, nullptr, 0u,      nullptr};
+                                   flag,    nullptr, nullptr, 0u,      nullptr, 0u};
 }
 
 // VEC elements of U that belong to one 16-byte vector of T.
@@ -206,7 +212,7 @@ struct alignas((VEC * sizeof(U)) >= 16 ? 16 : VEC * sizeof(U)) PayloadVec {
   U v[VEC];
 };
 
-// Clears the tile descriptors, the ticket and the count.  For the in-place partition it also
+// Clears the tile descriptors, the ticket and the count.  For the larger in-place partitions it also
 // decides the direction of the sweep from a sample of the input (workgroup 0: 4096 elements
 // spread evenly): the side the sample finds smaller is the one that gets parked in temporary
 // storage and copied back.  Whatever the sample says, both directions give the same result.
@@ -217,14 +223,15 @@ __global__ __launch_bounds__(256) void select_init_kernel(uint64_t* __restrict__
                                                           uint64_t* __restrict__ d_num,
                                                           const T* __restrict__ tested, uint64_t n,
                                                           Flagger flag,
-                                                          uint32_t* __restrict__ reverse) {
+                                                          uint32_t* __restrict__ reverse, bool samples_direction) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < count) words[i] = 0;
   if (i == 0) {
     *ticket = 0;
     *d_num = 0;
   }
-  if (reverse != nullptr && blockIdx.x == 0) {
+  if (reverse != nullptr && i == 0 && !samples_direction) *reverse = 0;
+  if (reverse != nullptr && blockIdx.x == 0 && samples_direction) {
     constexpr int PER_LANE = 16;
     __shared__ uint32_t s_hits;
     if (threadIdx.x == 0) s_hits = 0;
@@ -494,6 +501,9 @@ THRUST_AMD_DEVICE void select_tile(const SelectArgs<T, U, Flagger>& a, SelectSha
       select_emit<true, CHUNKS, VEC, G>(true, stage, fl, lane_excl, chunk_base, lane, wave_valid, out_true, out_false, get);
     } else {
       S* out_true = fwd_true + true_base;
+      if constexpr (TWO) {
+        if (a.one_tile) fwd_false = fwd_true + tile_cnt;
+      }
       if (fwd_false)
         select_emit<true, CHUNKS, VEC, G>(false, stage, fl, lane_excl, chunk_base, lane, wave_valid, out_true, fwd_false + false_base, get);
       else
@@ -505,17 +515,18 @@ THRUST_AMD_DEVICE void select_tile(const SelectArgs<T, U, Flagger>& a, SelectSha
 }
 
 // DIR 0: forward sweep.  DIR 1 / 2: the two kernels of the in-place partition, launched one
-// after the other; the one whose direction (1 forward, 2 from the back) the init kernel did not
+// after the other (up to 32 MiB only the first); the one whose direction (1 forward, 2 from the back) the init kernel did not
 // choose ends at once.  (One kernel that takes the direction as a run-time value, or that
 // holds both bodies, was measured at twice the time: 0.9 against 0.5 ms on 2^28 float32.)
 template <typename T, typename U, int MODE, bool HAS_PAYLOAD, bool TWO, int DIR, typename Flagger>
 __global__ __launch_bounds__((SelectShape<T, U, HAS_PAYLOAD, MODE, TWO>::BLOCK), (SelectShape<T, U, HAS_PAYLOAD, MODE, TWO>::WAVES_PER_SIMD))
 void select_kernel(SelectArgs<T, U, Flagger> a) {
   if constexpr (DIR != 0) {
-    if ((*a.reverse != 0) != (DIR == 2)) return;
+    if (!a.one_tile && (*a.reverse != 0) != (DIR == 2)) return;
   }
   __shared__ SelectShared<T, U, MODE, HAS_PAYLOAD, TWO> sh;
-  if (threadIdx.x == 0) sh.tile = atomicAdd(a.ticket, 1u);
+  // (the ticket of a call of one tile has not been cleared)
+  if (threadIdx.x == 0) sh.tile = a.n > SelectShape<T, U, HAS_PAYLOAD, MODE, TWO>::TILE ? atomicAdd(a.ticket, 1u) : 0u;
   __syncthreads();
   select_tile<T, U, MODE, HAS_PAYLOAD, TWO, DIR == 2>(a, sh);
 }
@@ -642,7 +653,8 @@ inline SelectTemp select_layout(uint64_t n, size_t extra_bytes) {
 
 // DUAL: the in-place partition; the init kernel picks the direction of the sweep and leaves it
 // in temp storage (the word 64 bytes behind the ticket) for the kernels that follow: one
-// selection kernel per direction, of which the other ends at once, and the copy back.
+// selection kernel per direction, of which the other ends at once (small arrays: the forward one
+// alone), and the copy back.
 template <typename T, typename U, int MODE, bool HAS_PAYLOAD, bool TWO = false, bool DUAL = false, typename Flagger>
 inline int select_launch(char* temp, const SelectTemp& lay, SelectArgs<T, U, Flagger> a, hipStream_t stream) {
   constexpr uint64_t TILE = SelectShape<T, U, HAS_PAYLOAD, MODE, TWO>::TILE;
@@ -657,20 +669,26 @@ inline int select_launch(char* temp, const SelectTemp& lay, SelectArgs<T, U, Fla
               (!HAS_PAYLOAD || (reinterpret_cast<uintptr_t>(a.payload) % PAY_ALIGN) == 0);
   const uint64_t words = tiles * TileWords<uint64_t>::W;
   const uint64_t init_threads = words ? words : 1;
-  THRUST_AMD_KERNEL_LAUNCH("select_init", stream, (select_init_kernel<T, MODE, Flagger>),
-                           dim3((uint32_t)((init_threads + 255) / 256)), dim3(256), a.status, words, a.ticket,
-                           a.d_num_true, a.tested, a.n, a.flag, reverse);
-  THRUST_AMD_SELECT_CHECK(hipPeekAtLastError());
-  if (a.n == 0) return 0;
-  if constexpr (DUAL) {
-    THRUST_AMD_KERNEL_LAUNCH("select", stream, (select_kernel<T, U, MODE, HAS_PAYLOAD, TWO, 1, Flagger>), dim3((uint32_t)tiles),
-              dim3(SelectShape<T, U, HAS_PAYLOAD, MODE, TWO>::BLOCK), a);
+  constexpr int BLOCK = SelectShape<T, U, HAS_PAYLOAD, MODE, TWO>::BLOCK;
+  // A call of one tile waits for no other tile: no descriptors to clear, and the partition in place reads its
+  // whole input before it writes, so it parks nothing.  One launch instead of two (instead of four, partition in
+  // place): 4097 elements, whole call, copy_if 15.9 -> 11.4 us, unique_by_key 16.0 -> 11.4, partition 28 -> 15.
+  const bool both_ways = DUAL && a.n * (sizeof(T) + (HAS_PAYLOAD ? sizeof(U) : 0)) > SELECT_ONE_WAY_MAX_BYTES;
+  if (tiles != 1) {
+    THRUST_AMD_KERNEL_LAUNCH("select_init", stream, (select_init_kernel<T, MODE, Flagger>),
+                             dim3((uint32_t)((init_threads + 255) / 256)), dim3(256), a.status, words, a.ticket,
+                             a.d_num_true, a.tested, a.n, a.flag, reverse, both_ways);
     THRUST_AMD_SELECT_CHECK(hipPeekAtLastError());
-    THRUST_AMD_KERNEL_LAUNCH("select", stream, (select_kernel<T, U, MODE, HAS_PAYLOAD, TWO, 2, Flagger>), dim3((uint32_t)tiles),
-              dim3(SelectShape<T, U, HAS_PAYLOAD, MODE, TWO>::BLOCK), a);
+    if (a.n == 0) return 0;
+  }
+  if constexpr (DUAL) {
+    a.one_tile = tiles == 1 ? 1u : 0u;  // (it sweeps forwards, whatever *reverse holds)
+    THRUST_AMD_KERNEL_LAUNCH("select", stream, (select_kernel<T, U, MODE, HAS_PAYLOAD, TWO, 1, Flagger>), dim3((uint32_t)tiles), dim3(BLOCK), a);
+    THRUST_AMD_SELECT_CHECK(hipPeekAtLastError());
+    if (!both_ways) return 0;
+    THRUST_AMD_KERNEL_LAUNCH("select", stream, (select_kernel<T, U, MODE, HAS_PAYLOAD, TWO, 2, Flagger>), dim3((uint32_t)tiles), dim3(BLOCK), a);
   } else {
-    THRUST_AMD_KERNEL_LAUNCH("select", stream, (select_kernel<T, U, MODE, HAS_PAYLOAD, TWO, 0, Flagger>), dim3((uint32_t)tiles),
-              dim3(SelectShape<T, U, HAS_PAYLOAD, MODE, TWO>::BLOCK), a);
+    THRUST_AMD_KERNEL_LAUNCH("select", stream, (select_kernel<T, U, MODE, HAS_PAYLOAD, TWO, 0, Flagger>), dim3((uint32_t)tiles), dim3(BLOCK), a);
   }
   THRUST_AMD_SELECT_CHECK(hipPeekAtLastError());
   return 0;
@@ -682,6 +700,18 @@ inline uint32_t tail_grid(uint64_t n) {
   return (uint32_t)((n + per_block - 1) / per_block + 1);
 }
 
+// The partition in place: the sweep, then the parked elements move to their place.  `data` is what is
+// partitioned (the tested elements, or the payload), S its element; parked elements lie at lay.off_extra.
+template <typename S, typename T, typename U, bool HAS_PAYLOAD, typename Flagger>
+inline int partition_in_place_launch(char* temp, const SelectTemp& lay, const SelectArgs<T, U, Flagger>& a, S* data, hipStream_t stream) {
+  const int rc = select_launch<T, U, FLAG_PRED, HAS_PAYLOAD, true, true>(temp, lay, a, stream);
+  if (rc != 0 || a.n <= SelectShape<T, U, HAS_PAYLOAD, FLAG_PRED, true>::TILE) return rc;  // one tile parks nothing
+  THRUST_AMD_KERNEL_LAUNCH("partition_tail", stream, (partition_tail_kernel<S>), dim3(tail_grid<S>(a.n)), dim3(TAIL_BLOCK), data,
+                           (const S*)(temp + lay.off_extra), a.n, (const uint64_t*)a.d_num_true,
+                           (const uint32_t*)(reinterpret_cast<uint32_t*>(temp + lay.off_ticket) + 16));
+  THRUST_AMD_SELECT_CHECK(hipPeekAtLastError());
+  return 0;
+}
 
 #undef THRUST_AMD_SELECT_CHECK
 

@@ -221,3 +221,58 @@ def test_unique_float_nan_and_zero(dev, oracle):
     ref = oracle.unique(x)
     assert cnt == ref.size
     assert np.array_equal(out.numpy(cnt).view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.int32, np.float64])
+@pytest.mark.parametrize("skip", [0, 1])
+def test_calls_of_one_tile_and_their_neighbours(dev, oracle, dtype, skip):
+    """Up to one tile a call is a single launch on descriptors that nobody has cleared (the temporary storage is filled
+    with ones here), and a partition in place parks nothing."""
+    import torch
+    temp = dev.Temp()
+    temp.buf = torch.full((1 << 20,), 255, dtype=torch.uint8, device="cuda")
+    thr = 0.3 if np.dtype(dtype).kind == "f" else 60
+    for edge in (64, 1024, 16384, 24576, 28672, 32768):
+        for n in (edge - 1, edge, edge + 1):
+            x = _vals(n + skip, dtype, 31)
+            st = _vals(n + skip, np.int32, 37)[skip:]
+            code = dev.DTYPE_OF_NP[np.dtype(dtype)]
+            fresh = lambda: dev.DeviceArray(n, code, dev.DeviceArray.from_numpy(x).storage[skip * x.itemsize:])
+            ds, y = dev.DeviceArray.from_numpy(st), x[skip:]
+            d = fresh()
+            out, cnt = dev.copy_if(d, dev.LT, thr, temp=temp)
+            assert cnt == np.count_nonzero(y < thr) and np.array_equal(out.numpy(cnt), y[y < thr]), n
+            cnt = dev.stable_partition(d, dev.LT, thr, temp=temp)
+            assert cnt == np.count_nonzero(y < thr) and np.array_equal(d.numpy(), np.concatenate([y[y < thr], y[y >= thr]])), n
+            d = fresh()
+            dev.stable_partition(d, dev.GE, 50, stencil=ds, temp=temp)
+            assert np.array_equal(d.numpy(), np.concatenate([y[st >= 50], y[st < 50]])), (n, "stencil")
+            keys = dev.DeviceArray.from_numpy(np.sort(st) // 3)
+            ko, vo, runs = dev.unique_by_key(keys, fresh(), temp=temp)
+            rk, rv = oracle.unique_by_key(np.sort(st) // 3, y)
+            assert runs == rk.size and np.array_equal(ko.numpy(runs), rk) and np.array_equal(vo.numpy(runs), rv), n
+
+
+@pytest.mark.parametrize("dtype,skip", [(np.int32, 0), (np.int32, 1), (np.uint64, 0), (np.uint8, 3)])
+def test_partition_in_place_on_both_sides_of_the_one_way_limit(dev, dtype, skip):
+    """Up to 32 MiB the sweep runs forwards whatever is selected, above it from the end that parks the smaller side."""
+    size = np.dtype(dtype).itemsize
+    for n in ((32 << 20) // size, (32 << 20) // size + 1, (40 << 20) // size + 7):
+        x = _vals(n + skip, dtype, 41)
+        y = x[skip:]
+        for thr in (10, 190):
+            d = dev.DeviceArray(n, dev.DTYPE_OF_NP[np.dtype(dtype)], dev.DeviceArray.from_numpy(x).storage[skip * size:])
+            cnt = dev.stable_partition(d, dev.LT, thr)
+            assert cnt == np.count_nonzero(y < thr)
+            assert np.array_equal(d.numpy(), np.concatenate([y[y < thr], y[y >= thr]])), (dtype, n, thr)
+
+
+def test_partition_in_place_by_stencil_beyond_the_one_way_limit(dev):
+    n = (5 << 20) + 3
+    st = _vals(n, np.int32, 43)
+    ds = dev.DeviceArray.from_numpy(st)
+    x = _vals(n, np.uint32, 47)
+    for thr in (10, 190):
+        d = dev.DeviceArray.from_numpy(x)
+        dev.stable_partition(d, dev.LT, thr, stencil=ds)
+        assert np.array_equal(d.numpy(), np.concatenate([x[st < thr], x[st >= thr]])), thr

@@ -45,13 +45,7 @@ static int select_by_predicate(void* temp, size_t* temp_bytes, const void* in, c
       if (!in_place)
         return a.tested_false ? select_launch<T, uint32_t, FLAG_PRED, false, true>(base, lay, a, stream)
                               : select_launch<T, uint32_t, FLAG_PRED, false>(base, lay, a, stream);
-      int rc = select_launch<T, uint32_t, FLAG_PRED, false, true, true>(base, lay, a, stream);
-      if (rc || n == 0) return rc;
-      TA_LAUNCH("partition_tail", stream, (partition_tail_kernel<T>), dim3(tail_grid<T>(n)), dim3(TAIL_BLOCK),
-                static_cast<T*>(out_true), (const T*)(base + lay.off_extra), n, (const uint64_t*)d_num,
-                (const uint32_t*)(reinterpret_cast<uint32_t*>(base + lay.off_ticket) + 16));
-      TA_CHECK_LAUNCH();
-      return 0;
+      return partition_in_place_launch<T, T, uint32_t, false>(base, lay, a, static_cast<T*>(out_true), stream);
     });
   }
   // stencil form, separate outputs: one pass, the stencil is tested in its own type and the

@@ -35,13 +35,7 @@ int partition_in_place_by_stencil(void* temp, size_t* temp_bytes, void* data, co
       a.payload_false = parked;
       a.d_num_true = d_num;
       a.n = n;
-      const int rc = select_launch<T, U, FLAG_PRED, true, true, true>(base, lay, a, stream);
-      if (rc || n == 0) return rc;
-      TA_LAUNCH("partition_tail", stream, (partition_tail_kernel<U>), dim3(tail_grid<U>(n)), dim3(TAIL_BLOCK),
-                static_cast<U*>(data), (const U*)parked, n, (const uint64_t*)d_num,
-                (const uint32_t*)(reinterpret_cast<uint32_t*>(base + lay.off_ticket) + 16));
-      TA_CHECK_LAUNCH();
-      return 0;
+      return partition_in_place_launch<U, T, U, true>(base, lay, a, static_cast<U*>(data), stream);
     });
   });
 }
