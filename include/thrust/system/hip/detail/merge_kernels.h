@@ -3,8 +3,9 @@
 // thrust_amd_merge_by_key; a translation unit compiled with hipcc instantiates it for its own
 // comparator and key type.
 //
-//   partition  one thread per output-tile boundary d = tile * TILE binary-searches the
+//   partition  a few lanes per output-tile boundary d = tile * TILE search the
 //              merge path: how many of the first d outputs come from range A
+//              (short merges: inside the next kernel)
 //   merge      a workgroup stages the two sub-ranges of its tile in LDS, every lane finds
 //              its own start on the path by binary search in LDS and merges ITEMS
 //              elements serially; values follow through LDS by the recorded source slot
@@ -28,6 +29,16 @@ constexpr int MERGE_BLOCK = 256;
 constexpr int MERGE_ITEMS = 16;
 constexpr int MERGE_TILE = MERGE_BLOCK * MERGE_ITEMS;
 
+// Up to so many outputs a workgroup finds its tile's two boundaries itself, 32 lanes each: one launch and no wait for
+// it, but every boundary is searched twice and by more probes.  Beyond, a launch of its own finds them, by 8 lanes
+// each, by 4 or by one, the fewer the more boundaries there are, for then what they read counts.  Whole call in us, pairs of 4 + 4 bytes, a launch
+// with one thread per boundary (as it was) / 4 lanes / 8 lanes / 16 lanes / no launch: 1e6 14.5 / - / - / - / 9.8,
+// 4e6 25.2 / 21.6 / 20.4 / 19.8 / 17.7, 8e6 36.2 / 32.4 / 31.6 / 30.6 / 31.3, 16e6 55.5 / 51.5 / 50.4 / 50.1 / 56.4,
+// 64e6 200 / 194 / 195 / 197 / 229, 1.34e8 398 / 398 / 402 / 409 / 463, 2^28 852 / 866 / - / - / -.
+constexpr uint64_t MERGE_SEARCHES_MAX = (uint64_t)1 << 23;
+constexpr uint64_t MERGE_EIGHT_LANES_MAX = (uint64_t)1 << 25;
+constexpr uint64_t MERGE_FOUR_LANES_MAX = (uint64_t)1 << 27;
+
 // Number of elements taken from A among the first `diag` outputs.
 template <typename T, typename PA, typename PB, typename Comp>
 THRUST_AMD_DEVICE uint64_t merge_path(PA a, uint64_t na, PB b, uint64_t nb, uint64_t diag, Comp& comp) {
@@ -43,22 +54,61 @@ THRUST_AMD_DEVICE uint64_t merge_path(PA a, uint64_t na, PB b, uint64_t nb, uint
   return lo;
 }
 
-template <typename T, typename Comp>
+// The same search by groups of 2^BITS consecutive lanes (every lane of the wave active), each group for a diagonal of
+// its own.  A round probes the multiples of 2^(BITS k) in the interval, at most a group of them, so that an interval
+// below 2^(BITS (k + 1)) shrinks below 2^(BITS k).  The places of the coarse rounds are the same for all groups and
+// come from the caches.
+template <int BITS, typename T, typename Comp>
+THRUST_AMD_DEVICE uint64_t group_merge_path(const T* __restrict__ a, uint64_t na, const T* __restrict__ b, uint64_t nb,
+                                            uint64_t diag, Comp& comp) {
+  constexpr uint32_t PROBES = 1u << BITS;
+  const uint32_t lane = threadIdx.x % WAVE;
+  uint64_t lo = diag > nb ? diag - nb : 0;
+  uint64_t hi = diag < na ? diag : na;
+  const uint64_t longest = na < nb ? na : nb;  // no interval is longer
+  int bit = longest > 1 ? (63 - __builtin_clzll(longest)) / BITS * BITS : 0;
+  for (; bit >= 0; bit -= BITS) {
+    const uint64_t unit = 1ull << bit;
+    const uint64_t first = (lo + unit - 1) & ~(unit - 1);
+    const uint64_t mid = first + (uint64_t)(lane % PROBES) * unit;
+    bool from_a = false;
+    if (mid < hi) {
+      const T ka = a[mid];
+      const T kb = b[diag - 1 - mid];
+      from_a = !comp(kb, ka);
+    }
+    // in each group the lanes that say yes are the lowest ones
+    const uint64_t said_yes = __builtin_amdgcn_ballot_w64(from_a) >> (lane & ~(PROBES - 1));
+    const uint32_t yes = (uint32_t)__builtin_popcount((uint32_t)said_yes & (uint32_t)((1ull << PROBES) - 1));
+    const uint64_t no = first + (uint64_t)yes * unit;  // the first probe that said no, if it was one
+    if (yes > 0) lo = no - unit + 1;
+    if (yes < PROBES && no < hi) hi = no;
+  }
+  return lo;
+}
+
+// Tile boundary t for group t of 2^BITS lanes.  With MERGE_TILE a multiple of the probes' coarse distances, the places of
+// a diagonal's rounds in b are shared between groups as those in a are.
+template <int BITS, typename T, typename Comp>
 __global__ __launch_bounds__(256) void merge_partition_kernel(const T* __restrict__ a, uint64_t na,
                                                               const T* __restrict__ b, uint64_t nb,
                                                               uint64_t tiles, Comp comp,
                                                               uint64_t* __restrict__ a_split) {
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t > tiles) return;
+  const uint64_t t = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> BITS;
   const uint64_t total = na + nb;
   uint64_t diag = t * MERGE_TILE;
   if (diag > total) diag = total;
-  // the merge-path search of merge_path() below, over the whole ranges: probes shared between threads
-  a_split[t] = aligned_partition_point(diag > nb ? diag - nb : 0, diag < na ? diag : na, [&](uint64_t mid) {
-    const T ka = a[mid];
-    const T kb = b[diag - 1 - mid];
-    return !comp(kb, ka);
-  });
+  uint64_t split;
+  if constexpr (BITS == 0) {
+    split = aligned_partition_point(diag > nb ? diag - nb : 0, diag < na ? diag : na, [&](uint64_t mid) {
+      const T ka = a[mid];
+      const T kb = b[diag - 1 - mid];
+      return !comp(kb, ka);
+    });
+  } else {
+    split = group_merge_path<BITS, T>(a, na, b, nb, diag, comp);
+  }
+  if (t <= tiles && threadIdx.x % (1u << BITS) == 0) a_split[t] = split;
 }
 
 // Slot of output element e in the LDS exchange buffer: one spare slot after every
@@ -67,7 +117,8 @@ __global__ __launch_bounds__(256) void merge_partition_kernel(const T* __restric
 THRUST_AMD_DEVICE uint32_t merge_slot(uint32_t e) { return e + e / MERGE_ITEMS; }
 constexpr int MERGE_SLOTS = MERGE_TILE + MERGE_TILE / MERGE_ITEMS + 1;
 
-template <typename T, typename V, bool HAS_VALUES, typename Comp>
+// SEARCHES: the workgroup finds its tile's boundaries itself instead of reading them from a_split.
+template <typename T, typename V, bool HAS_VALUES, bool SEARCHES, typename Comp>
 __global__ __launch_bounds__(MERGE_BLOCK) void merge_kernel(
     const T* __restrict__ a, uint64_t na, const T* __restrict__ b, uint64_t nb,
     const V* __restrict__ va, const V* __restrict__ vb, T* __restrict__ out, V* __restrict__ vout,
@@ -81,7 +132,23 @@ __global__ __launch_bounds__(MERGE_BLOCK) void merge_kernel(
   const uint64_t total = na + nb;
   const uint64_t d0 = tile * MERGE_TILE;
   const uint64_t d1 = (d0 + MERGE_TILE < total) ? d0 + MERGE_TILE : total;
-  const uint64_t a0 = a_split[tile], a1 = a_split[tile + 1];
+  uint64_t a0, a1;
+  if constexpr (SEARCHES) {
+    __shared__ uint64_t s_split[2];
+    if (threadIdx.x < WAVE) {
+      const uint64_t split = group_merge_path<5, T>(a, na, b, nb, threadIdx.x < WAVE / 2 ? d0 : d1, comp);
+      if (threadIdx.x % (WAVE / 2) == 0) s_split[threadIdx.x / (WAVE / 2)] = split;
+    }
+    __syncthreads();
+    a0 = wave_uniform(s_split[0]);
+    a1 = wave_uniform(s_split[1]);
+    // keys that are in no order (NaN among them) must not lead out of the ranges
+    if (a1 < a0) a1 = a0;
+    if (a1 - a0 > d1 - d0) a1 = a0 + (d1 - d0);
+  } else {
+    a0 = a_split[tile];
+    a1 = a_split[tile + 1];
+  }
   const uint64_t b0 = d0 - a0, b1 = d1 - a1;
   const uint32_t ca = (uint32_t)(a1 - a0), cb = (uint32_t)(b1 - b0);
   const uint32_t count = ca + cb;  // == d1 - d0
@@ -172,11 +239,21 @@ inline int merge_launch(uint64_t* split, const T* a, uint64_t na, const T* b, ui
   const uint64_t total = na + nb;
   const uint64_t tiles = (total + MERGE_TILE - 1) / MERGE_TILE;
   if (tiles > 0x7fffffffull) return (int)hipErrorInvalidValue;
-  THRUST_AMD_KERNEL_LAUNCH("merge_partition", stream, (merge_partition_kernel<T, Comp>),
-                           dim3((uint32_t)((tiles + 1 + 255) / 256)), dim3(256), a, na, b, nb, tiles, comp, split);
+  if (total <= MERGE_SEARCHES_MAX) {
+    THRUST_AMD_KERNEL_LAUNCH("merge", stream, (merge_kernel<T, V, HAS_VALUES, true, Comp>), dim3((uint32_t)tiles),
+                             dim3(MERGE_BLOCK), a, na, b, nb, va, vb, out, vout, comp, (const uint64_t*)nullptr);
+    return (int)hipPeekAtLastError();
+  }
+  auto partition = [&](auto kernel, int bits) {
+    const uint64_t threads = (tiles + 1) << bits;
+    THRUST_AMD_KERNEL_LAUNCH("merge_partition", stream, kernel, dim3((uint32_t)((threads + 255) / 256)), dim3(256), a, na, b, nb, tiles, comp, split);
+  };
+  if (total <= MERGE_EIGHT_LANES_MAX) partition(merge_partition_kernel<3, T, Comp>, 3);
+  else if (total <= MERGE_FOUR_LANES_MAX) partition(merge_partition_kernel<2, T, Comp>, 2);
+  else partition(merge_partition_kernel<0, T, Comp>, 0);
   hipError_t e = hipPeekAtLastError();
   if (e != hipSuccess) return (int)e;
-  THRUST_AMD_KERNEL_LAUNCH("merge", stream, (merge_kernel<T, V, HAS_VALUES, Comp>), dim3((uint32_t)tiles),
+  THRUST_AMD_KERNEL_LAUNCH("merge", stream, (merge_kernel<T, V, HAS_VALUES, false, Comp>), dim3((uint32_t)tiles),
                            dim3(MERGE_BLOCK), a, na, b, nb, va, vb, out, vout, comp, (const uint64_t*)split);
   return (int)hipPeekAtLastError();
 }

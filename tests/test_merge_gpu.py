@@ -82,3 +82,24 @@ def test_config5_merge_full_size(dev):
     order = np.argsort(keys, kind="stable")
     assert np.array_equal(out_k.numpy(), keys[order])
     assert np.array_equal(out_v.numpy(), vals[order])
+
+
+@pytest.mark.parametrize("n,kind", [(n, kind) for n in (4095, 4097, (1 << 23) - 1, 1 << 23, (1 << 23) + 1, (1 << 25) + 1)
+                                    for kind in ("mixed", "equal", "apart", "short", "none")] + [((1 << 27) + 1, "mixed")])
+def test_boundaries_by_groups_of_lanes(dev, n, kind):
+    """The boundaries of the tiles on the merge path, by every group size, at both ends of its range: ranges that
+    interleave, of one key, one wholly before the other, one of 33 elements, one empty."""
+    na = {"mixed": n // 2, "equal": n // 3, "apart": n // 2 + 5, "short": 33, "none": 0}[kind]
+    raw = (datagen.splitmix64(5, n) >> np.uint64(33)).astype(np.uint32)
+    if kind == "equal":
+        raw[:] = 7
+    a, b = np.sort(raw[:na]), np.sort(raw[na:])
+    if kind == "apart":
+        a, b = a + np.uint32(1 << 31), b & np.uint32((1 << 31) - 1)
+    va, vb = np.arange(na, dtype=np.uint32), np.arange(na, n, dtype=np.uint32)
+    arrays = [dev.DeviceArray.from_numpy(x) for x in (a, b, va, vb)]
+    keys, values = dev.merge_by_key(*arrays)
+    both = np.concatenate([a, b])
+    order = np.argsort(both, kind="stable")
+    assert np.array_equal(keys.numpy(), both[order]) and np.array_equal(values.numpy(), order.astype(np.uint32))
+    assert np.array_equal(dev.merge(arrays[0], arrays[1]).numpy(), both[order])
