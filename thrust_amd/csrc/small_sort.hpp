@@ -12,12 +12,13 @@
 //     Should a group turn out larger than SMALL_GROUP_MAX, all digits get their pass, from the lowest
 //     (the arrangement so far is a stable one, so equal keys still come out in their original order).
 // One copy and one sort, back to back, against the same through the chained passes (eight launches):
-// 3001 uint32 53.7 -> 13.2 us, 8192 uint32 56.7 -> 23.3, 8192 float32 58.7 -> 26.2, 3001 (int64, uint32)
-// 81.0 -> 18.0, 8192 float64 79.6 -> 30.5.  All digits of the float64 take 93 us: the passes' ranking is what
+// 3001 uint32 53.7 -> 12.7 us, 8192 uint32 56.7 -> 20.9, 8192 float32 58.7 -> 24.3, 3001 (uint64, uint32)
+// 81.0 -> 17.3, 8192 float64 79.6 -> 30.  (All loads in flight at the start, the values' too, instead of one after
+// the other and the values behind the sort: 8192 uint32 23.0 -> 20.9, with uint32 values 29.1 -> 25.0.)  All digits of the float64 take 93 us: the passes' ranking is what
 // the time goes into, hence the effort to leave passes out.  Beyond 8192 keys one CU is no longer
 // fast enough (its ranking alone takes 3 us per pass and 8192 keys).
-// Values do not travel with the keys: every key carries its 16-bit index, the values are staged in
-// LDS at the end and picked up by it.
+// Values do not travel with the keys: every key carries its 16-bit index, the values wait in registers, are
+// staged in LDS at the end and picked up by it.
 #pragma once
 #include "common.hpp"
 #include "launch.hpp"
@@ -55,20 +56,27 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
   uint32_t* my_cnt = s_cnt + wave * RADIX_SIZE;
   const K range = (K)((end_bit - begin_bit >= (int)sizeof(K) * 8 ? ~(K)0 : (K)(((K)1 << (end_bit - begin_bit)) - 1)) << begin_bit);
 
-  // ---- load; slots past the end sort last
+  // ---- load, keys and values, all in flight together: without predicates (a predicated load is waited for before
+  // the next is issued), the last element in the place of those behind it; slots past the end sort last
   K e[SMALL_ITEMS];
+  V v[HAS_VALUES ? SMALL_ITEMS : 1];
   uint32_t idx[SMALL_ITEMS];
-  const K first = codec.encode(keys[0]);
+  K first = keys[0];
+#pragma unroll
+  for (int r = 0; r < SMALL_ITEMS; ++r) e[r] = keys[span + r * WAVE < n ? span + r * WAVE : n - 1];
+  if constexpr (HAS_VALUES) {
+#pragma unroll
+    for (int r = 0; r < SMALL_ITEMS; ++r) v[r] = vals[span + r * WAVE < n ? span + r * WAVE : n - 1];
+  }
+  first = codec.encode(first);
   K differ = 0;
 #pragma unroll
   for (int r = 0; r < SMALL_ITEMS; ++r) {
     const uint32_t pos = span + r * WAVE;
-    e[r] = (K)~(K)0;
     idx[r] = pos;
-    if (r < rounds && pos < n) {
-      e[r] = codec.encode(keys[pos]);
-      differ |= e[r] ^ first;
-    }
+    e[r] = codec.encode(e[r]);
+    differ |= e[r] ^ first;
+    if (r >= rounds || pos >= n) e[r] = (K)~(K)0;
   }
   {
     struct Or {
@@ -235,7 +243,7 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
 #pragma unroll
     for (int r = 0; r < SMALL_ITEMS; ++r) {
       const uint32_t pos = span + r * WAVE;
-      if (r < rounds && pos < n) s_vals[pos] = vals[pos];
+      if (r < rounds && pos < n) s_vals[pos] = v[r];
     }
     __syncthreads();
   }
