@@ -176,6 +176,60 @@ def test_sizes_where_the_kernels_change(dev, dtype, vdtype, edge):
             assert np.array_equal(k.numpy().view(np.uint8), x[order].view(np.uint8)), (n, descending)
 
 
+# (key, value, longest array whose passes behind the short way run in one launch: REST_MAX in thrust_amd/csrc/radix_sort.hip)
+ONE_LAUNCH = [(np.uint32, None, 1 << 20), (np.int32, np.uint8, 3 << 18), (np.uint32, np.uint64, 3 << 18),
+              (np.int64, None, 3 << 15), (np.uint64, np.uint16, 3 << 15), (np.float64, np.uint64, 3 << 15)]
+
+
+@pytest.mark.parametrize("dtype,vdtype,edge", ONE_LAUNCH)
+@pytest.mark.parametrize("kind", ["skewed", "ids", "normal"])
+def test_passes_left_over_in_one_launch(dev, dtype, vdtype, edge, kind):
+    """Keys that decline the short way, with an even and an odd number of digits that vary (the result is copied back)."""
+    temp = dev.Temp()
+    for n in (8193, edge // 2, edge, edge + 1):
+        x = _keys(kind, dtype, n)
+        for descending in (False, True):
+            order = _order(x, descending)
+            k = dev.DeviceArray.from_numpy(x)
+            if vdtype is None:
+                dev.sort_keys(k, descending=descending, temp=temp)
+            else:
+                v = np.arange(n).astype(vdtype)
+                w = dev.DeviceArray.from_numpy(v)
+                dev.sort_pairs(k, w, descending=descending, temp=temp)
+                assert np.array_equal(w.numpy(), v[order]), (n, descending)
+            assert np.array_equal(k.numpy().view(np.uint8), x[order].view(np.uint8)), (n, descending)
+            assert _control(temp)["gave_up"] == 0
+
+
+def test_passes_in_one_launch_on_several_streams(dev):
+    """Eight sorts at a time that decline the short way: the workgroups of all of them do not fit the GPU together."""
+    import torch
+    streams = [torch.cuda.Stream() for _ in range(8)]
+    xs = [_keys("skewed", np.uint32, 1_000_000 + i) for i in range(8)]
+    orders = [_order(x, False) for x in xs]
+    for _ in range(3):
+        keys = [dev.DeviceArray.from_numpy(x) for x in xs]
+        values = [dev.DeviceArray.from_numpy(np.arange(x.size, dtype=np.uint32)) for x in xs]
+        temps = [dev.Temp() for _ in xs]
+        torch.cuda.synchronize()
+        for i, stream in enumerate(streams):
+            with torch.cuda.stream(stream):
+                if i % 2:
+                    dev.sort_keys(keys[i], temp=temps[i])
+                else:
+                    small = dev.DeviceArray(780_000, keys[i].dtype, keys[i].storage)
+                    dev.sort_pairs(small, values[i], temp=temps[i])
+        torch.cuda.synchronize()
+        for i, x in enumerate(xs):
+            if i % 2:
+                assert np.array_equal(keys[i].numpy(), x[orders[i]])
+            else:
+                order = _order(x[:780_000], False)
+                assert np.array_equal(keys[i].numpy(780_000), x[:780_000][order])
+                assert np.array_equal(values[i].numpy(780_000), order.astype(np.uint32))
+
+
 def test_long_stretches_among_many_keys(dev):
     """2^25 eight-byte keys, four values 7000 times: the plan takes two digits, the tail sorts the windows that hold them."""
     n = 1 << 25

@@ -2,6 +2,7 @@
 // prefix of the keys, and every stretch of equal prefixes is short enough to be ordered in one workgroup.
 //
 //   bounds  for every window of `window` positions the first place at or behind its start where a new prefix begins
+//           (two digits; stretches of one begin where the histogram says, which finish looks up itself)
 //   finish  a workgroup takes the stretches that begin inside its window, orders them by the whole key in registers
 //           and LDS and writes them to their place in the caller's array.  More than CAP keys (a stretch that the plan
 //           did not expect) are left to the
@@ -83,7 +84,8 @@ TA_DEVICE uint32_t row_inclusive_scan(uint32_t x) {
 template <typename K, typename V, bool HAS_VALUES>
 __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShape<K, V, HAS_VALUES>::WAVES_PER_SIMD)) void sort_finish_kernel(
     K* __restrict__ keys_a, const K* __restrict__ keys_b, V* __restrict__ vals_a, const V* __restrict__ vals_b, uint32_t n,
-    KeyCodec<K> codec, const uint32_t* __restrict__ bounds, const SortCtl* __restrict__ ctl, uint32_t* __restrict__ long_windows,
+    KeyCodec<K> codec, const uint32_t* __restrict__ bounds,  // (8-byte keys)
+    const uint32_t* __restrict__ hist, const SortCtl* __restrict__ ctl, uint32_t* __restrict__ long_windows,
     uint32_t* __restrict__ long_list,  // windows for the tail, *long_windows of them
     uint32_t* __restrict__ status, uint64_t status_words) {
   using Shape = FinishShape<K, V, HAS_VALUES>;
@@ -129,8 +131,21 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
 
   const uint32_t w = blockIdx.x;
   if (w >= windows) return;
-  const uint32_t first = bounds[w];
-  const uint32_t count = bounds[w + 1] - first;
+  uint32_t first, count;
+  if constexpr (sizeof(K) == 8) {
+    first = bounds[w];
+    count = bounds[w + 1] - first;
+  } else {
+    // one digit: its stretches begin where the histogram says
+    const uint4 starts = reinterpret_cast<const uint4*>(hist + (ctl->prefix_bit / RADIX_BITS) * RADIX_SIZE)[threadIdx.x % WAVE];
+    auto start_behind = [&](uint32_t edge) {
+      uint32_t at = n;
+      for (const uint32_t s : {starts.x, starts.y, starts.z, starts.w}) at = s >= edge && s < at ? s : at;
+      return wave_reduce(at, OpMin{});
+    };
+    first = start_behind(w * window);
+    count = (w + 1 == windows ? n : start_behind((w + 1) * window)) - first;
+  }
   if (count == 0) return;
   const uint32_t tid = threadIdx.x;
   if (count > (uint32_t)CAP) {

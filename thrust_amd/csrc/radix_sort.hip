@@ -14,6 +14,7 @@
 //              learns the global offset of each of its 256 digit runs by decoupled
 //              look-back over the tiles before it, and scatters keys (and values)
 //   copy-back  only if an odd number of passes ran (8-byte keys: in the launch of the short way's tail)
+//   rest       behind the short way of a short array: the passes left over and the copy back in one launch
 //
 // Ranking inside a tile uses the wave64 match pattern (radix_rank.hpp): rank = wave-private LDS counter
 // + number of peers in lower lanes.  Lanes hold keys wave-striped (lane l of wave w holds
@@ -441,249 +442,121 @@ __global__ __launch_bounds__(BLOCK, CROWDED ? 2 * BLOCK / WAVE / 4 : 1) void one
   for (int i = threadIdx.x; i < WAVES * RADIX_SIZE; i += BLOCK) s_cnt[i] = 0;
   __syncthreads();
   const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);
-  const uint32_t tile_base = tile * (uint32_t)TILE;
-  const uint32_t valid = (n - tile_base < (uint32_t)TILE) ? (n - tile_base) : (uint32_t)TILE;
-  const int wave = threadIdx.x / WAVE;
-  const int lane = threadIdx.x % WAVE;
-  const uint32_t span = (uint32_t)wave * (WAVE * ITEMS) + lane;  // + r*64
+#define TA_PASS_LOAD(item) (item)
+#define TA_PASS_STORE(item, value) (item) = (value)
+#include "radix_pass_tile.inc"
+#undef TA_PASS_LOAD
+#undef TA_PASS_STORE
+}
 
-  const int shift = geo.begin_bit + pass * RADIX_BITS;
-  const int nbits = (geo.end_bit - shift) < RADIX_BITS ? (geo.end_bit - shift) : RADIX_BITS;
-  const uint32_t dmask = (1u << nbits) - 1u;
-  auto digit_of = [&](K x) -> uint32_t {
-    if constexpr (sizeof(K) == 8) return __builtin_amdgcn_ubfe((uint32_t)(x >> shift), 0u, (uint32_t)nbits);
-    else return __builtin_amdgcn_ubfe((uint32_t)x, (uint32_t)shift, (uint32_t)nbits);
+// ------------------------------------------------------------------ several passes in one launch
+// The passes of the slots [first_slot, slots) and, if `copies`, the copy back: what stands behind the short way, and
+// mostly finds nothing to do.  A workgroup takes tiles of a pass in rising order until there are none left and
+// then waits until the others have written theirs.  Whoever waits, waits only for workgroups that run and wait for
+// nobody but earlier tiles of the same pass, so this works with any number of workgroups resident.
+// What one pass writes and another XCD's workgroup reads in the next goes past the caches that are not coherent
+// (agent scope): a write-back of the L2 per tile took 35 us a pass.  Short runs leave as partial lines then, so longer
+// arrays keep a launch per pass.  Copy and sort, us, a launch per pass (and the bounds of the short way in a launch, as
+// it was) against this: short way taken, 65536 uint32 40.0 -> 25.9, 2^20 47.5 -> 37.1, 65536 (uint32, uint32) 48.0 -> 30.3,
+// 65536 uint64 54.9 -> 35.9, with uint32 values 60.9 -> 40.6; not taken (90 % one key), 65536 uint32 46.3 -> 43.8, 2^20
+// 63.6 -> 65.0, 1.5e6 72 -> 79, 7.9e5 (uint32, uint32) 66.5 -> 67.7, 65536 uint64 74.2 -> 72.9, 131072 77.4 -> 78.6,
+// 2^20 127 -> 170.  A line is drawn where a sort that declines would pay some per cent.
+// tickets[slot]: word 0 counts the tiles taken, word TICKET_STRIDE those written.
+template <typename K, bool HAS_VALUES>
+constexpr uint64_t REST_MAX = sizeof(K) == 8 ? 3u << 15 : HAS_VALUES ? 3u << 18 : 1u << 20;
+
+template <typename K, typename V, bool HAS_VALUES, int BLOCK, int ITEMS>
+__global__ __launch_bounds__(BLOCK) void onesweep_rest_kernel(
+    K* keys_a, K* keys_b, V* vals_a, V* vals_b,
+    uint32_t n, int first_slot, int slots, uint32_t tiles, SortGeometry geo, KeyCodec<K> codec, const uint32_t* __restrict__ hist,
+    uint32_t* __restrict__ statuses, uint64_t slot_words,
+    uint32_t* __restrict__ tickets, const SortCtl* __restrict__ ctl, SortCtl* __restrict__ ctl_out, bool copies) {
+  if (ctl->finishes()) return;
+  using Shape = PassShape<K, V, HAS_VALUES, BLOCK, ITEMS>;
+  using D = uint32_t;
+  using Desc = Descriptor<D>;
+  constexpr bool OFF32 = true;
+  constexpr int WAVES = Shape::WAVES;
+  constexpr int TILE = Shape::TILE;
+  __shared__ __attribute__((aligned(16))) unsigned char s_union[Shape::UNION_BYTES];
+  __shared__ uint32_t s_scatter_base[RADIX_SIZE];
+  __shared__ uint32_t s_digit_wave[RADIX_SIZE / WAVE];
+  __shared__ uint32_t s_tile, s_todo[2];
+  uint32_t* s_cnt = reinterpret_cast<uint32_t*>(s_union);
+  K* s_keys = reinterpret_cast<K*>(s_union);
+  V* s_vals = reinterpret_cast<V*>(s_union);
+  uint32_t* finished = nullptr;  // tiles written by the pass before
+  // Thread 0, until the pass before is complete: true, or false if somebody has given up.
+  auto is_complete = [&]() -> bool {
+    for (uint32_t spins = 0; finished != nullptr && __hip_atomic_load(finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != tiles;) {
+      __builtin_amdgcn_s_sleep(2);
+      if (++spins >= LOOKBACK_SPIN_LIMIT) {
+        ctl_out->strike_out(-1, [](uint32_t* p, uint32_t x) {
+          __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        });
+        break;
+      }
+    }
+    return __hip_atomic_load(&ctl_out->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
   };
-  // element i of an array, addressed the cheaper way where the offsets allow it
-  auto at = [&](auto* base, uint32_t i) -> auto& {
-    using T = std::remove_reference_t<decltype(*base)>;
-    if constexpr (OFF32) {
-      using B = std::conditional_t<std::is_const<T>::value, const char, char>;
-      return *reinterpret_cast<T*>(reinterpret_cast<B*>(base) + (uint32_t)(i * (uint32_t)sizeof(T)));
-    } else {
-      return base[i];
-    }
+  auto clear_counters = [&] {
+    for (int i = threadIdx.x; i < WAVES * RADIX_SIZE; i += BLOCK) s_cnt[i] = 0;
   };
-
-  // Keys travel between the passes in their encoded form: the first pass that runs encodes them as
-  // it loads, the last one decodes them as it stores (unsigned ascending keys need no transform).
-  const bool encodes = !codec.plain && SortCtl::encodes(todo);  // uniform
-  const bool decodes = !codec.plain && SortCtl::decodes(todo);
-
-  // ---- load (wave-striped); slots past the end sort last inside the tile
-  K e[ITEMS];
-  if (valid == (uint32_t)TILE) {
-    const K* __restrict__ tile_keys = keys_in + tile_base;  // scalar
-#pragma unroll
-    for (int r = 0; r < ITEMS; ++r) e[r] = at(tile_keys, span + r * WAVE);
-    if (encodes) {
-#pragma unroll
-      for (int r = 0; r < ITEMS; ++r) e[r] = codec.encode(e[r]);
-    }
-  } else {
-#pragma unroll
-    for (int r = 0; r < ITEMS; ++r) {
-      const uint32_t pos = span + r * WAVE;
-      K x = (K)~(K)0;
-      if (pos < valid) {
-        x = keys_in[tile_base + pos];
-        if (encodes) x = codec.encode(x);
+  for (int slot = first_slot; slot < slots; ++slot) {
+    uint32_t* ticket = tickets + (size_t)slot * TICKET_CLASSES * TICKET_STRIDE;
+    // One thread asks what there is to do, so that the whole workgroup goes the same way whenever it changes.
+    if (threadIdx.x == 0) {
+      uint32_t todo = __hip_atomic_load(&ctl_out->slot[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (SortCtl::runs(todo)) {
+        s_tile = atomicAdd(ticket, 1u);  // (on its way while the pass before ends)
+        if (!is_complete()) todo = SortCtl::SKIP;
       }
-      e[r] = x;
+      s_todo[slot & 1] = todo;
     }
-  }
-
-  // The values start their way now, so that they have arrived by the time the keys have left:
-  // loaded only after the look-back, their latency was the longest part of what a tile still
-  // had to do once its offsets were known.
-  V v[HAS_VALUES ? ITEMS : 1];
-  if constexpr (HAS_VALUES) {
-    if (valid == (uint32_t)TILE) {
-      // whole tile: no predicates, so that all loads are in flight together (a predicated
-      // load makes the compiler wait for it before issuing the next one)
-      const V* __restrict__ tile_vals = vals_in + tile_base;  // scalar
-#pragma unroll
-      for (int r = 0; r < ITEMS; ++r) v[r] = at(tile_vals, span + r * WAVE);
-    } else {
-#pragma unroll
-      for (int r = 0; r < ITEMS; ++r) {
-        const uint32_t pos = span + r * WAVE;
-        v[r] = (pos < valid) ? vals_in[tile_base + pos] : V{};
-      }
-    }
-  }
-
-  // ---- rank inside the wave by digit
-  uint32_t* my_cnt = s_cnt + wave * RADIX_SIZE;
-  // ranks are < TILE <= 65536: two per register
-  static_assert(TILE <= 65536 && ITEMS % 2 == 0, "rank packing");
-  uint32_t rank2[ITEMS / 2];
-#pragma unroll
-  for (int r = 0; r < ITEMS; ++r) {
-    const uint32_t rank = wave_rank_round(digit_of(e[r]), my_cnt);
-    if (r % 2 == 0) rank2[r / 2] = rank;
-    else rank2[r / 2] |= rank << 16;
-    // pin the packed rank here: otherwise the add is sunk past the barrier and its operands
-    // of every round stay live
-    asm volatile("" : "+v"(rank2[r / 2]));
-    // keep the scheduler from computing all peer masks first (two live registers per
-    // round): rounds are finished in pairs
-    if (r % 2 == 1) __builtin_amdgcn_sched_barrier(0);
-  }
-  __syncthreads();
-
-  // ---- per digit: offsets of the waves, tile count; publish the tile's partial counts
-  uint32_t digit_count = 0;
-  D* my_status = status + (size_t)tile * RADIX_SIZE;
-  if (threadIdx.x < RADIX_SIZE) {
-    const int d = threadIdx.x;
-    uint32_t sum = 0;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      const uint32_t c = s_cnt[w * RADIX_SIZE + d];
-      s_cnt[w * RADIX_SIZE + d] = sum;
-      sum += c;
-    }
-    digit_count = sum;
-    // padding slots carry the all-ones key and must not be counted
-    if (d == (int)dmask) digit_count -= ((uint32_t)TILE - valid);
-    if (tile != 0)
-      __hip_atomic_store(my_status + d, (D)(Desc::PARTIAL | digit_count), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    // exclusive scan of the (padded) counts over the digits -> local run offsets;
-    // the part inside this wave of 64 digits now, the preceding waves after the barrier
-    const uint32_t incl = wave_inclusive_scan(sum, OpPlus{});
-    if (lane == WAVE - 1) s_digit_wave[wave] = incl;
-    s_scatter_base[d] = incl - sum;
-  }
-  __syncthreads();
-  uint32_t local_base = 0;
-  if (threadIdx.x < RADIX_SIZE) {
-    const int d = threadIdx.x;
-    local_base = s_scatter_base[d];
-    for (int w = 0; w < wave; ++w) local_base += s_digit_wave[w];
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) s_cnt[w * RADIX_SIZE + d] += local_base;
-  }
-  __syncthreads();
-
-  // ---- final position of every key inside the tile
-#pragma unroll
-  for (int r = 0; r < ITEMS; ++r) {
-    const uint32_t d = digit_of(e[r]);
-    rank2[r / 2] += my_cnt[d] << (16 * (r % 2));  // no carry: each half stays < TILE
-  }
-  __syncthreads();  // all reads of s_cnt done: the exchange buffer may overwrite it
-
-#pragma unroll
-  for (int r = 0; r < ITEMS; ++r) s_keys[(rank2[r / 2] >> (16 * (r % 2))) & 0xffffu] = e[r];
-
-  // ---- look-back: global offset of each digit run of this tile
-  // Windowed: the descriptors of the LOOKBACK_WINDOW nearest unread predecessors are
-  // fetched together (one memory round trip instead of one per tile), then folded nearest
-  // first up to the first inclusive one.  A descriptor not yet published stops the fold;
-  // the next window starts at that tile.
-  if (threadIdx.x < RADIX_SIZE) {
-    const int d = threadIdx.x;
-    uint32_t excl;
-    if (tile == 0) {
-      excl = bin_base[d];
-    } else {
-      uint32_t acc = 0;
-      int t = (int)tile - 1;  // tile counts stay below 2^20
-      const D* my_col = status + d;
-      uint32_t spins = 0;
-      for (;;) {
-        D s[LOOKBACK_WINDOW];
-#pragma unroll
-        for (int k = 0; k < LOOKBACK_WINDOW; ++k) {
-          const uint32_t tk = (uint32_t)((t - k) > 0 ? (t - k) : 0);  // tile 0 is always inclusive
-          s[k] = __hip_atomic_load(my_col + (size_t)tk * RADIX_SIZE, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // all loads are in flight before the first is used
-        bool done = false;
-        int used = 0;
-#pragma unroll
-        for (int k = 0; k < LOOKBACK_WINDOW; ++k) {
-          const D flag = s[k] & ~Desc::VALUE_MASK;
-          const bool take = !done && used == k && flag != 0;
-          if (take) {
-            acc += (uint32_t)(s[k] & Desc::VALUE_MASK);
-            used = k + 1;
-            done = flag == Desc::INCLUSIVE;
-          }
-        }
-        if (done) break;
-        t -= used;
-        if (used < LOOKBACK_WINDOW) {
-          __builtin_amdgcn_s_sleep(1);
-          ++spins;
-          if (spins >= LOOKBACK_SPIN_LIMIT ||
-              (spins % 1024u == 0 &&
-               __hip_atomic_load(&ctl_out->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-            ctl_out->strike_out(slot, [](uint32_t* p, uint32_t x) {
-              __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            });
-            break;
-          }
-        }
-      }
-      excl = acc;
-    }
-    __hip_atomic_store(my_status + d, (D)(Desc::INCLUSIVE | (D)(uint32_t)(excl + digit_count)), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    // (in bytes of a key where the offsets are 32-bit)
-    s_scatter_base[d] = OFF32 ? (excl - local_base) * (uint32_t)sizeof(K) : excl - local_base;
-  }
-  __syncthreads();
-
-  // ---- keys leave in tile-sorted order: consecutive lanes write consecutive addresses
-  // Batched so that the 2*ITEMS LDS reads are independent and in flight together.
-  uint32_t gpos[ITEMS];
-  {
-    K ek[ITEMS];
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) ek[k] = s_keys[(uint32_t)k * BLOCK + threadIdx.x];
-    // gpos: the key's place in the output, as a byte offset where those fit 32 bits
-    auto key_slot = [&](uint32_t g) -> K& {
-      if constexpr (OFF32) return *reinterpret_cast<K*>(reinterpret_cast<char*>(keys_out) + g);
-      else return keys_out[g];
-    };
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k)
-      gpos[k] = s_scatter_base[digit_of(ek[k])] +
-                (OFF32 ? (uint32_t)(threadIdx.x * sizeof(K)) + (uint32_t)(k * BLOCK * sizeof(K))
-                       : (uint32_t)k * BLOCK + threadIdx.x);
-    if (decodes) {
-#pragma unroll
-      for (int k = 0; k < ITEMS; ++k) ek[k] = codec.decode(ek[k]);
-    }
-    if (valid == (uint32_t)TILE) {
-#pragma unroll
-      for (int k = 0; k < ITEMS; ++k) key_slot(gpos[k]) = ek[k];
-    } else {
-#pragma unroll
-      for (int k = 0; k < ITEMS; ++k)
-        if ((uint32_t)k * BLOCK + threadIdx.x < valid) key_slot(gpos[k]) = ek[k];
-    }
-  }
-  if constexpr (HAS_VALUES) {
-    __syncthreads();  // keys have been read out of the exchange buffer
-#pragma unroll
-    for (int r = 0; r < ITEMS; ++r) s_vals[(rank2[r / 2] >> (16 * (r % 2))) & 0xffffu] = v[r];
+    clear_counters();
     __syncthreads();
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const uint32_t q = (uint32_t)k * BLOCK + threadIdx.x;
-      if constexpr (OFF32) {
-        uint32_t vbyte;
-        if constexpr (sizeof(V) >= sizeof(K)) vbyte = gpos[k] * (uint32_t)(sizeof(V) / sizeof(K));
-        else vbyte = gpos[k] / (uint32_t)(sizeof(K) / sizeof(V));
-        if (q < valid) *reinterpret_cast<V*>(reinterpret_cast<char*>(vals_out) + vbyte) = s_vals[q];
-      } else {
-        if (q < valid) vals_out[gpos[k]] = s_vals[q];
+    const uint32_t todo = __builtin_amdgcn_readfirstlane(s_todo[slot & 1]);
+    if (!SortCtl::runs(todo)) continue;
+    finished = ticket + TICKET_STRIDE;
+    const int pass = (int)SortCtl::digit(todo);
+    const uint32_t* __restrict__ bin_base = hist + pass * RADIX_SIZE;
+    const bool from_alt = SortCtl::src_alt(todo);
+    // (not __restrict__: the next pass reads what this one writes)
+    const K* keys_in = from_alt ? keys_b : keys_a;
+    K* keys_out = from_alt ? keys_a : keys_b;
+    const V* vals_in = from_alt ? vals_b : vals_a;
+    V* vals_out = from_alt ? vals_a : vals_b;
+    D* status = statuses + (size_t)slot * slot_words;
+    for (;;) {
+      const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);
+      if (tile >= tiles) break;
+#define TA_PASS_LOAD(item) __hip_atomic_load(&(item), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+#define TA_PASS_STORE(item, value) __hip_atomic_store(&(item), value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+#include "radix_pass_tile.inc"
+#undef TA_PASS_LOAD
+#undef TA_PASS_STORE
+      // counted in when all of the workgroup's stores have been acknowledged
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        __hip_atomic_fetch_add(finished, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_tile = atomicAdd(ticket, 1u);
       }
+      clear_counters();
+      __syncthreads();
+    }
+    __syncthreads();  // everybody has seen that there are no more tiles
+  }
+  if (!copies) return;
+  if (threadIdx.x == 0) {
+    const bool copy = __hip_atomic_load(&ctl_out->final_in_alt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    s_todo[slots & 1] = copy && is_complete() ? 1u : 0u;
+  }
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(s_todo[slots & 1]) != 0) {
+    for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
+      keys_a[i] = __hip_atomic_load(keys_b + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if constexpr (HAS_VALUES) vals_a[i] = __hip_atomic_load(vals_b + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
 }
@@ -830,13 +703,27 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   TA_CHECK_LAUNCH();
   uint32_t* bounds = reinterpret_cast<uint32_t*>(base + off_bounds);
   uint32_t* long_list = reinterpret_cast<uint32_t*>(base + off_long);
+  const bool tail = top_slots == 2;  // (8-byte keys)
+  const int single_launches = hybrid && n <= REST_MAX<K, HAS_VALUES> ? top_slots : slots;  // passes with a launch of their own
   for (int slot = 0; slot < slots; ++slot) {
     if constexpr (sizeof(K) >= 4) {
       if (hybrid && slot == top_slots) {
-        TA_LAUNCH("sort_bounds", stream, sort_bounds_kernel<K>, dim3((uint32_t)(max_windows / 256 + 1)), dim3(256), (const K*)keys_a, (const K*)keys_b, (uint32_t)n, (uint32_t)Finish::CAP, bounds, (const SortCtl*)ctl);
+        // (stretches of one digit begin where the histogram says)
+        if constexpr (sizeof(K) == 8) {
+          TA_LAUNCH("sort_bounds", stream, sort_bounds_kernel<K>, dim3((uint32_t)(max_windows / 256 + 1)), dim3(256), (const K*)keys_a, (const K*)keys_b, (uint32_t)n, (uint32_t)Finish::CAP, bounds, (const SortCtl*)ctl);
+          TA_CHECK_LAUNCH();
+        }
+        TA_LAUNCH("sort_finish", stream, (sort_finish_kernel<K, V, HAS_VALUES>), dim3((uint32_t)max_windows), dim3(Finish::BLOCK), keys_a, (const K*)keys_b, vals_a, (const V*)vals_b, (uint32_t)n, codec, (const uint32_t*)bounds, (const uint32_t*)hist, (const SortCtl*)ctl, &ctl->long_windows, long_list, status + (size_t)top_slots * slot_words, (uint64_t)((slots - top_slots) * slot_words));
         TA_CHECK_LAUNCH();
-        TA_LAUNCH("sort_finish", stream, (sort_finish_kernel<K, V, HAS_VALUES>), dim3((uint32_t)max_windows), dim3(Finish::BLOCK), keys_a, (const K*)keys_b, vals_a, (const V*)vals_b, (uint32_t)n, codec, (const uint32_t*)bounds, (const SortCtl*)ctl, &ctl->long_windows, long_list, status + (size_t)top_slots * slot_words, (uint64_t)((slots - top_slots) * slot_words));
+      }
+    }
+    if constexpr (sizeof(K) >= 4) {
+      if (slot >= single_launches) {
+        static_assert(REST_MAX<K, HAS_VALUES> <= Plan::FINE_MAX, "tiles as in the passes before, 32-bit offsets");
+        TA_LAUNCH("onesweep_rest", stream, (onesweep_rest_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::FINE_ITEMS>), dim3((uint32_t)tiles), dim3(Plan::BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, slot, slots, (uint32_t)tiles, geo, codec, (const uint32_t*)hist, status, (uint64_t)slot_words, tickets, (const SortCtl*)ctl, ctl, !tail);
         TA_CHECK_LAUNCH();
+        if (!tail) return 0;
+        break;
       }
     }
     const char* label = hybrid && slot >= top_slots ? "onesweep_rest" : "onesweep_pass";

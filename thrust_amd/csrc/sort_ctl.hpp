@@ -38,7 +38,7 @@ struct SortCtl {
   TA_CTL_FN bool finishes() const { return fast != 0; }
   TA_CTL_FN bool copies_back() const { return final_in_alt != 0; }
 
-  // What a tile of the launch in `slot` does when it stops waiting.  The array is not in the order, and does not hold
+  // What a tile of the pass in slot `at` does when it stops waiting (-1: between passes).  The array is not in the order, and does not hold
   // the keys, that the launches behind it count on -- their positions could leave it -- so they are struck out: the
   // call ends with an unfinished sort.  store(address, value) has to reach the next launch; fields that the
   // running launch reads stay as they are.
