@@ -146,12 +146,14 @@ def test_sorts_by_top_digits(dev, dtype, kind):
                 assert np.array_equal(w.numpy(), v[order]), (n, vdtype, descending)
 
 
-# Sizes up to which the last step fits one digit, tiles are small, and pairs of 4-byte keys run two workgroups per CU
+# Sizes up to which the last step fits one digit, tiles are small, and tiles of 4-byte keys are of the middle size
 # (SortPlan and sort_impl in thrust_amd/csrc/radix_sort.hip), and where the two-digit way ends.
 EDGES = [(np.uint32, None, 256 * 6144), (np.int32, np.uint16, 256 * 6144), (np.float32, np.uint32, 8 * 6144),
          (np.int32, np.uint64, 256 * 2560), (np.float64, None, 1 << 19),
          (np.uint8, None, 16384 * 160), (np.uint16, np.uint64, 8192 * 160), (np.uint32, None, 18432 * 160),
          (np.int32, np.uint8, 16384 * 160), (np.uint64, np.uint32, 8192 * 160),
+         (np.uint32, np.uint32, 14336 * 160), (np.float32, np.uint8, 14336 * 160), (np.uint32, None, 10240 * 512),
+         (np.float32, np.uint32, 10240 * 512), (np.int32, np.uint16, 10240 * 512),
          (np.uint32, np.uint8, 1 << 22), (np.int32, np.uint16, 1 << 22), (np.float32, np.uint32, 1 << 22),
          (np.uint32, np.uint16, (1 << 24) - 1)]
 

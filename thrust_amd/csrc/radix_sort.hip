@@ -401,9 +401,8 @@ constexpr int LOOKBACK_WINDOW = 4;
 // OFF32: every key and value of the call lies within 4 GiB of its array's start, so that
 // global addresses are a scalar base plus a 32-bit byte offset (one vector instruction per
 // access less than with 64-bit address arithmetic).
-// CROWDED: registers are held to what two workgroups per CU leave each, at the cost of some spills.
-template <typename K, typename V, bool HAS_VALUES, int BLOCK, int ITEMS, typename D, bool OFF32, bool CROWDED>
-__global__ __launch_bounds__(BLOCK, CROWDED ? 2 * BLOCK / WAVE / 4 : 1) void onesweep_pass_kernel(
+template <typename K, typename V, bool HAS_VALUES, int BLOCK, int ITEMS, typename D, bool OFF32>
+__global__ __launch_bounds__(BLOCK) void onesweep_pass_kernel(
     K* __restrict__ keys_a, K* __restrict__ keys_b, V* __restrict__ vals_a, V* __restrict__ vals_b,
     uint32_t n, int slot, SortGeometry geo, KeyCodec<K> codec,
     const uint32_t* __restrict__ hist,      // [passes][RADIX_SIZE] global digit offsets
@@ -580,26 +579,34 @@ __global__ __launch_bounds__(256) void sort_copy_back_kernel(K* __restrict__ key
 // ------------------------------------------------------------------ host side
 template <typename K, typename V, bool HAS_VALUES>
 struct SortPlan {
-  // Large tiles (16K-18K keys of 4 bytes) keep the number of tiles in flight, and with it
+  // Large tiles (14K-18K keys of 4 bytes) keep the number of tiles in flight, and with it
   // the length of every look-back, small; two blocks of 1024 threads fill a CU (64 VGPRs,
-  // 80 KB of LDS each).  8-byte keys or values halve the tile to fit LDS.
+  // 80 KB of LDS each).  8-byte keys or values halve the tile to fit LDS.  4-byte keys with values: 14 keys per lane are
+  // what 64 registers hold.  With 16, 74 registers and one workgroup per CU, or 64 and 36 bytes of spills: a pass over
+  // 8e6 pairs 36.9 us (with spills) -> 34.8, 1.6e7 72.9 -> 57.5, 2.4e7 114 -> 94, 6.4e7 249 -> 235, 1.34e8 486 -> 463; with 12
+  // 35.2, 59.6, 94, 235, 474.
   static constexpr int BLOCK = 1024;
   static constexpr int ITEMS = (sizeof(K) == 8 || (HAS_VALUES && sizeof(V) == 8)) ? 8
-                               : (sizeof(K) == 4 && !HAS_VALUES)                 ? 18
+                               : sizeof(K) == 4                                  ? (HAS_VALUES ? 14 : 18)
                                                                                  : 16;
   static constexpr int TILE = BLOCK * ITEMS;
+  // Arrays of 4 GiB and more need 64-bit addresses, with which one workgroup of either size fills a CU's registers.
+  static constexpr int FAR_ITEMS = ITEMS == 14 ? 16 : ITEMS;
   // Where tiles of this size are fewer than the CUs: a third or half of it.  The time is that of one or two tiles
   // then, and shorter with smaller ones.  Sort of 1e6 and 2.6e6 random keys, large tiles against small ones: float32 76 -> 65,
-  // 97 -> 93 us; with uint32 values 86 -> 75, 102 -> 94; uint8 29.4 -> 27.5, 34.3 -> 34.3; uint16 42.6 -> 38.8, 50.6 -> 50.5;
-  // (uint16, uint64) 47 -> 45, and 51.5 -> 51.7 at 1.6e6; float64 137 -> 130 at 1e6.  Float32 at 4e6: 106 -> 110.
+  // 97 -> 93 us; with uint32 values (tiles of 16384) 86 -> 75, 102 -> 94; uint8 29.4 -> 27.5, 34.3 -> 34.3; uint16 42.6 -> 38.8,
+  // 50.6 -> 50.5; (uint16, uint64) 47 -> 45, and 51.5 -> 51.7 at 1.6e6; float64 137 -> 130 at 1e6.  Float32 at 4e6: 106 -> 110.
   static constexpr int FINE_ITEMS = ITEMS == 8 ? 4 : 6;
   static constexpr uint64_t FINE_MAX = (uint64_t)TILE * NUM_CU * 5 / 8;
-  // 4-byte keys with values need 74 registers, a workgroup per CU.  Two with 64 and 36 bytes of spills each win while
-  // there are a few tiles per CU (8e6 pairs 194 -> 177 us) and lose with one or with many (4e6 115 -> 126, 16e6
-  // 352 -> 353, 32e6 695 -> 718).
-  static constexpr bool TIGHT = sizeof(K) == 4 && HAS_VALUES && ITEMS == 16;
-  static constexpr uint64_t TIGHT_MIN = (uint64_t)TILE * NUM_CU, TIGHT_MAX = 1u << 24;
   static constexpr int FINE_TILE = BLOCK * FINE_ITEMS;
+  // 4-byte keys, as long as tiles of 10 keys per lane all run at once, two to a CU: copy and sort of 3.2e6, 4e6 and 5.2e6
+  // keys 101 -> 96, 104 -> 103, 115 -> 106 us, with uint32 values 108 -> 108, 114 -> 115, 154 -> 126 (14 keys per lane: 134),
+  // and in a second round the others are better: 6e6 keys 119.6 against 121, pairs 136 against 148.  8-byte keys with 6 per
+  // lane: 4e6 118 against 124.
+  static constexpr bool HAS_MID = sizeof(K) == 4 && ITEMS != 8;
+  static constexpr int MID_ITEMS = HAS_MID ? 10 : ITEMS;
+  static constexpr int MID_TILE = BLOCK * MID_ITEMS;
+  static constexpr uint64_t MID_MAX = HAS_MID ? (uint64_t)MID_TILE * NUM_CU * 2 : 0;
 };
 
 template <typename K, typename V, bool HAS_VALUES>
@@ -614,16 +621,16 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   geo.end_bit = end_bit;
   geo.passes = (end_bit - begin_bit + RADIX_BITS - 1) / RADIX_BITS;
   const bool fine = n <= Plan::FINE_MAX;
-  const bool crowded = Plan::TIGHT && n > Plan::TIGHT_MIN && n < Plan::TIGHT_MAX;
-  const uint64_t tile = fine ? Plan::FINE_TILE : Plan::TILE;
+  const bool mid = !fine && n <= Plan::MID_MAX;
+  const bool wide = n > SORT_MAX_N_NARROW;  // prefixes need more than 30 bits: 64-bit descriptors
+  // every key and value within 4 GiB of its array's start: 32-bit byte offsets
+  const bool off32 = !wide && n * (uint64_t)((HAS_VALUES && sizeof(V) > sizeof(K)) ? sizeof(V) : sizeof(K)) <= (1ull << 32);
+  const uint64_t tile = fine ? Plan::FINE_TILE : mid ? Plan::MID_TILE : off32 ? Plan::TILE : Plan::BLOCK * Plan::FAR_ITEMS;
   const uint64_t tiles = (n + tile - 1) / tile;
 
   TempLayout lay;
   const size_t off_ctl = lay.add(sizeof(SortCtl));
   // contiguous zero-initialised region: tickets, histograms, tile descriptors
-  const bool wide = n > SORT_MAX_N_NARROW;  // prefixes need more than 30 bits: 64-bit descriptors
-  // every key and value within 4 GiB of its array's start: 32-bit byte offsets
-  const bool off32 = !wide && n * (uint64_t)((HAS_VALUES && sizeof(V) > sizeof(K)) ? sizeof(V) : sizeof(K)) <= (1ull << 32);
   // The short way, over whole keys only.  Against all digits' passes, sort of random keys:
   //   8-byte keys      1e4 keys 84 -> 48 us, 1e6 135 -> 79, 8e6 309 -> 166, 1.34e8 4130 -> 1960; with 4-byte values
   //                    92 -> 49, 157 -> 86, 363 -> 197, 5790 -> 2700 us; where keys repeat 10 to 30 times 0.66-0.85 of the
@@ -732,11 +739,11 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
     auto launch = [&](auto kernel, auto* descriptors) {
       TA_LAUNCH(label, stream, kernel, dim3((uint32_t)tiles), dim3(Plan::BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, slot, geo, codec, (const uint32_t*)hist, descriptors, slot_tickets, (const SortCtl*)ctl, ctl);
     };
-    if (fine) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::FINE_ITEMS, uint32_t, true, false>, slot_status);
-    else if (off32 && crowded) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, true, Plan::TIGHT>, slot_status);
-    else if (off32) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, true, false>, slot_status);
-    else if (wide) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint64_t, false, false>, reinterpret_cast<uint64_t*>(slot_status));
-    else launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, false, false>, slot_status);
+    if (fine) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::FINE_ITEMS, uint32_t, true>, slot_status);
+    else if (mid) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::MID_ITEMS, uint32_t, true>, slot_status);
+    else if (off32) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::ITEMS, uint32_t, true>, slot_status);
+    else if (wide) launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::FAR_ITEMS, uint64_t, false>, reinterpret_cast<uint64_t*>(slot_status));
+    else launch(onesweep_pass_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::FAR_ITEMS, uint32_t, false>, slot_status);
     TA_CHECK_LAUNCH();
   }
   if constexpr (sizeof(K) == 8) {
