@@ -13,8 +13,8 @@
 // turns counts into starts, the keys are laid out by bin, and each key counts the keys of its bin that belong in front
 // of it -- the smaller ones and, among equal ones, those that stood in front -- so the atomics' order does not show.
 // What bounds it: the latency of its ten steps for the 2000 keys of a workgroup, three workgroups to a CU, and vector
-// instructions: 142 per pair of (uint64, uint32) keep the SIMDs half busy; LDS is busy 28 % of the time.  2^27 pairs: 0.97 ms
-// (3.3 TB/s) in place of six passes of 0.69; keys alone 0.65 in place of six of 0.48.  Workgroups that loop over windows
+// instructions.  2^27 pairs of (uint64, uint32): 0.69 ms (4.7 TB/s) in place of six passes of 0.69; keys alone 0.56 in place
+// of six of 0.48.  Workgroups that loop over windows
 // save their dispatch where the chained passes do the sort (40 us for 2^27 keys), but cost registers (0.85 -> 1.19 ms).
 // A bin of more than FINISH_BIN_MAX keys (many equal keys, values in clusters) makes the workgroup run stable passes
 // over the digits that vary instead: three times as long for 2^27 uint64 that repeat 30 times (the sort still takes 0.8
@@ -90,13 +90,11 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
     uint32_t* __restrict__ status, uint64_t status_words) {
   using Shape = FinishShape<K, V, HAS_VALUES>;
   constexpr int BLOCK = Shape::BLOCK, ITEMS = Shape::ITEMS, CAP = Shape::CAP, WAVES = BLOCK / WAVE;
-  constexpr bool BIG = Shape::BIG;
   constexpr int BINS = CAP;                // 16-bit counts, two to a word
   constexpr int BIN_WORDS = BINS / 2;
   constexpr int LOG_BINS = __builtin_ctz(BINS);
   constexpr int MY_WORDS = BIN_WORDS / BLOCK;
   constexpr int TRASH = 32;
-  constexpr int GROUP = 2;                 // rounds without a branch between them
   constexpr int SIDE = 7;                  // places looked at on either side of a key
   // 8-byte keys are told apart by 32 bits; they are then moved like values, by the 16-bit place they had before
   constexpr bool KEYS_MOVE = sizeof(K) == 8;
@@ -106,7 +104,6 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   constexpr size_t REST_BYTES = KEYS_MOVE ? CAP * sizeof(uint32_t) : 0;  // what the codes leave out of a key
   constexpr size_t FRONT_BYTES = CODE_BYTES + REST_BYTES > CAP * ITEM ? CODE_BYTES + REST_BYTES : CAP * ITEM;
   static_assert(BLOCK >= RADIX_SIZE && (CAP & (CAP - 1)) == 0 && CAP <= 8192 && MY_WORDS % 4 == 0, "shape");
-  static_assert(ITEMS % GROUP == 0, "groups");
   static_assert(WAVES * RADIX_SIZE <= BIN_WORDS, "the passes' counters lie over the bins");
 
   if (!ctl->finishes()) {
@@ -158,18 +155,16 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   const V* __restrict__ vals_in = HAS_VALUES ? (ctl->fast_src_alt ? vals_b : vals_a) + first : nullptr;
   K* __restrict__ keys_out = keys_a + first;
   V* __restrict__ vals_out = HAS_VALUES ? vals_a + first : nullptr;
-  // f(r, the place r * BLOCK + tid) for all rounds, in groups of straight-line code: a branch per round makes the
-  // compiler wait for each round's loads before the next one's
+  // f(r, the place r * BLOCK + tid) for all rounds, each behind a branch of its own (in pairs, without a branch inside,
+  // the loads of two are in flight together, but an odd round more is computed and registers spill: 0.97 against 0.73 ms
+  // for 2^27 pairs of (uint64, uint32), 0.63 against 0.56 for keys alone)
   // (opaque copy: what a sweep derives from the place is not kept in registers for the next)
   auto each_round = [&](auto f) {
     uint32_t t = tid;
     asm volatile("" : "+v"(t));
 #pragma unroll
-    for (int g = 0; g < ITEMS; g += GROUP) {
-      if (g < rounds) {
-#pragma unroll
-        for (int r = g; r < g + GROUP; ++r) f(r, (uint32_t)r * BLOCK + t);
-      }
+    for (int r = 0; r < ITEMS; ++r) {
+      if (r < rounds) f(r, (uint32_t)r * BLOCK + t);
     }
   };
 
@@ -180,7 +175,6 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   auto load_values = [&] {
     each_round([&](int r, uint32_t p) { v[r] = vals_in[p < count ? p : count - 1]; });
   };
-  if constexpr (HAS_VALUES && BIG) load_values();
   // the prefixes are in order, so the first and the last one say where all keys lie
   const int prefix_bit = (int)ctl->prefix_bit;
   const K lo = keys_in[0] >> prefix_bit << prefix_bit;
@@ -268,7 +262,9 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
       s_code[count + tid] = ~0u;
     }
     __syncthreads();
-    if constexpr (HAS_VALUES && !BIG) load_values();  // not earlier: the registers hold the keys until here
+    // not earlier: the registers hold the keys until here (asked for with the 8-byte keys, values cost 32 bytes of
+    // spills: 2^27 pairs 0.73 against 0.69 ms, 1.6e7 109 against 82 us)
+    if constexpr (HAS_VALUES) load_values();
     // ---- inside the bins: keys of lower bins are smaller and lie in front, so a lane counts the keys on the wrong
     // side of its own, without asking for their bins, as far as the fullest bin can reach.  4-byte keys leave
     // straight for their places: a wave's lie next to each other but for those steps.

@@ -632,12 +632,12 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   const size_t off_ctl = lay.add(sizeof(SortCtl));
   // contiguous zero-initialised region: tickets, histograms, tile descriptors
   // The short way, over whole keys only.  Against all digits' passes, sort of random keys:
-  //   8-byte keys      1e4 keys 84 -> 48 us, 1e6 135 -> 79, 8e6 309 -> 166, 1.34e8 4130 -> 1960; with 4-byte values
-  //                    92 -> 49, 157 -> 86, 363 -> 197, 5790 -> 2700 us; where keys repeat 10 to 30 times 0.66-0.85 of the
+  //   8-byte keys      1e4 keys 84 -> 32 us, 1e6 135 -> 79, 8e6 309 -> 166, 1.34e8 4130 -> 1880; with 4-byte values
+  //                    92 -> 36, 157 -> 85, 363 -> 180, 5790 -> 2430 us; where keys repeat 10 to 30 times 0.66-0.85 of the
   //                    time, where the plan declines 1.00-1.05 (5 to 10 us up to 8e6 keys, 1 % at 1.34e8; 1.04-1.09 where
   //                    one digit varies): two launches that do nothing, one of them of a workgroup per window
-  //   4-byte integers  by one digit (as long as its bins can fit at all) 1e4 keys 68 -> 40 us, 1e6 75 -> 49; with
-  //                    values 70 -> 41, 85 -> 55.  Never by two digits: that saves two passes and costs the last step,
+  //   4-byte integers  by one digit (as long as its bins can fit at all) 1e4 keys 68 -> 22 us, 1e6 75 -> 35; with
+  //                    values 70 -> 26, 85 -> 50.  Never by two digits: that saves two passes and costs the last step,
   //                    0.95-1.06 times as fast for random keys of 2^25 and more, and where keys repeat (ten times or a
   //                    thousand) the stretches outgrow a workgroup: 2^28 keys 2170 -> 3220 us when all passes follow.
   //   floats           share few exponents: 4-byte ones outgrow a workgroup at some 20000 keys, 8-byte ones (four
