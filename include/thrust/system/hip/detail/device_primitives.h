@@ -9,6 +9,8 @@
 #include <stdint.h>
 #include <type_traits>
 
+#include "merge_search.h"
+
 #define THRUST_AMD_DEVICE __device__ __forceinline__
 #define THRUST_AMD_HOST_DEVICE __host__ __device__ __forceinline__
 
@@ -217,25 +219,6 @@ template <typename Pred>
 THRUST_AMD_DEVICE uint64_t partition_point(uint64_t lo, uint64_t hi, Pred pred) {
   while (lo < hi) {
     const uint64_t mid = (lo + hi) >> 1;
-    if (pred(mid)) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
-
-
-// The same search, probing at every step the index of its interval that is a multiple of the
-// largest power of two.  It needs as many steps as the bisection at worst, but the probes of the
-// first steps are the same few indices for every thread that searches the same arrays (the
-// nodes of one implicit tree over the index range), so they come from the caches instead of
-// each being a miss of its own: the searches for the tile boundaries of a merge of 2 x 2^27 keys
-// (65537 threads, 27 dependent steps each) took 108 us with the plain bisection.
-template <typename Pred>
-THRUST_AMD_DEVICE uint64_t aligned_partition_point(uint64_t lo, uint64_t hi, Pred pred) {
-  while (lo < hi) {
-    const uint64_t last = hi - 1;
-    const uint64_t differ = lo ^ last;
-    const uint64_t mid = differ ? (last & ~((1ull << (63 - __builtin_clzll(differ))) - 1ull)) : lo;
     if (pred(mid)) lo = mid + 1;
     else hi = mid;
   }

@@ -55,36 +55,26 @@ THRUST_AMD_DEVICE uint64_t merge_path(PA a, uint64_t na, PB b, uint64_t nb, uint
 }
 
 // The same search by groups of 2^BITS consecutive lanes (every lane of the wave active), each group for a diagonal of
-// its own.  A round probes the multiples of 2^(BITS k) in the interval, at most a group of them, so that an interval
-// below 2^(BITS (k + 1)) shrinks below 2^(BITS k).  The places of the coarse rounds are the same for all groups and
-// come from the caches.
+// its own.  The places of the coarse rounds are the same for all groups and come from the caches.
 template <int BITS, typename T, typename Comp>
 THRUST_AMD_DEVICE uint64_t group_merge_path(const T* __restrict__ a, uint64_t na, const T* __restrict__ b, uint64_t nb,
                                             uint64_t diag, Comp& comp) {
   constexpr uint32_t PROBES = 1u << BITS;
   const uint32_t lane = threadIdx.x % WAVE;
-  uint64_t lo = diag > nb ? diag - nb : 0;
-  uint64_t hi = diag < na ? diag : na;
-  const uint64_t longest = na < nb ? na : nb;  // no interval is longer
-  int bit = longest > 1 ? (63 - __builtin_clzll(longest)) / BITS * BITS : 0;
-  for (; bit >= 0; bit -= BITS) {
-    const uint64_t unit = 1ull << bit;
-    const uint64_t first = (lo + unit - 1) & ~(unit - 1);
-    const uint64_t mid = first + (uint64_t)(lane % PROBES) * unit;
+  SplitInterval in(diag, na, nb);
+  for (int bit = GroupRound<BITS>::first_bit(na, nb); bit >= 0; bit -= BITS) {
+    const GroupRound<BITS> round(in, bit);
+    const uint64_t mid = round.probe(lane % PROBES);
     bool from_a = false;
-    if (mid < hi) {
+    if (mid < in.hi) {
       const T ka = a[mid];
       const T kb = b[diag - 1 - mid];
       from_a = !comp(kb, ka);
     }
-    // in each group the lanes that say yes are the lowest ones
     const uint64_t said_yes = __builtin_amdgcn_ballot_w64(from_a) >> (lane & ~(PROBES - 1));
-    const uint32_t yes = (uint32_t)__builtin_popcount((uint32_t)said_yes & (uint32_t)((1ull << PROBES) - 1));
-    const uint64_t no = first + (uint64_t)yes * unit;  // the first probe that said no, if it was one
-    if (yes > 0) lo = no - unit + 1;
-    if (yes < PROBES && no < hi) hi = no;
+    round.narrow(in, (uint32_t)__builtin_popcount((uint32_t)said_yes & (uint32_t)((1ull << PROBES) - 1)));
   }
-  return lo;
+  return in.lo;
 }
 
 // Tile boundary t for group t of 2^BITS lanes.  With MERGE_TILE a multiple of the probes' coarse distances, the places of
@@ -100,7 +90,8 @@ __global__ __launch_bounds__(256) void merge_partition_kernel(const T* __restric
   if (diag > total) diag = total;
   uint64_t split;
   if constexpr (BITS == 0) {
-    split = aligned_partition_point(diag > nb ? diag - nb : 0, diag < na ? diag : na, [&](uint64_t mid) {
+    const SplitInterval in(diag, na, nb);
+    split = aligned_partition_point(in.lo, in.hi, [&](uint64_t mid) {
       const T ka = a[mid];
       const T kb = b[diag - 1 - mid];
       return !comp(kb, ka);
@@ -132,7 +123,7 @@ __global__ __launch_bounds__(MERGE_BLOCK) void merge_kernel(
   const uint64_t total = na + nb;
   const uint64_t d0 = tile * MERGE_TILE;
   const uint64_t d1 = (d0 + MERGE_TILE < total) ? d0 + MERGE_TILE : total;
-  uint64_t a0, a1;
+  uint64_t split0, split1;
   if constexpr (SEARCHES) {
     __shared__ uint64_t s_split[2];
     if (threadIdx.x < WAVE) {
@@ -140,15 +131,14 @@ __global__ __launch_bounds__(MERGE_BLOCK) void merge_kernel(
       if (threadIdx.x % (WAVE / 2) == 0) s_split[threadIdx.x / (WAVE / 2)] = split;
     }
     __syncthreads();
-    a0 = wave_uniform(s_split[0]);
-    a1 = wave_uniform(s_split[1]);
-    // keys that are in no order (NaN among them) must not lead out of the ranges
-    if (a1 < a0) a1 = a0;
-    if (a1 - a0 > d1 - d0) a1 = a0 + (d1 - d0);
+    split0 = wave_uniform(s_split[0]);
+    split1 = wave_uniform(s_split[1]);
   } else {
-    a0 = a_split[tile];
-    a1 = a_split[tile + 1];
+    split0 = a_split[tile];
+    split1 = a_split[tile + 1];
   }
+  const TileSplit split(split0, split1, d1 - d0);
+  const uint64_t a0 = split.a0, a1 = split.a1;
   const uint64_t b0 = d0 - a0, b1 = d1 - a1;
   const uint32_t ca = (uint32_t)(a1 - a0), cb = (uint32_t)(b1 - b0);
   const uint32_t count = ca + cb;  // == d1 - d0

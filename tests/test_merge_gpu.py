@@ -103,3 +103,21 @@ def test_boundaries_by_groups_of_lanes(dev, n, kind):
     order = np.argsort(both, kind="stable")
     assert np.array_equal(keys.numpy(), both[order]) and np.array_equal(values.numpy(), order.astype(np.uint32))
     assert np.array_equal(dev.merge(arrays[0], arrays[1]).numpy(), both[order])
+
+
+@pytest.mark.parametrize("n", [30011, (1 << 23) - 5, (1 << 23) + 4099, (1 << 25) + 1])
+def test_keys_in_no_order_stay_inside_the_ranges(dev, n):
+    """NaN in the keys breaks what merge asks of its input, and the boundaries of its tiles may run backward then: the
+    result has no order to check, but every element of it is one of the input's, with its own value."""
+    raw = (datagen.splitmix64(17, n) >> np.uint64(40)).astype(np.float32)
+    na = n // 2
+    keys = np.concatenate([np.sort(raw[:na]), np.sort(raw[na:])])
+    keys[datagen.splitmix64(19, n) % np.uint64(3) == 0] = np.nan
+    keys[:na // 10] = np.nan
+    da, db = dev.DeviceArray.from_numpy(keys[:na]), dev.DeviceArray.from_numpy(keys[na:])
+    index = np.arange(n, dtype=np.uint32)
+    out_k, out_v = dev.merge_by_key(da, db, dev.DeviceArray.from_numpy(index[:na]), dev.DeviceArray.from_numpy(index[na:]))
+    values = out_v.numpy()
+    assert values.max() < n
+    assert np.array_equal(out_k.numpy().view(np.uint32), keys.view(np.uint32)[values])
+    assert dev.merge(da, db).numpy().size == n
