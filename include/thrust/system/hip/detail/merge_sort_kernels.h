@@ -27,6 +27,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "merge_search.h"
+
 #ifndef THRUST_AMD_MERGE_SORT_LAUNCH
 #define THRUST_AMD_MERGE_SORT_LAUNCH(label, stream, kernel, grid, block, ...) \
   hipLaunchKernelGGL(kernel, grid, block, 0, stream, __VA_ARGS__)
@@ -253,8 +255,9 @@ __global__ __launch_bounds__(BLOCK) void merge_pass_kernel(const K* keys_in, con
   const PairOfRuns p = pair_of<LONE>(tile, run, n);
   const uint64_t pair_len = p.na + p.nb;
   const uint64_t out1 = (p.out0 + TILE < pair_len) ? p.out0 + TILE : pair_len;
-  const uint64_t a0 = split[tile];
-  const uint64_t a1 = (out1 == pair_len) ? p.na : split[tile + 1];  // same pair: tile + 1 < tiles
+  // (same pair: tile + 1 < tiles); a comparator that is no strict weak order -- NaN keys -- must not lead out of the runs
+  const prim::TileSplit ends(split[tile], (out1 == pair_len) ? p.na : split[tile + 1], out1 - p.out0);
+  const uint64_t a0 = ends.a0, a1 = ends.a1;
   const uint64_t b0 = p.out0 - a0, b1 = out1 - a1;
   const uint32_t ca = (uint32_t)(a1 - a0), cb = (uint32_t)(b1 - b0);
   const uint32_t count = ca + cb;

@@ -152,3 +152,17 @@ def test_merge_sort_full_size_properties(dev):
     assert bool((keys[ov.to(torch.int64)] == ok).all().item())          # every value still sits with its key
     same = ok[1:] == ok[:-1]
     assert bool((ov[1:][same] > ov[:-1][same]).all().item())            # equal keys keep their input order
+
+
+@pytest.mark.parametrize("n", [8192, 25 * 4096, (1 << 21) + 4096])
+def test_keys_without_an_order_stay_inside_the_runs(dev, n):
+    """NaN keys are outside what the comparison sort promises to order, and the boundaries of its merges' tiles may run
+    backward then: every element of the result is one of the input's all the same, with its own value (whole tiles only:
+    what fills up a ragged one has the greatest key and another value)."""
+    keys = (datagen.splitmix64(23, n) >> np.uint64(40)).astype(np.float32)
+    keys[datagen.splitmix64(29, n) % np.uint64(3) == 0] = np.nan
+    d, v = dev.DeviceArray.from_numpy(keys), dev.DeviceArray.from_numpy(np.arange(n, dtype=np.uint32))
+    dev.merge_sort_pairs(d, v)
+    values = v.numpy()
+    assert values.max() < n
+    assert np.array_equal(d.numpy().view(np.uint32), keys.view(np.uint32)[values])
