@@ -35,9 +35,12 @@ constexpr uint64_t SCAN_LARGE_MIN_BYTES = (uint64_t)32 << 20;
 // Tiles of 64 KiB instead of 16: 64 MB 32.5, the others alike.
 struct ScanShapeTwo { static constexpr int BLOCK = 256, CHUNKS = 4; };
 constexpr uint64_t SCAN_TWO_MAX_BYTES = (uint64_t)64 << 20;
-// An array that fits one workgroup of this shape (128 KiB) takes the second launch alone: 32768 int32
-// 9.7 -> 6.8 us with its host call, which is what both figures are made of.
-struct ScanShapeOne { static constexpr int BLOCK = 1024, CHUNKS = 8; };
+// An array that fits one workgroup takes the second launch alone: up to 16 KiB one of the shape above, elements of 4 and
+// 8 bytes up to 64 KiB one of this shape.  Whole call back to back in us, single pass / here: 4093 int32 7.2 / 4.3, 8445
+// 7.3 / 4.7, 16381 7.2 / 6.8 (two launches 7.1), 8189 float64 7.5 / 4.8; int8 8189 7.9 / 6.3, uint8 minimum 4093 7.7 / 5.7.
+// Eight vectors per lane, and arrays of up to 128 KiB: 16381 int32 7.1, 32509 11.7 (two launches 7.2); smaller elements, as
+// many more of them, spill, 102397 int8 36 (two launches 7.9).
+struct ScanShapeOne { static constexpr int BLOCK = 1024, CHUNKS = 4; };
 
 static __global__ void tile_state_init_kernel(uint64_t* __restrict__ words, uint64_t count,
                                        uint32_t* __restrict__ counters, uint32_t num_counters) {
@@ -340,11 +343,18 @@ __global__ __launch_bounds__(Shape::BLOCK) void scan_apply_kernel(const T* in, T
   __syncthreads();
   T wave_prefix = id;
   T prefix = id;
+  if constexpr (WAVES > 4) {
+    // the totals of many waves by a scan of their own: fewer terms in a row, in time and in rounding
+    const T totals = wave_inclusive_scan(lane < WAVES ? s_wave_agg[lane] : id, op, id);
+    if (wave > 0) wave_prefix = readlane(totals, wave - 1);
+  } else {
 #pragma unroll
-  for (int w = 0; w < WAVES; ++w) {
-    if (w < wave) wave_prefix = op(wave_prefix, s_wave_agg[w]);
-    prefix = op(prefix, s_before[w]);
+    for (int w = 0; w < WAVES; ++w) {
+      if (w < wave) wave_prefix = op(wave_prefix, s_wave_agg[w]);
+    }
   }
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) prefix = op(prefix, s_before[w]);
   if constexpr (EXCLUSIVE) prefix = (tile == 0) ? init : op(init, prefix);
   prefix = op(prefix, wave_prefix);
 #pragma unroll
@@ -399,28 +409,44 @@ struct ScanLaunch {
     return 0;
   }
 
-  // One launch where the array is one tile, else two; `temp` holds the partials of the tiles.
+  // An array of one tile, in one launch.
   template <typename T, typename Op, typename Shape>
+  static int run_one_tile(void* temp, size_t* temp_bytes, const T* in, T* out, uint64_t n, const void* init, hipStream_t stream) {
+    T init_v;
+    const int rc = check_args<T, Op>(temp, temp_bytes, partials_bytes<T>(n), in, out, n, init, init_v);
+    if (rc != 0 || temp == nullptr || n == 0) return rc;
+    return launch_apply<T, Op, Shape>(1, in, out, n, init_v, nullptr, stream);
+  }
+
+  // Two launches; `temp` holds the partials of the tiles.
+  template <typename T, typename Op>
   static int run_two_launches(void* temp, size_t* temp_bytes, const T* in, T* out, uint64_t n, const void* init,
                               hipStream_t stream) {
-    const uint32_t tiles = (uint32_t)((n + tile_of<Shape, T>() - 1) / tile_of<Shape, T>());
-    TempLayout lay;
-    const size_t off_partials = lay.add((size_t)tiles * sizeof(T));
+    using Shape = ScanShapeTwo;
     T init_v;
-    const int rc = check_args<T, Op>(temp, temp_bytes, lay.total, in, out, n, init, init_v);
+    const int rc = check_args<T, Op>(temp, temp_bytes, partials_bytes<T>(n), in, out, n, init, init_v);
     if (rc != 0 || temp == nullptr || n == 0) return rc;
-    T* partials = reinterpret_cast<T*>(static_cast<char*>(temp) + off_partials);
-    if (tiles > 1) {
-      if (is_aligned16(in))
-        TA_LAUNCH("scan_partials", stream, (scan_partials_kernel<T, Op, Pre, true, Shape>), dim3(tiles - 1), dim3(Shape::BLOCK), in, partials);
-      else
-        TA_LAUNCH("scan_partials", stream, (scan_partials_kernel<T, Op, Pre, false, Shape>), dim3(tiles - 1), dim3(Shape::BLOCK), in, partials);
-      TA_CHECK_LAUNCH();
-    }
-    if (is_aligned16(in) && is_aligned16(out))
-      TA_LAUNCH("scan", stream, (scan_apply_kernel<T, Op, Pre, EXCLUSIVE, true, Shape>), dim3(tiles), dim3(Shape::BLOCK), in, out, n, init_v, (const T*)partials);
+    const uint32_t tiles = (uint32_t)((n + tile_of<Shape, T>() - 1) / tile_of<Shape, T>());
+    T* partials = static_cast<T*>(temp);
+    if (is_aligned16(in))
+      TA_LAUNCH("scan_partials", stream, (scan_partials_kernel<T, Op, Pre, true, Shape>), dim3(tiles - 1), dim3(Shape::BLOCK), in, partials);
     else
-      TA_LAUNCH("scan", stream, (scan_apply_kernel<T, Op, Pre, EXCLUSIVE, false, Shape>), dim3(tiles), dim3(Shape::BLOCK), in, out, n, init_v, (const T*)partials);
+      TA_LAUNCH("scan_partials", stream, (scan_partials_kernel<T, Op, Pre, false, Shape>), dim3(tiles - 1), dim3(Shape::BLOCK), in, partials);
+    TA_CHECK_LAUNCH();
+    return launch_apply<T, Op, Shape>(tiles, in, out, n, init_v, partials, stream);
+  }
+
+  template <typename T>
+  static size_t partials_bytes(uint64_t n) {
+    return align_up((size_t)(n / tile_of<ScanShapeTwo, T>() + 1) * sizeof(T), 256);
+  }
+
+  template <typename T, typename Op, typename Shape>
+  static int launch_apply(uint32_t tiles, const T* in, T* out, uint64_t n, T init, const T* partials, hipStream_t stream) {
+    if (is_aligned16(in) && is_aligned16(out))
+      TA_LAUNCH("scan", stream, (scan_apply_kernel<T, Op, Pre, EXCLUSIVE, true, Shape>), dim3(tiles), dim3(Shape::BLOCK), in, out, n, init, partials);
+    else
+      TA_LAUNCH("scan", stream, (scan_apply_kernel<T, Op, Pre, EXCLUSIVE, false, Shape>), dim3(tiles), dim3(Shape::BLOCK), in, out, n, init, partials);
     TA_CHECK_LAUNCH();
     return 0;
   }
@@ -446,9 +472,13 @@ struct ScanLaunch {
     T* out = static_cast<T*>(out_);
     if (n > SCAN_TWO_MAX_BYTES / sizeof(T))
       return run_single_pass<T, Op, ScanShapeLarge, false>(temp, temp_bytes, in, out, n, init, stream);
-    if (n <= tile_of<ScanShapeOne, T>())
-      return run_two_launches<T, Op, ScanShapeOne>(temp, temp_bytes, in, out, n, init, stream);
-    return run_two_launches<T, Op, ScanShapeTwo>(temp, temp_bytes, in, out, n, init, stream);
+    if (n <= tile_of<ScanShapeTwo, T>())
+      return run_one_tile<T, Op, ScanShapeTwo>(temp, temp_bytes, in, out, n, init, stream);
+    if constexpr (sizeof(T) >= 4) {
+      if (n <= tile_of<ScanShapeOne, T>())
+        return run_one_tile<T, Op, ScanShapeOne>(temp, temp_bytes, in, out, n, init, stream);
+    }
+    return run_two_launches<T, Op>(temp, temp_bytes, in, out, n, init, stream);
   }
 
   template <typename T, typename Op>
