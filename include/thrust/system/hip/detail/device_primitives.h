@@ -42,6 +42,24 @@ struct TempLayout {
   }
 };
 
+// ------------------------------------------------------------------ where memory lies
+// True for memory of the current device: what a kernel reads twice comes from its caches the second time.  Not so host
+// and managed memory and other devices', which are read over a link, nor addresses the runtime does not know.  A lookup
+// of 0.06 us, and one more where there are several devices.
+inline bool is_memory_of_this_device(const void* p) {
+  static const int devices = [] {
+    int count = 0;
+    return hipGetDeviceCount(&count) == hipSuccess ? count : 0;
+  }();
+  hipPointerAttribute_t attr;
+  int device = 0;
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess || (devices != 1 && hipGetDevice(&device) != hipSuccess)) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return attr.type == hipMemoryTypeDevice && (devices == 1 || attr.device == device);
+}
+
 // ------------------------------------------------------------------ raw bits
 template <int BYTES> struct UIntOf;
 template <> struct UIntOf<1> { using type = uint8_t; };

@@ -75,9 +75,9 @@ def test_scans_int_bit_exact(dev, oracle, dtype):
 def _edges(dtype):
     """Sizes around the ends of one workgroup's tile, of the tiles of two launches and of their range, and of the reduction by one workgroup."""
     size = np.dtype(dtype).itemsize
-    one, two = (128 << 10) // size, (16 << 10) // size
+    one, two, mid = (128 << 10) // size, (16 << 10) // size, (64 << 10) // size
     most_two, most_reduce = (64 << 20) // size, (512 << 10) // size
-    for edge in (one, one + two, 3 * one, most_reduce, most_two):
+    for edge in (two, mid, mid + two, one, one + two, 3 * one, most_reduce, most_two):
         yield from (edge - 1, edge, edge + 1)
 
 
@@ -93,6 +93,60 @@ def test_scan_and_reduce_at_the_edges_of_their_shapes(dev, dtype):
             assert np.array_equal(dev.exclusive_scan(d, 3).numpy(), shifted), (dtype, n, skip)
             assert dev.reduce(d, dev.PLUS, 0).numpy()[0] == sums[-1], (dtype, n, skip)
             assert dev.reduce(d, dev.MIN, 127).numpy()[0] == min(x[skip:].min(), 127), (dtype, n, skip)
+
+
+@pytest.mark.parametrize("kind", ["device", "pinned", "managed"])
+def test_short_scans_read_memory_behind_a_link_once(dev, kind):
+    """Two launches read the input twice, the second time from the caches; host memory is not in them."""
+    import ctypes
+
+    import torch
+    lib = dev.load()
+    for n in (40_000, (1 << 20) + 1, 9_000_001):
+        x = _ints(n, np.int32, 61)
+        if kind == "managed":
+            ptr = ctypes.c_void_p()
+            dev.check(lib.thrust_amd_malloc_universal(ctypes.byref(ptr), x.nbytes), "malloc")
+            ctypes.memmove(ptr, x.ctypes.data, x.nbytes)
+            src = ptr.value
+        else:
+            t = torch.from_numpy(x)
+            t = t.cuda() if kind == "device" else t.pin_memory()
+            src = t.data_ptr()
+        out = dev.DeviceArray(n, dev.I32)
+        temp, need = dev.Temp(), ctypes.c_size_t(0)
+        dev.check(lib.thrust_amd_inclusive_scan(None, ctypes.byref(need), src, out.ptr, n, dev.I32, dev.PLUS, None), "size")
+        temp.buf = torch.full((need.value,), 255, dtype=torch.uint8, device="cuda")
+        dev.profile_collect()
+        dev.profile_enable()
+        dev.check(lib.thrust_amd_inclusive_scan(temp.buf.data_ptr(), ctypes.byref(need), src, out.ptr, n, dev.I32, dev.PLUS,
+                                                dev.stream_ptr()), "scan")
+        dev.profile_enable(False)
+        kernels = dev.profile_collect()
+        assert np.array_equal(out.numpy(), np.cumsum(x, dtype=np.int32)), n
+        assert ("scan_partials" in kernels) == (kind == "device"), (n, kernels)
+        if kind == "managed":
+            lib.thrust_amd_free_universal(ptr)
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.uint8, np.float64])
+def test_temp_storage_asked_for_with_a_longer_array_serves_a_shorter_one(dev, dtype):
+    """From 32 MiB on the storage a scan asks for grows with the array, and what was asked for with a longer one holds."""
+    import ctypes
+
+    import torch
+    lib = dev.load()
+    size, code = np.dtype(dtype).itemsize, dev.DTYPE_OF_NP[np.dtype(dtype)]
+    longer, shorter = (100 << 20) // size, (48 << 20) // size
+    need = ctypes.c_size_t(0)
+    dev.check(lib.thrust_amd_inclusive_scan(None, ctypes.byref(need), None, None, longer, code, dev.PLUS, None), "size")
+    held = torch.full((need.value + 4096,), 255, dtype=torch.uint8, device="cuda")
+    x = (_ints(shorter, np.uint8, 67) % 4).astype(dtype)
+    d, out = dev.DeviceArray.from_numpy(x), dev.DeviceArray(shorter, code)
+    dev.check(lib.thrust_amd_inclusive_scan(held.data_ptr(), ctypes.byref(need), d.ptr, out.ptr, shorter, code, dev.PLUS,
+                                            dev.stream_ptr()), "scan")
+    assert np.array_equal(out.numpy(), np.cumsum(x, dtype=dtype))
+    assert bool((held[need.value:] == 255).all())  # nothing behind what was given
 
 
 def test_scan_in_place_and_unaligned(dev, oracle):

@@ -27,12 +27,14 @@ struct ScanShapeLarge { static constexpr int BLOCK = 1024, CHUNKS = 12; };
 struct ScanShapeSmall { static constexpr int BLOCK = 256, CHUNKS = 4; };
 constexpr uint64_t SCAN_LARGE_MIN_BYTES = (uint64_t)32 << 20;
 
-// Arrays below SCAN_TWO_MAX_BYTES are scanned by two launches that wait for nothing (scan_partials_kernel,
+// Arrays of up to SCAN_TWO_MAX_BYTES are scanned by two launches that wait for nothing (scan_partials_kernel,
 // scan_apply_kernel): their second read of the input meets the caches, and no tile queues at the ticket.
 // Whole call in us, single pass with its better shape against two launches: 4 MB of int32 10.4 -> 9.7,
 // 16 MB 15.6 (27 with the shape it took) -> 11.3, 32 MB 26 (46) -> 17, 64 MB 35.8 -> 31.7, 128 MB 51 -> 58;
 // int64 8 MB 12 (17) -> 9.7, 32 MB 18 (48) -> 17.7, 64 MB 31.8 -> 32.2, 128 MB 54 -> 60.
 // Tiles of 64 KiB instead of 16: 64 MB 32.5, the others alike.
+// Only where the input is memory of this device: elsewhere both reads go over the link (4 MiB of pinned or managed host
+// memory 91 us by the single pass, 192 by two launches, 64 MiB 1260 and 2500), and the single pass does it.
 struct ScanShapeTwo { static constexpr int BLOCK = 256, CHUNKS = 4; };
 constexpr uint64_t SCAN_TWO_MAX_BYTES = (uint64_t)64 << 20;
 // An array that fits one workgroup takes the second launch alone: up to 16 KiB one of the shape above, elements of 4 and
@@ -379,53 +381,54 @@ struct ScanLaunch {
   template <typename Shape, typename T>
   static constexpr uint64_t tile_of() { return (uint64_t)Shape::BLOCK * Shape::CHUNKS * Vec16<T>::N; }
 
-  // The single-pass kernel.  KEPT_CLEAN: `temp` is storage of the library's own that only this function uses
-  // and that was all zero to begin with; the kernel then clears up after itself and no clearing launch precedes it.
-  template <typename T, typename Op, typename Shape, bool KEPT_CLEAN>
-  static int run_single_pass(void* temp, size_t* temp_bytes, const T* in, T* out, uint64_t n, const void* init,
-                             hipStream_t stream) {
-    constexpr int W = TileWords<T>::W;
-    const uint64_t tiles = (n + tile_of<Shape, T>() - 1) / tile_of<Shape, T>();
-    if (tiles > 0xffffffffull) return (int)hipErrorInvalidValue;
+  // The single-pass kernel's temporary storage for n elements: shape, tiles, and where what begins.
+  struct SinglePass {
+    bool large;
+    uint64_t tiles;
+    size_t off_ticket, off_status, bytes;
+  };
+  template <typename T>
+  static SinglePass single_pass(uint64_t n) {
+    SinglePass p;
+    p.large = n >= SCAN_LARGE_MIN_BYTES / sizeof(T);
+    const uint64_t tile = p.large ? tile_of<ScanShapeLarge, T>() : tile_of<ScanShapeSmall, T>();
+    p.tiles = n / tile + (n % tile != 0);
     TempLayout lay;
-    const size_t off_ticket = lay.add(2 * sizeof(uint32_t));  // the ticket and the count of finished tiles
-    const size_t off_status = lay.add((size_t)tiles * W * sizeof(uint64_t));
-    T init_v;
-    const int rc = check_args<T, Op>(temp, temp_bytes, lay.total, in, out, n, init, init_v);
-    if (rc != 0 || temp == nullptr || n == 0) return rc;
-    uint32_t* ticket = reinterpret_cast<uint32_t*>(static_cast<char*>(temp) + off_ticket);
-    uint64_t* status = reinterpret_cast<uint64_t*>(static_cast<char*>(temp) + off_status);
-    const uint64_t words = tiles * W;
+    p.off_ticket = lay.add(2 * sizeof(uint32_t));  // the ticket and the count of finished tiles
+    p.off_status = lay.add((size_t)p.tiles * TileWords<T>::W * sizeof(uint64_t));
+    p.bytes = lay.total;
+    return p;
+  }
+
+  // KEPT_CLEAN: `temp` is storage of the library's own that only this function uses and that was all zero to begin
+  // with; the kernel then clears up after itself and no clearing launch precedes it.
+  template <typename T, typename Op, typename Shape, bool KEPT_CLEAN>
+  static int launch_single_pass(void* temp, const SinglePass& p, const T* in, T* out, uint64_t n, T init, hipStream_t stream) {
+    uint32_t* ticket = reinterpret_cast<uint32_t*>(static_cast<char*>(temp) + p.off_ticket);
+    uint64_t* status = reinterpret_cast<uint64_t*>(static_cast<char*>(temp) + p.off_status);
+    const uint64_t words = p.tiles * TileWords<T>::W;
     uint32_t* finished = KEPT_CLEAN ? ticket + 1 : nullptr;
     if (!KEPT_CLEAN) {
       TA_LAUNCH("tile_state_init", stream, tile_state_init_kernel, dim3((uint32_t)((words + 255) / 256)), dim3(256), status, words, ticket, 2u);
       TA_CHECK_LAUNCH();
     }
     if (is_aligned16(in) && is_aligned16(out))
-      TA_LAUNCH("scan", stream, (scan_kernel<T, Op, Pre, EXCLUSIVE, true, Shape>), dim3((uint32_t)tiles), dim3(Shape::BLOCK), in, out, n, init_v, status, ticket, finished);
+      TA_LAUNCH("scan", stream, (scan_kernel<T, Op, Pre, EXCLUSIVE, true, Shape>), dim3((uint32_t)p.tiles), dim3(Shape::BLOCK), in, out, n, init, status, ticket, finished);
     else
-      TA_LAUNCH("scan", stream, (scan_kernel<T, Op, Pre, EXCLUSIVE, false, Shape>), dim3((uint32_t)tiles), dim3(Shape::BLOCK), in, out, n, init_v, status, ticket, finished);
+      TA_LAUNCH("scan", stream, (scan_kernel<T, Op, Pre, EXCLUSIVE, false, Shape>), dim3((uint32_t)p.tiles), dim3(Shape::BLOCK), in, out, n, init, status, ticket, finished);
     TA_CHECK_LAUNCH();
     return 0;
   }
 
-  // An array of one tile, in one launch.
-  template <typename T, typename Op, typename Shape>
-  static int run_one_tile(void* temp, size_t* temp_bytes, const T* in, T* out, uint64_t n, const void* init, hipStream_t stream) {
-    T init_v;
-    const int rc = check_args<T, Op>(temp, temp_bytes, partials_bytes<T>(n), in, out, n, init, init_v);
-    if (rc != 0 || temp == nullptr || n == 0) return rc;
-    return launch_apply<T, Op, Shape>(1, in, out, n, init_v, nullptr, stream);
+  // Two launches; `temp` holds the partials of the tiles.
+  template <typename T>
+  static size_t partials_bytes(uint64_t n) {
+    return align_up((size_t)(n / tile_of<ScanShapeTwo, T>() + 1) * sizeof(T), 256);
   }
 
-  // Two launches; `temp` holds the partials of the tiles.
   template <typename T, typename Op>
-  static int run_two_launches(void* temp, size_t* temp_bytes, const T* in, T* out, uint64_t n, const void* init,
-                              hipStream_t stream) {
+  static int launch_two(void* temp, const T* in, T* out, uint64_t n, T init, hipStream_t stream) {
     using Shape = ScanShapeTwo;
-    T init_v;
-    const int rc = check_args<T, Op>(temp, temp_bytes, partials_bytes<T>(n), in, out, n, init, init_v);
-    if (rc != 0 || temp == nullptr || n == 0) return rc;
     const uint32_t tiles = (uint32_t)((n + tile_of<Shape, T>() - 1) / tile_of<Shape, T>());
     T* partials = static_cast<T*>(temp);
     if (is_aligned16(in))
@@ -433,12 +436,7 @@ struct ScanLaunch {
     else
       TA_LAUNCH("scan_partials", stream, (scan_partials_kernel<T, Op, Pre, false, Shape>), dim3(tiles - 1), dim3(Shape::BLOCK), in, partials);
     TA_CHECK_LAUNCH();
-    return launch_apply<T, Op, Shape>(tiles, in, out, n, init_v, partials, stream);
-  }
-
-  template <typename T>
-  static size_t partials_bytes(uint64_t n) {
-    return align_up((size_t)(n / tile_of<ScanShapeTwo, T>() + 1) * sizeof(T), 256);
+    return launch_apply<T, Op, Shape>(tiles, in, out, n, init, partials, stream);
   }
 
   template <typename T, typename Op, typename Shape>
@@ -451,15 +449,11 @@ struct ScanLaunch {
     return 0;
   }
 
-  // Answers the size query (temp null) and checks the arguments; reads the initial value where there is one.
+  // Checks the arguments of a call; reads the initial value where there is one.
   template <typename T, typename Op>
-  static int check_args(void* temp, size_t* temp_bytes, size_t need, const T* in, T* out, uint64_t n, const void* init, T& init_v) {
+  static int check_args(size_t held, size_t need, const T* in, T* out, uint64_t n, const void* init, T& init_v) {
     init_v = Op::template identity<T>();
-    if (temp == nullptr) {
-      *temp_bytes = need;
-      return 0;
-    }
-    if (*temp_bytes < need) return (int)hipErrorInvalidValue;
+    if (held < need) return (int)hipErrorInvalidValue;
     if (n == 0) return 0;
     if (!in || !out || (EXCLUSIVE && !init)) return (int)hipErrorInvalidValue;
     if (EXCLUSIVE) __builtin_memcpy(&init_v, init, sizeof(T));
@@ -470,24 +464,43 @@ struct ScanLaunch {
   static int run(void* temp, size_t* temp_bytes, const void* in_, void* out_, uint64_t n, const void* init, hipStream_t stream) {
     const T* in = static_cast<const T*>(in_);
     T* out = static_cast<T*>(out_);
-    if (n > SCAN_TWO_MAX_BYTES / sizeof(T))
-      return run_single_pass<T, Op, ScanShapeLarge, false>(temp, temp_bytes, in, out, n, init, stream);
-    if (n <= tile_of<ScanShapeTwo, T>())
-      return run_one_tile<T, Op, ScanShapeTwo>(temp, temp_bytes, in, out, n, init, stream);
-    if constexpr (sizeof(T) >= 4) {
-      if (n <= tile_of<ScanShapeOne, T>())
-        return run_one_tile<T, Op, ScanShapeOne>(temp, temp_bytes, in, out, n, init, stream);
+    const SinglePass single = single_pass<T>(n);
+    if (single.tiles > 0xffffffffull) return (int)hipErrorInvalidValue;
+    const bool two = n <= SCAN_TWO_MAX_BYTES / sizeof(T);
+    const size_t partials = two ? partials_bytes<T>(n) : 0;
+    if (temp == nullptr) {
+      *temp_bytes = single.bytes > partials ? single.bytes : partials;
+      return 0;
     }
-    return run_two_launches<T, Op>(temp, temp_bytes, in, out, n, init, stream);
+    T init_v;
+    const int rc = check_args<T, Op>(*temp_bytes, single.bytes, in, out, n, init, init_v);
+    if (rc != 0 || n == 0) return rc;
+    if (n <= tile_of<ScanShapeTwo, T>()) return launch_apply<T, Op, ScanShapeTwo>(1, in, out, n, init_v, nullptr, stream);
+    if constexpr (sizeof(T) >= 4) {
+      if (n <= tile_of<ScanShapeOne, T>()) return launch_apply<T, Op, ScanShapeOne>(1, in, out, n, init_v, nullptr, stream);
+    }
+    // (storage that was asked for with a longer array may hold the single pass's descriptors and not the partials)
+    if (two && *temp_bytes >= partials && is_memory_of_this_device(in)) return launch_two<T, Op>(temp, in, out, n, init_v, stream);
+    return single.large ? launch_single_pass<T, Op, ScanShapeLarge, false>(temp, single, in, out, n, init_v, stream)
+                        : launch_single_pass<T, Op, ScanShapeSmall, false>(temp, single, in, out, n, init_v, stream);
   }
 
+  // In storage that is kept clean (temp null: the size query).
   template <typename T, typename Op>
   static int run_kept_clean(void* temp, size_t* temp_bytes, const void* in_, void* out_, uint64_t n, hipStream_t stream) {
     const T* in = static_cast<const T*>(in_);
     T* out = static_cast<T*>(out_);
-    if (n * sizeof(T) >= SCAN_LARGE_MIN_BYTES)
-      return run_single_pass<T, Op, ScanShapeLarge, true>(temp, temp_bytes, in, out, n, nullptr, stream);
-    return run_single_pass<T, Op, ScanShapeSmall, true>(temp, temp_bytes, in, out, n, nullptr, stream);
+    const SinglePass single = single_pass<T>(n);
+    if (single.tiles > 0xffffffffull) return (int)hipErrorInvalidValue;
+    if (temp == nullptr) {
+      *temp_bytes = single.bytes;
+      return 0;
+    }
+    T init_v;
+    const int rc = check_args<T, Op>(*temp_bytes, single.bytes, in, out, n, nullptr, init_v);
+    if (rc != 0 || n == 0) return rc;
+    return single.large ? launch_single_pass<T, Op, ScanShapeLarge, true>(temp, single, in, out, n, init_v, stream)
+                        : launch_single_pass<T, Op, ScanShapeSmall, true>(temp, single, in, out, n, init_v, stream);
   }
 };
 
