@@ -77,7 +77,7 @@ def _edges(dtype):
     size = np.dtype(dtype).itemsize
     one, two, mid = (128 << 10) // size, (16 << 10) // size, (64 << 10) // size
     most_two, most_reduce = (64 << 20) // size, (512 << 10) // size
-    for edge in (two, mid, mid + two, one, one + two, 3 * one, most_reduce, most_two):
+    for edge in (two, mid, mid + two, one, one + two, 3 * one, most_reduce, (33 << 20) // size, (36 << 20) // size, most_two):
         yield from (edge - 1, edge, edge + 1)
 
 

@@ -29,14 +29,31 @@ constexpr uint64_t SCAN_LARGE_MIN_BYTES = (uint64_t)32 << 20;
 
 // Arrays of up to SCAN_TWO_MAX_BYTES are scanned by two launches that wait for nothing (scan_partials_kernel,
 // scan_apply_kernel): their second read of the input meets the caches, and no tile queues at the ticket.
-// Whole call in us, single pass with its better shape against two launches: 4 MB of int32 10.4 -> 9.7,
-// 16 MB 15.6 (27 with the shape it took) -> 11.3, 32 MB 26 (46) -> 17, 64 MB 35.8 -> 31.7, 128 MB 51 -> 58;
-// int64 8 MB 12 (17) -> 9.7, 32 MB 18 (48) -> 17.7, 64 MB 31.8 -> 32.2, 128 MB 54 -> 60.
-// Tiles of 64 KiB instead of 16: 64 MB 32.5, the others alike.
+// Whole call back to back in us, single pass with the shape it takes at that size / two launches: 4 MiB of int32 11.2 / 7.2,
+// 17 MiB 28.6 / 10.9, 31 MiB 45 / 17, 44 MiB 32.0 / 24.0, 60 MiB 45 / 31.7; int64 4 MiB 11.7 / 7.1, 31 MiB 47 / 17.4;
+// int8 60 MiB 325 / 50; int16 60 MiB 70 / 37.  Tiles of 64 KiB instead of 16: 64 MB 32.5, the others alike.
+// The single pass is the faster one where its large tiles all run at once, if the last, ragged one, which is loaded
+// element by element, is short: int32 34, 37, 40, 43 and 46 MiB (that tile a third full) 19.1 / 18.7, 19.7 / 21.5, 20.1 / 23.0,
+// 20.6 / 24.6, 21.6 / 25.9, but two thirds full 38 MiB 24.7 / 22.0, 44 MiB 25.3 / 24.9, 47 MiB 26.2 / 26.5; a third full 49 MiB
+// 30.2 / 27.3, 58 MiB 30.7 / 30.6, 64 MiB 32.9 / 33.6.  With 8-byte elements the ragged tile matters less: 33 MiB 19.5 / 18.4,
+// 34 MiB 18.4 / 19.0, 35 MiB 18.8 / 20.2, 47 MiB 22.1 / 26.7, 50 MiB 29.8 / 28.1, 61 MiB 31.5 / 32.6.
 // Only where the input is memory of this device: elsewhere both reads go over the link (4 MiB of pinned or managed host
 // memory 91 us by the single pass, 192 by two launches, 64 MiB 1260 and 2500), and the single pass does it.
 struct ScanShapeTwo { static constexpr int BLOCK = 256, CHUNKS = 4; };
 constexpr uint64_t SCAN_TWO_MAX_BYTES = (uint64_t)64 << 20;
+constexpr uint64_t SCAN_TWO_MAX_BYTES_8 = (uint64_t)33 << 20;        // 8-byte elements
+constexpr uint64_t SCAN_TWO_MAX_BYTES_4_SHORT = (uint64_t)36 << 20;  // 4-byte elements, last tile at most half full
+
+template <typename T>
+inline bool scan_takes_two(uint64_t n) {
+  if (n > SCAN_TWO_MAX_BYTES / sizeof(T)) return false;
+  const uint64_t bytes = n * sizeof(T);
+  if (sizeof(T) == 8) return bytes <= SCAN_TWO_MAX_BYTES_8;
+  constexpr uint64_t LARGE_TILE = (uint64_t)ScanShapeLarge::BLOCK * ScanShapeLarge::CHUNKS * 16;
+  if (sizeof(T) == 4 && bytes % LARGE_TILE <= LARGE_TILE / 2) return bytes <= SCAN_TWO_MAX_BYTES_4_SHORT;
+  return true;
+}
+
 // An array that fits one workgroup takes the second launch alone: up to 16 KiB one of the shape above, elements of 4 and
 // 8 bytes up to 64 KiB one of this shape.  Whole call back to back in us, single pass / here: 4093 int32 7.2 / 4.3, 8445
 // 7.3 / 4.7, 16381 7.2 / 6.8 (two launches 7.1), 8189 float64 7.5 / 4.8; int8 8189 7.9 / 6.3, uint8 minimum 4093 7.7 / 5.7.
@@ -466,7 +483,7 @@ struct ScanLaunch {
     T* out = static_cast<T*>(out_);
     const SinglePass single = single_pass<T>(n);
     if (single.tiles > 0xffffffffull) return (int)hipErrorInvalidValue;
-    const bool two = n <= SCAN_TWO_MAX_BYTES / sizeof(T);
+    const bool two = scan_takes_two<T>(n);
     const size_t partials = two ? partials_bytes<T>(n) : 0;
     if (temp == nullptr) {
       *temp_bytes = single.bytes > partials ? single.bytes : partials;
