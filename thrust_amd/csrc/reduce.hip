@@ -6,7 +6,7 @@
 //             partial per workgroup.
 //   kernel 2  one workgroup folds init and the partials and writes *d_out.
 //
-// Up to REDUCE_ONE_MAX_BYTES one workgroup does it all in one launch.
+// Short arrays one workgroup folds in one launch (reduce_takes_one).
 //
 // HBM traffic: n*sizeof(T) read, (grid+1)*sizeof(T) written -- the kernel is bound by
 // the read stream alone.  Replaces the ReduceAgent pair of the reference
@@ -29,6 +29,20 @@ namespace ta {
 // 3.5e-8 (6.8e-8), 131072 4.4e-8 / 4.5e-8 (6.5e-8); float64 20011 9.2e-17 / 7.7e-17 (1.4e-16), 65536 8.1e-17 / 7.9e-17 (1.1e-16).
 constexpr int REDUCE_ONE_BLOCK = 1024;
 constexpr uint64_t REDUCE_ONE_MAX_BYTES = (uint64_t)512 << 10;
+// Single bytes: unpacking them is what takes the time (int8 minimum back to back, two launches / one, 300 KiB 7.3 / 6.9 us,
+// 511 KiB 7.3 / 9.5).
+constexpr uint64_t REDUCE_ONE_MAX_BYTES_1 = (uint64_t)256 << 10;
+// Memory behind a link, pinned host memory for one: a workgroup alone draws some 25 GB/s from it (100 KiB of int32 8.4 / 6.2
+// us, 300 KiB 11.1 / 15.2, 511 KiB 15.6 / 22.0).
+constexpr uint64_t REDUCE_ONE_MAX_BYTES_FAR = (uint64_t)128 << 10;
+
+// Whether one workgroup folds an array of so many bytes (at least one element).
+template <typename T>
+inline bool reduce_takes_one(const T* in, uint64_t n) {
+  constexpr uint64_t most = sizeof(T) == 1 ? REDUCE_ONE_MAX_BYTES_1 : REDUCE_ONE_MAX_BYTES;
+  if (n > most / sizeof(T)) return false;
+  return n <= REDUCE_ONE_MAX_BYTES_FAR / sizeof(T) || is_memory_of_this_device(in);
+}
 
 template <typename T, typename Op, bool ALIGNED>
 __global__ __launch_bounds__(REDUCE_BLOCK) void reduce_partials_kernel(const T* __restrict__ in,
@@ -144,7 +158,7 @@ struct ReduceLaunch {
       TA_CHECK_LAUNCH();
       return 0;
     }
-    if (n <= REDUCE_ONE_MAX_BYTES / sizeof(T)) {
+    if (reduce_takes_one(src, n)) {
       if (is_aligned16(in))
         TA_LAUNCH("reduce_one", stream, (reduce_one_kernel<T, Op, true>), dim3(1), dim3(REDUCE_ONE_BLOCK), src, (uint32_t)n, init_v, static_cast<T*>(d_out));
       else
