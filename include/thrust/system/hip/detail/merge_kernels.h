@@ -35,7 +35,11 @@ constexpr int MERGE_TILE = MERGE_BLOCK * MERGE_ITEMS;
 // with one thread per boundary (as it was) / 4 lanes / 8 lanes / 16 lanes / no launch: 1e6 14.5 / - / - / - / 9.8,
 // 4e6 25.2 / 21.6 / 20.4 / 19.8 / 17.7, 8e6 36.2 / 32.4 / 31.6 / 30.6 / 31.3, 16e6 55.5 / 51.5 / 50.4 / 50.1 / 56.4,
 // 64e6 200 / 194 / 195 / 197 / 229, 1.34e8 398 / 398 / 402 / 409 / 463, 2^28 852 / 866 / - / - / -.
+// Ranges behind a link, in pinned host memory for one, are searched by one thread per boundary in a launch of its own
+// unless the merge is short: there a probe's trip is what counts, and how many there are (uint32, a launch / none, 2e5 39 / 32
+// us, 1e6 114 / 141, 4e6 374 / 573; 9.4e6 one thread / 8 lanes 821 / 898).
 constexpr uint64_t MERGE_SEARCHES_MAX = (uint64_t)1 << 23;
+constexpr uint64_t MERGE_SEARCHES_FAR_MAX = (uint64_t)1 << 18;
 constexpr uint64_t MERGE_EIGHT_LANES_MAX = (uint64_t)1 << 25;
 constexpr uint64_t MERGE_FOUR_LANES_MAX = (uint64_t)1 << 27;
 
@@ -229,7 +233,10 @@ inline int merge_launch(uint64_t* split, const T* a, uint64_t na, const T* b, ui
   const uint64_t total = na + nb;
   const uint64_t tiles = (total + MERGE_TILE - 1) / MERGE_TILE;
   if (tiles > 0x7fffffffull) return (int)hipErrorInvalidValue;
-  if (total <= MERGE_SEARCHES_MAX) {
+  // (beyond 2^27 outputs one thread searches anyway)
+  const bool far = total > MERGE_SEARCHES_FAR_MAX && total <= MERGE_FOUR_LANES_MAX &&
+                   !((na == 0 || is_memory_of_this_device(a)) && (nb == 0 || is_memory_of_this_device(b)));
+  if (total <= MERGE_SEARCHES_MAX && !far) {
     THRUST_AMD_KERNEL_LAUNCH("merge", stream, (merge_kernel<T, V, HAS_VALUES, true, Comp>), dim3((uint32_t)tiles),
                              dim3(MERGE_BLOCK), a, na, b, nb, va, vb, out, vout, comp, (const uint64_t*)nullptr);
     return (int)hipPeekAtLastError();
@@ -238,7 +245,8 @@ inline int merge_launch(uint64_t* split, const T* a, uint64_t na, const T* b, ui
     const uint64_t threads = (tiles + 1) << bits;
     THRUST_AMD_KERNEL_LAUNCH("merge_partition", stream, kernel, dim3((uint32_t)((threads + 255) / 256)), dim3(256), a, na, b, nb, tiles, comp, split);
   };
-  if (total <= MERGE_EIGHT_LANES_MAX) partition(merge_partition_kernel<3, T, Comp>, 3);
+  if (far) partition(merge_partition_kernel<0, T, Comp>, 0);
+  else if (total <= MERGE_EIGHT_LANES_MAX) partition(merge_partition_kernel<3, T, Comp>, 3);
   else if (total <= MERGE_FOUR_LANES_MAX) partition(merge_partition_kernel<2, T, Comp>, 2);
   else partition(merge_partition_kernel<0, T, Comp>, 0);
   hipError_t e = hipPeekAtLastError();

@@ -42,3 +42,17 @@ def test_reduce(dev, dtype, kind):
                                                                          dev.stream_ptr()))
         assert out.numpy()[0] == x.sum(dtype=dtype), n
         assert ("reduce_one" in kernels) == (n <= (near_most if kind == "device" else far_most)), (n, kernels)
+
+
+@pytest.mark.parametrize("places", [("device", "device"), ("pinned", "device"), ("device", "pinned")])
+def test_merge(dev, places):
+    for n in (1 << 18, (1 << 18) + 1, (1 << 20) + 3, (1 << 23) + 5):
+        raw = (datagen.splitmix64(5, n) >> np.uint64(33)).astype(np.uint32)
+        na = n // 2 + 7
+        a, b = np.sort(raw[:na]), np.sort(raw[na:])
+        da, db, out = _placed(a.view(np.int32), places[0]), _placed(b.view(np.int32), places[1]), dev.DeviceArray(n, dev.U32)
+        kernels = _kernels(dev, lambda t, s: dev.load().thrust_amd_merge(t, s, da.data_ptr(), na, db.data_ptr(), n - na, out.ptr,
+                                                                        dev.U32, 0, dev.stream_ptr()))
+        assert np.array_equal(out.numpy(), np.sort(raw)), n
+        searched_inside = n <= (1 << 23 if places == ("device", "device") else 1 << 18)
+        assert ("merge_partition" in kernels) != searched_inside, (n, kernels)
