@@ -42,6 +42,14 @@ int main() {
       }
     }
   }
+  // a launch of several passes: whatever it still reads of the slots stays, the launches behind it are struck out
+  for (int passes = 1; passes <= MAX_PASSES; ++passes) {
+    SortCtl c = plan(passes, 0);
+    const SortCtl before = c;
+    c.strike_out(MAX_PASSES - 1, [](uint32_t* p, uint32_t x) { *p = x; });
+    for (int s = 0; s < MAX_PASSES; ++s) expect(c.slot[s] == before.slot[s], "the running launch reads all slots", passes, 0, s);
+    expect(c.gave_up == 1 && !c.finishes() && !c.copies_back(), "nothing runs behind a launch of several passes", passes, 0, MAX_PASSES - 1);
+  }
   if (failures == 0) std::printf("PASSED\n");
   return failures != 0;
 }

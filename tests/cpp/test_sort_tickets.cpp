@@ -15,7 +15,7 @@
 
 #include "../../thrust_amd/csrc/sort_tickets.hpp"
 
-using ta::class_tile;
+using namespace ta;
 
 static bool bijection(uint32_t tiles) {
   std::vector<uint8_t> seen(tiles, 0);
@@ -89,7 +89,34 @@ static bool finishes(uint32_t tiles, bool bound_to_xcd, uint32_t slots_per_xcd, 
   return true;
 }
 
+// Every written tile is counted on a counter of its own slot, and the counters hold what is due exactly when all are.
+static bool counts(uint32_t tiles) {
+  std::vector<uint32_t> held(COUNTERS, 0);
+  for (uint32_t t = 0; t < tiles; ++t) {
+    bool complete = true;
+    for (uint32_t c = 0; c < COUNTERS; ++c) complete = complete && held[c] == due_on(c, tiles);
+    if (complete || counter_of(t) >= COUNTERS) return false;  // complete too early, or no such counter
+    ++held[counter_of(t)];
+  }
+  // a pass of which any tile gave up is never complete, and its counters say so
+  for (uint32_t bad : {0u, tiles / 2, tiles - 1}) {
+    const uint32_t c = counter_of(bad), with = held[c] - 1 + COUNT_GAVE_UP;
+    if (with == due_on(c, tiles) || with < COUNT_GAVE_UP || due_on(c, tiles) >= COUNT_GAVE_UP) return false;
+  }
+  for (uint32_t c = 0; c < COUNTERS; ++c) {
+    if (held[c] != due_on(c, tiles)) return false;
+    // apart from the word that hands the tiles out, from each other, and inside the slot
+    if (counter_word(c) < TICKET_STRIDE || counter_word(c) % TICKET_STRIDE != 0 || counter_word(c) >= TICKET_CLASSES * TICKET_STRIDE) return false;
+  }
+  return true;
+}
+
 int main() {
+  for (uint32_t tiles = 1; tiles <= 2000; ++tiles)
+    if (!counts(tiles)) {
+      std::printf("tiles=%u: the counters of a pass do not say when it is complete\n", tiles);
+      return 1;
+    }
   for (uint32_t tiles = 1; tiles <= 20000; ++tiles)
     if (!bijection(tiles)) {
       std::printf("tiles=%u: not every tile exactly once, or not rising inside a class\n", tiles);

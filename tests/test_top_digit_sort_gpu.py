@@ -178,9 +178,11 @@ def test_sizes_where_the_kernels_change(dev, dtype, vdtype, edge):
             assert np.array_equal(k.numpy().view(np.uint8), x[order].view(np.uint8)), (n, descending)
 
 
-# (key, value, longest array whose passes behind the short way run in one launch: REST_MAX in thrust_amd/csrc/radix_sort.hip)
+# (key, value, a length): the longest arrays whose passes behind the short way run in one launch (REST_MAX in
+# thrust_amd/csrc/radix_sort.hip), and longer ones of 8-byte keys or values
 ONE_LAUNCH = [(np.uint32, None, 1 << 20), (np.int32, np.uint8, 3 << 18), (np.uint32, np.uint64, 3 << 18),
-              (np.int64, None, 3 << 15), (np.uint64, np.uint16, 3 << 15), (np.float64, np.uint64, 3 << 15)]
+              (np.int64, None, 3 << 15), (np.uint64, np.uint16, 3 << 15), (np.float64, np.uint64, 3 << 15),
+              (np.uint32, np.uint64, 1 << 19), (np.int64, None, 1 << 15), (np.uint64, np.uint16, 1 << 15), (np.float64, np.uint64, 1 << 15)]
 
 
 @pytest.mark.parametrize("dtype,vdtype,edge", ONE_LAUNCH)

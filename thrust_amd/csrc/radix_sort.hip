@@ -443,9 +443,14 @@ __global__ __launch_bounds__(BLOCK) void onesweep_pass_kernel(
   const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);
 #define TA_PASS_LOAD(item) (item)
 #define TA_PASS_STORE(item, value) (item) = (value)
+#define TA_PASS_GIVES_UP() strike_out(slot)
+  auto strike_out = [&](int at) {
+    ctl_out->strike_out(at, [](uint32_t* p, uint32_t x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
+  };
 #include "radix_pass_tile.inc"
 #undef TA_PASS_LOAD
 #undef TA_PASS_STORE
+#undef TA_PASS_GIVES_UP
 }
 
 // ------------------------------------------------------------------ several passes in one launch
@@ -454,15 +459,19 @@ __global__ __launch_bounds__(BLOCK) void onesweep_pass_kernel(
 // then waits until the others have written theirs.  Whoever waits, waits only for workgroups that run and wait for
 // nobody but earlier tiles of the same pass, so this works with any number of workgroups resident.
 // What one pass writes and another XCD's workgroup reads in the next goes past the caches that are not coherent
-// (agent scope): a write-back of the L2 per tile took 35 us a pass.  Short runs leave as partial lines then, so longer
-// arrays keep a launch per pass.  Copy and sort, us, a launch per pass (and the bounds of the short way in a launch, as
-// it was) against this: short way taken, 65536 uint32 40.0 -> 25.9, 2^20 47.5 -> 37.1, 65536 (uint32, uint32) 48.0 -> 30.3,
-// 65536 uint64 54.9 -> 35.9, with uint32 values 60.9 -> 40.6; not taken (90 % one key), 65536 uint32 46.3 -> 43.8, 2^20
-// 63.6 -> 65.0, 1.5e6 72 -> 79, 7.9e5 (uint32, uint32) 66.5 -> 67.7, 65536 uint64 74.2 -> 72.9, 131072 77.4 -> 78.6,
-// 2^20 127 -> 170.  A line is drawn where a sort that declines would pay some per cent.
-// tickets[slot]: word 0 counts the tiles taken, word TICKET_STRIDE those written.
-template <typename K, bool HAS_VALUES>
-constexpr uint64_t REST_MAX = sizeof(K) == 8 ? 3u << 15 : HAS_VALUES ? 3u << 18 : 1u << 20;
+// (agent scope): a write-back of the L2 per tile took 35 us a pass.  Short runs leave as partial lines then, and every
+// pass ends with a trip to memory for its count and one for the next pass's wait, so longer arrays keep a launch per pass.
+// Copy and sort, us, a launch per pass (and the bounds of the short way in a launch) against this: short way taken, 65536
+// uint32 40.0 -> 25.9, 2^20 47.5 -> 36.6, 65536 (uint32, uint32) 48.0 -> 30.3, 30011 uint64 50.4 -> 37.0, with uint64 values
+// 50.8 -> 38.8; not taken (90 % one key), 65536 uint32 46.1 -> 43.6, 2^20 65.7 -> 62.3, 1.5e6 72 -> 79, 7.9e5 (uint32, uint32)
+// 65.7 -> 63.2, 5.2e5 (uint32, uint64) 62.4 -> 62.1, 30011 uint64 70.5 -> 70.4, with uint64 values 78.7 -> 78.9, 10007 of
+// them 74.5 -> 76 (waited for 94 -> 89).  The line is drawn where a sort that declines would pay: 65536 uint64 72.6 -> 74.5, with uint64 values 80.8 -> 84.8, 98304 84.1 -> 87.7,
+// permuted 7.9e5 (uint32, uint64) 66.4 -> 68.0.
+// (One counter for the tiles written instead of seven: 2^20 uint32 66.9, permuted 61.2 against 55.9; flag and slot asked for
+// behind every pass, and the loads of the copy back one after the other, cost another us each.)
+// tickets[slot]: word 0 counts the tiles taken, those at counter_word() the tiles written.
+template <typename K, typename V, bool HAS_VALUES>
+constexpr uint64_t REST_MAX = sizeof(K) == 8 ? 1u << 15 : !HAS_VALUES ? 1u << 20 : sizeof(V) == 8 ? 1u << 19 : 3u << 18;
 
 template <typename K, typename V, bool HAS_VALUES, int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) void onesweep_rest_kernel(
@@ -480,43 +489,62 @@ __global__ __launch_bounds__(BLOCK) void onesweep_rest_kernel(
   __shared__ __attribute__((aligned(16))) unsigned char s_union[Shape::UNION_BYTES];
   __shared__ uint32_t s_scatter_base[RADIX_SIZE];
   __shared__ uint32_t s_digit_wave[RADIX_SIZE / WAVE];
-  __shared__ uint32_t s_tile, s_todo[2];
+  __shared__ uint32_t s_tile, s_go, s_gave_up;
   uint32_t* s_cnt = reinterpret_cast<uint32_t*>(s_union);
   K* s_keys = reinterpret_cast<K*>(s_union);
   V* s_vals = reinterpret_cast<V*>(s_union);
-  uint32_t* finished = nullptr;  // tiles written by the pass before
-  // Thread 0, until the pass before is complete: true, or false if somebody has given up.
+  // What there is to do is read from ctl->slot, which nothing in this launch writes; whether a pass is complete, and
+  // whether one of its tiles gave up, from its counters alone.  A pass begins, and the copy back does, only behind the
+  // complete pass before, so nothing works on keys that a pass left out of place.
+  uint32_t* written = nullptr;  // the counters of the pass before
+  // (the launches behind this one; no slot is struck out)
+  auto strike_out = [&] {
+    ctl_out->strike_out(MAX_PASSES - 1, [](uint32_t* p, uint32_t x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
+  };
+  // The first wave, until the pass before is complete: true, or false if a tile of it gave up or this wait did.
   auto is_complete = [&]() -> bool {
-    for (uint32_t spins = 0; finished != nullptr && __hip_atomic_load(finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != tiles;) {
+    const uint32_t lane = threadIdx.x;
+    const uint32_t due = lane < COUNTERS ? due_on(lane, tiles) : 0;
+    for (uint32_t spins = 0; written != nullptr;) {
+      uint32_t have = due;
+      if (lane < COUNTERS) have = __hip_atomic_load(written + counter_word(lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__builtin_amdgcn_ballot_w64(have >= COUNT_GAVE_UP) != 0) return false;
+      if (__builtin_amdgcn_ballot_w64(have != due) == 0) break;
       __builtin_amdgcn_s_sleep(2);
-      if (++spins >= LOOKBACK_SPIN_LIMIT) {
-        ctl_out->strike_out(-1, [](uint32_t* p, uint32_t x) {
-          __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        });
-        break;
+      ++spins;
+      if (spins % 1024u == 0 &&
+          __builtin_amdgcn_readfirstlane(__hip_atomic_load(&ctl_out->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0)
+        return false;
+      if (spins >= LOOKBACK_SPIN_LIMIT) {
+        strike_out();
+        return false;
       }
     }
-    return __hip_atomic_load(&ctl_out->gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+    return true;
   };
   auto clear_counters = [&] {
     for (int i = threadIdx.x; i < WAVES * RADIX_SIZE; i += BLOCK) s_cnt[i] = 0;
   };
+  if (threadIdx.x == 0) s_gave_up = 0;
+  bool odd = false;  // an odd number of passes leaves the result in the alternate buffer
+  for (int slot = 0; slot < slots; ++slot) odd = odd != SortCtl::runs(ctl->slot[slot]);
   for (int slot = first_slot; slot < slots; ++slot) {
+    const uint32_t todo = ctl->slot[slot];
+    if (!SortCtl::runs(todo)) continue;
     uint32_t* ticket = tickets + (size_t)slot * TICKET_CLASSES * TICKET_STRIDE;
-    // One thread asks what there is to do, so that the whole workgroup goes the same way whenever it changes.
-    if (threadIdx.x == 0) {
-      uint32_t todo = __hip_atomic_load(&ctl_out->slot[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (SortCtl::runs(todo)) {
-        s_tile = atomicAdd(ticket, 1u);  // (on its way while the pass before ends)
-        if (!is_complete()) todo = SortCtl::SKIP;
+    if (threadIdx.x < WAVE) {
+      uint32_t first = 0;
+      if (threadIdx.x == 0) first = atomicAdd(ticket, 1u);  // (on its way while the pass before ends)
+      const bool go = is_complete();
+      if (threadIdx.x == 0) {
+        s_tile = first;
+        s_go = go ? 1u : 0u;
       }
-      s_todo[slot & 1] = todo;
     }
     clear_counters();
     __syncthreads();
-    const uint32_t todo = __builtin_amdgcn_readfirstlane(s_todo[slot & 1]);
-    if (!SortCtl::runs(todo)) continue;
-    finished = ticket + TICKET_STRIDE;
+    if (__builtin_amdgcn_readfirstlane(s_go) == 0) return;
+    written = ticket;
     const int pass = (int)SortCtl::digit(todo);
     const uint32_t* __restrict__ bin_base = hist + pass * RADIX_SIZE;
     const bool from_alt = SortCtl::src_alt(todo);
@@ -526,36 +554,56 @@ __global__ __launch_bounds__(BLOCK) void onesweep_rest_kernel(
     const V* vals_in = from_alt ? vals_b : vals_a;
     V* vals_out = from_alt ? vals_a : vals_b;
     D* status = statuses + (size_t)slot * slot_words;
+    // what the last pass writes stays for the next launch, unless it is copied back here
+    const bool nobody_reads = SortCtl::decodes(todo) && !(copies && odd);
     for (;;) {
       const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);
       if (tile >= tiles) break;
 #define TA_PASS_LOAD(item) __hip_atomic_load(&(item), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-#define TA_PASS_STORE(item, value) __hip_atomic_store(&(item), value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+#define TA_PASS_STORE(item, value) (nobody_reads ? (void)((item) = (value)) : __hip_atomic_store(&(item), value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+#define TA_PASS_GIVES_UP() (s_gave_up = 1, strike_out())
 #include "radix_pass_tile.inc"
 #undef TA_PASS_LOAD
 #undef TA_PASS_STORE
+#undef TA_PASS_GIVES_UP
       // counted in when all of the workgroup's stores have been acknowledged
+      uint32_t next = 0;
+      if (threadIdx.x == 0) next = atomicAdd(ticket, 1u);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       if (threadIdx.x == 0) {
-        __hip_atomic_fetch_add(finished, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_tile = atomicAdd(ticket, 1u);
+        __hip_atomic_fetch_add(ticket + counter_word(counter_of(tile)), s_gave_up != 0 ? COUNT_GAVE_UP : 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_tile = next;
       }
       clear_counters();
       __syncthreads();
     }
     __syncthreads();  // everybody has seen that there are no more tiles
   }
-  if (!copies) return;
-  if (threadIdx.x == 0) {
-    const bool copy = __hip_atomic_load(&ctl_out->final_in_alt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-    s_todo[slots & 1] = copy && is_complete() ? 1u : 0u;
+  if (!copies || !odd) return;
+  if (threadIdx.x < WAVE) {
+    // (no pass of this launch: one of an earlier launch may have given up)
+    const bool go = written != nullptr ? is_complete() : ctl->gave_up == 0;
+    if (threadIdx.x == 0) s_go = go ? 1u : 0u;
   }
   __syncthreads();
-  if (__builtin_amdgcn_readfirstlane(s_todo[slots & 1]) != 0) {
-    for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
-      keys_a[i] = __hip_atomic_load(keys_b + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if constexpr (HAS_VALUES) vals_a[i] = __hip_atomic_load(vals_b + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_amdgcn_readfirstlane(s_go) != 0) {
+    // (all loads in flight together, the last element in the place of those behind it)
+    const uint32_t first = blockIdx.x * BLOCK + threadIdx.x, stride = gridDim.x * BLOCK;
+    K k[ITEMS];
+    V v[HAS_VALUES ? ITEMS : 1];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+      const uint32_t i = first + r * stride < n ? first + r * stride : n - 1;
+      k[r] = __hip_atomic_load(keys_b + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if constexpr (HAS_VALUES) v[r] = __hip_atomic_load(vals_b + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+      const uint32_t i = first + r * stride;
+      if (i >= n) break;
+      keys_a[i] = k[r];
+      if constexpr (HAS_VALUES) vals_a[i] = v[r];
     }
   }
 }
@@ -711,7 +759,7 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
   uint32_t* bounds = reinterpret_cast<uint32_t*>(base + off_bounds);
   uint32_t* long_list = reinterpret_cast<uint32_t*>(base + off_long);
   const bool tail = top_slots == 2;  // (8-byte keys)
-  const int single_launches = hybrid && n <= REST_MAX<K, HAS_VALUES> ? top_slots : slots;  // passes with a launch of their own
+  const int single_launches = hybrid && n <= REST_MAX<K, V, HAS_VALUES> ? top_slots : slots;  // passes with a launch of their own
   for (int slot = 0; slot < slots; ++slot) {
     if constexpr (sizeof(K) >= 4) {
       if (hybrid && slot == top_slots) {
@@ -726,7 +774,7 @@ static int sort_impl(void* temp, size_t* temp_bytes, void* keys, void* values, u
     }
     if constexpr (sizeof(K) >= 4) {
       if (slot >= single_launches) {
-        static_assert(REST_MAX<K, HAS_VALUES> <= Plan::FINE_MAX, "tiles as in the passes before, 32-bit offsets");
+        static_assert(REST_MAX<K, V, HAS_VALUES> <= Plan::FINE_MAX, "tiles as in the passes before, 32-bit offsets");
         TA_LAUNCH("onesweep_rest", stream, (onesweep_rest_kernel<K, V, HAS_VALUES, Plan::BLOCK, Plan::FINE_ITEMS>), dim3((uint32_t)tiles), dim3(Plan::BLOCK), keys_a, keys_b, vals_a, vals_b, (uint32_t)n, slot, slots, (uint32_t)tiles, geo, codec, (const uint32_t*)hist, status, (uint64_t)slot_words, tickets, (const SortCtl*)ctl, ctl, !tail);
         TA_CHECK_LAUNCH();
         if (!tail) return 0;

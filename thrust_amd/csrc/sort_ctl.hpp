@@ -38,10 +38,11 @@ struct SortCtl {
   TA_CTL_FN bool finishes() const { return fast != 0; }
   TA_CTL_FN bool copies_back() const { return final_in_alt != 0; }
 
-  // What a tile of the pass in slot `at` does when it stops waiting (-1: between passes).  The array is not in the order, and does not hold
+  // What a tile of the pass in slot `at` does when it stops waiting.  The array is not in the order, and does not hold
   // the keys, that the launches behind it count on -- their positions could leave it -- so they are struck out: the
   // call ends with an unfinished sort.  store(address, value) has to reach the next launch; fields that the
-  // running launch reads stay as they are.
+  // running launch reads stay as they are.  A launch of several passes reads every slot, so it strikes out none
+  // (at = MAX_PASSES - 1): there a pass begins only behind a complete one, and one of which a tile gave up never is.
   template <typename Store>
   TA_CTL_FN void strike_out(int at, Store store) {
     for (int s = at + 1; s < MAX_PASSES; ++s) store(&slot[s], (uint32_t)SKIP);

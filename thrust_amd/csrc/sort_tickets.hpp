@@ -38,4 +38,13 @@ TA_TICKETS_FN uint32_t class_tile(uint32_t k, uint32_t c, uint32_t tiles) {
   return whole * S + before + (c - whole * G);
 }
 
+// Several passes in one launch: the tiles of a pass that are written count themselves in, tile t on counter
+// counter_of(t) of the slot's others than the first, which hands the tiles out; the pass is complete when every counter
+// holds what is due on it.  (Atomics on one word retire 12 ns apart: 2 us for 171 tiles on one counter.)
+constexpr uint32_t COUNTERS = TICKET_CLASSES - 1;
+constexpr uint32_t COUNT_GAVE_UP = 1u << 16;  // what a tile adds that gave up: never due, so the pass is never complete
+TA_TICKETS_FN uint32_t counter_of(uint32_t tile) { return tile % COUNTERS; }
+TA_TICKETS_FN uint32_t due_on(uint32_t counter, uint32_t tiles) { return (tiles + COUNTERS - 1 - counter) / COUNTERS; }
+TA_TICKETS_FN uint32_t counter_word(uint32_t counter) { return (1 + counter) * TICKET_STRIDE; }
+
 }  // namespace ta
