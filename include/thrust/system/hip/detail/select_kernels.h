@@ -20,7 +20,7 @@
 // contiguous addresses.
 //
 // The in-place partition parks one side in temp storage and copies it back afterwards (unless the array
-// is one tile).  From 32 MiB on its init kernel samples the input and picks the direction of the sweep so that the parked side
+// is one tile).  From 32 MiB on (single bytes from 16) its init kernel samples the input and picks the direction of the sweep so that the parked side
 // is the smaller one: forwards, the selected elements are written in place (each lands at or
 // before its source) and the rejected ones are parked; from the back, the rejected elements
 // are written in place (each lands at or behind its source) and the selected ones are parked.
@@ -76,11 +76,17 @@ constexpr int SELECT_LEAN_ITEMS = 64;
 constexpr int SELECT_LEAN_HEAD_ITEMS = 56;
 constexpr int SELECT_LEAN_TWO_ITEMS = 48;
 constexpr int SELECT_LANE_BYTES = 256;
-// In-place partitions of up to so many bytes sweep forwards without asking which side is the smaller: the sample's
-// loads and a launch cost more than parking the larger side.  Whole call with its copy, us, either way against
-// forwards: int32 with 50 % selected 1e6 32.6 -> 21.7, 4e6 44 -> 34, 16e6 81 -> 71; with 5 % (95 % parked) 4e6
-// 40 -> 36, 12e6 63.7 -> 61.6, 16e6 78 -> 80; float64 with 5 % 4e6 47 -> 42, 8e6 73 -> 74, 16e6 117 -> 141.
+// In-place partitions of up to so many bytes, tested and moved ones, sweep forwards without asking which side is the
+// smaller: the sample's loads and a launch cost more than parking the larger side, unless nearly all of it is parked.  Whole
+// call with its copy back to back, us, either way against forwards: int32 4 MiB with 50 % selected 31.2 / 22.4, 16 MiB 43.8 /
+// 35.6, 31 MiB 56.7 / 47.5; 2 % selected 8 MiB 32.8 / 27.2, 16 MiB 39.2 / 37.3; 0.1 % 8 MiB 32.5 / 27.3, 16 MiB 38.4 / 37.8, 32
+// MiB 50.4 / 49.3 (a call that is waited for: 37.3 / 35.4, 41.3 / 44.7, 49.7 / 51.6).  float64 16 MiB with 50 % 45.0 / 35.1,
+// 0.1 % 37.8 / 36.1.  By a stencil, 24 and 32 MiB in all: int32 by int32 with 1 % selected 42.2 / 35.8, float64 by uint8
+// 46.5 / 42.0, float32 by uint8 47.5 / 42.0.  Beyond 32 MiB of int32 with 5 % selected 78 / 80, of float64 117 / 141.
 constexpr uint64_t SELECT_ONE_WAY_MAX_BYTES = (uint64_t)32 << 20;
+// Single bytes, moved one by one where the two sides do not lie alike: 8 MiB with 50 % 46 / 41, 2 % 45.7 / 40.8, 0.1 % 39.5 /
+// 40.5; 16 MiB 65.3 / 55.4, 62.4 / 54.5, 55.1 / 54.1; 24 MiB 73.2 / 63.4, 72.2 / 71.9, 65.3 / 71.8.
+constexpr uint64_t SELECT_ONE_WAY_MAX_BYTES_1 = (uint64_t)16 << 20;
 constexpr int SELECT_MIN_ITEMS = 8;   // sizes the descriptor array
 constexpr int SELECT_MAX_ITEMS = 32;
 
@@ -515,7 +521,7 @@ THRUST_AMD_DEVICE void select_tile(const SelectArgs<T, U, Flagger>& a, SelectSha
 }
 
 // DIR 0: forward sweep.  DIR 1 / 2: the two kernels of the in-place partition, launched one
-// after the other (up to 32 MiB only the first); the one whose direction (1 forward, 2 from the back) the init kernel did not
+// after the other (smaller arrays only the first); the one whose direction (1 forward, 2 from the back) the init kernel did not
 // choose ends at once.  (One kernel that takes the direction as a run-time value, or that
 // holds both bodies, was measured at twice the time: 0.9 against 0.5 ms on 2^28 float32.)
 template <typename T, typename U, int MODE, bool HAS_PAYLOAD, bool TWO, int DIR, typename Flagger>
@@ -673,7 +679,8 @@ inline int select_launch(char* temp, const SelectTemp& lay, SelectArgs<T, U, Fla
   // A call of one tile waits for no other tile: no descriptors to clear, and the partition in place reads its
   // whole input before it writes, so it parks nothing.  One launch instead of two (instead of four, partition in
   // place): 4097 elements, whole call, copy_if 15.9 -> 11.4 us, unique_by_key 16.0 -> 11.4, partition 28 -> 15.
-  const bool both_ways = DUAL && a.n * (sizeof(T) + (HAS_PAYLOAD ? sizeof(U) : 0)) > SELECT_ONE_WAY_MAX_BYTES;
+  constexpr uint64_t ONE_WAY_MAX_BYTES = sizeof(std::conditional_t<HAS_PAYLOAD, U, T>) == 1 ? SELECT_ONE_WAY_MAX_BYTES_1 : SELECT_ONE_WAY_MAX_BYTES;
+  const bool both_ways = DUAL && a.n * (sizeof(T) + (HAS_PAYLOAD ? sizeof(U) : 0)) > ONE_WAY_MAX_BYTES;
   if (tiles != 1) {
     THRUST_AMD_KERNEL_LAUNCH("select_init", stream, (select_init_kernel<T, MODE, Flagger>),
                              dim3((uint32_t)((init_threads + 255) / 256)), dim3(256), a.status, words, a.ticket,

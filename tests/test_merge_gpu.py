@@ -85,10 +85,11 @@ def test_config5_merge_full_size(dev):
 
 
 @pytest.mark.parametrize("n,kind", [(n, kind) for n in (4095, 4097, (1 << 23) - 1, 1 << 23, (1 << 23) + 1, (1 << 25) + 1)
-                                    for kind in ("mixed", "equal", "apart", "short", "none")] + [((1 << 27) + 1, "mixed")])
+                                    for kind in ("mixed", "equal", "apart", "short", "none")] + [(n, "mixed") for n in (1 << 25, 1 << 27, (1 << 27) + 1)])
 def test_boundaries_by_groups_of_lanes(dev, n, kind):
-    """The boundaries of the tiles on the merge path, by every group size, at both ends of its range: ranges that
-    interleave, of one key, one wholly before the other, one of 33 elements, one empty."""
+    """The boundaries of the tiles on the merge path, by every group size, at both ends of its range (one lane: at the
+    lower one): ranges that interleave and, for the most sizes, of one key, one wholly before the other, one of 33
+    elements, one empty."""
     na = {"mixed": n // 2, "equal": n // 3, "apart": n // 2 + 5, "short": 33, "none": 0}[kind]
     raw = (datagen.splitmix64(5, n) >> np.uint64(33)).astype(np.uint32)
     if kind == "equal":

@@ -232,7 +232,7 @@ def test_calls_of_one_tile_and_their_neighbours(dev, oracle, dtype, skip):
     temp = dev.Temp()
     temp.buf = torch.full((1 << 20,), 255, dtype=torch.uint8, device="cuda")
     thr = 0.3 if np.dtype(dtype).kind == "f" else 60
-    for edge in (64, 1024, 16384, 24576, 28672, 32768):
+    for edge in (64, 1024, 16384, 20480, 24576, 28672, 32768):
         for n in (edge - 1, edge, edge + 1):
             x = _vals(n + skip, dtype, 31)
             st = _vals(n + skip, np.int32, 37)[skip:]
@@ -265,6 +265,15 @@ def test_partition_in_place_on_both_sides_of_the_one_way_limit(dev, dtype, skip)
             cnt = dev.stable_partition(d, dev.LT, thr)
             assert cnt == np.count_nonzero(y < thr)
             assert np.array_equal(d.numpy(), np.concatenate([y[y < thr], y[y >= thr]])), (dtype, n, thr)
+
+
+def test_partition_of_bytes_on_both_sides_of_their_limit(dev):
+    for n in (16 << 20, (16 << 20) + 1):
+        x = _vals(n, np.uint8, 53)
+        for thr in (2, 190):
+            d = dev.DeviceArray.from_numpy(x)
+            assert dev.stable_partition(d, dev.LT, thr) == np.count_nonzero(x < thr)
+            assert np.array_equal(d.numpy(), np.concatenate([x[x < thr], x[x >= thr]])), (n, thr)
 
 
 def test_partition_in_place_by_stencil_beyond_the_one_way_limit(dev):
