@@ -156,8 +156,8 @@ __global__ __launch_bounds__((FinishShape<K, V, HAS_VALUES>::BLOCK), (FinishShap
   K* __restrict__ keys_out = keys_a + first;
   V* __restrict__ vals_out = HAS_VALUES ? vals_a + first : nullptr;
   // f(r, the place r * BLOCK + tid) for all rounds, each behind a branch of its own (in pairs, without a branch inside,
-  // the loads of two are in flight together, but an odd round more is computed and registers spill: 0.97 against 0.73 ms
-  // for 2^27 pairs of (uint64, uint32), 0.63 against 0.56 for keys alone)
+  // the loads of two are in flight together, but an odd round more is computed, and with values registers spill: 0.97
+  // against 0.73 ms for 2^27 pairs of (uint64, uint32), 0.63 against 0.56 for keys alone, which spill neither way)
   // (opaque copy: what a sweep derives from the place is not kept in registers for the next)
   auto each_round = [&](auto f) {
     uint32_t t = tid;

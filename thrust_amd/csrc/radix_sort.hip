@@ -462,11 +462,11 @@ __global__ __launch_bounds__(BLOCK) void onesweep_pass_kernel(
 // (agent scope): a write-back of the L2 per tile took 35 us a pass.  Short runs leave as partial lines then, and every
 // pass ends with a trip to memory for its count and one for the next pass's wait, so longer arrays keep a launch per pass.
 // Copy and sort, us, a launch per pass (and the bounds of the short way in a launch) against this: short way taken, 65536
-// uint32 40.0 -> 25.9, 2^20 47.5 -> 36.6, 65536 (uint32, uint32) 48.0 -> 30.3, 30011 uint64 50.4 -> 37.0, with uint64 values
-// 50.8 -> 38.8; not taken (90 % one key), 65536 uint32 46.1 -> 43.6, 2^20 65.7 -> 62.3, 1.5e6 72 -> 79, 7.9e5 (uint32, uint32)
+// uint32 40.0 -> 25.9, 2^20 47.5 -> 36.6, 65536 (uint32, uint32) 48.0 -> 30.3, 30011 uint64 48.9 -> 36.8, with uint64 values
+// 49.4 -> 38.5; not taken (90 % one key), 65536 uint32 46.1 -> 43.6, 2^20 65.7 -> 62.3, 1.5e6 72 -> 79, 7.9e5 (uint32, uint32)
 // 65.7 -> 63.2, 5.2e5 (uint32, uint64) 62.4 -> 62.1, 30011 uint64 70.5 -> 70.4, with uint64 values 78.7 -> 78.9, 10007 of
-// them 74.5 -> 76 (waited for 94 -> 89).  The line is drawn where a sort that declines would pay: 65536 uint64 72.6 -> 74.5, with uint64 values 80.8 -> 84.8, 98304 84.1 -> 87.7,
-// permuted 7.9e5 (uint32, uint64) 66.4 -> 68.0.
+// them 74.5 -> 76 (waited for 94 -> 89).  The line is drawn where a sort that declines would pay: 65536 uint64 72.6 -> 74.5,
+// with uint64 values 80.8 -> 84.8, 98304 84.1 -> 87.7, permuted 7.9e5 (uint32, uint64) 66.4 -> 68.0.
 // (One counter for the tiles written instead of seven: 2^20 uint32 66.9, permuted 61.2 against 55.9; flag and slot asked for
 // behind every pass, and the loads of the copy back one after the other, cost another us each.)
 // tickets[slot]: word 0 counts the tiles taken, those at counter_word() the tiles written.
