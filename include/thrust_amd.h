@@ -253,7 +253,8 @@ int thrust_amd_inclusive_scan(void* temp, size_t* temp_bytes, const void* in, vo
  * 1 MiB array inside the library's device image (one copy per GPU, held until the process
  * ends); the call performs no hipMalloc / hipFree.  The array is all zero when the library is
  * loaded and the scan kernel clears what it used before it ends, so the call is ONE kernel
- * launch (the entry point with temporary storage needs another launch first).
+ * launch (the entry point with temporary storage needs another launch first, but for
+ * the shortest arrays).
  * n is limited by that array: up to 131040 tiles (about 6.4e9 elements of 4 bytes or less,
  * 1.6e9 of 8 bytes); a larger n returns hipErrorInvalidValue and launches nothing.  Every
  * call on a GPU shares that GPU's array.  The library orders such calls itself: each call's
