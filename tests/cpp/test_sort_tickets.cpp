@@ -7,7 +7,10 @@
 //      lower tile has been taken (its look-back then finds their counts).  Model A: the
 //      workgroups of class k run on XCD k only, each XCD dispatching its own in order at its own
 //      pace into any number of slots.  Model B: workgroups are dispatched in order of their index
-//      into at least 64 slots anywhere.  Random paces and finishing orders, many seeds.
+//      into at least 64 slots anywhere.  Random paces and finishing orders, many seeds;
+//   3. several passes in one launch (onesweep_rest_kernel) end with any number of workgroups resident: no pass begins
+//      before every tile of the one before is written, every tile is written once, and a tile that gives up ends the
+//      launch with no later pass begun.
 #include <cstdint>
 #include <cstdio>
 #include <random>
@@ -89,6 +92,79 @@ static bool finishes(uint32_t tiles, bool bound_to_xcd, uint32_t slots_per_xcd, 
   return true;
 }
 
+// Several passes in one launch: each workgroup draws tiles of a pass until there are none, then waits until the counters
+// of the pass hold what is due.  A tile is written once all lower ones of its pass have been drawn (its look-back finds
+// their counts then).  `bad` (pass, tile): a tile that gives up.  False when stuck or out of turn.
+static bool shares_launch(uint32_t tiles, uint32_t passes, uint32_t slots, uint32_t seed, int bad_pass, uint32_t bad_tile) {
+  std::mt19937 rnd(seed);
+  struct Group {
+    uint32_t pass;
+    int64_t tile;  // -1: has to draw; -2: waits for the pass before
+  };
+  std::vector<uint32_t> ticket(passes, 0);
+  std::vector<std::vector<uint32_t>> held(passes, std::vector<uint32_t>(COUNTERS, 0));
+  std::vector<std::vector<uint8_t>> written(passes, std::vector<uint8_t>(tiles, 0));
+  auto state_of = [&](uint32_t pass) {  // 1 complete, 0 not yet, -1 never
+    bool complete = true;
+    for (uint32_t c = 0; c < COUNTERS; ++c) {
+      if (held[pass][c] >= COUNT_GAVE_UP) return -1;
+      complete = complete && held[pass][c] == due_on(c, tiles);
+    }
+    return complete ? 1 : 0;
+  };
+  std::vector<Group> resident;
+  uint32_t started = 0, ended = 0;
+  while (ended < tiles) {
+    bool can_move = false;
+    while (resident.size() < slots && started < tiles) {
+      resident.push_back(Group{0, -2});
+      ++started;
+      can_move = true;
+    }
+    std::vector<Group> keep;
+    for (Group g : resident) {
+      bool ends = false;
+      if (g.tile == -2) {
+        const int before = g.pass == 0 ? 1 : state_of(g.pass - 1);
+        if (before != 0) {
+          can_move = true;
+          if (rnd() % 2) {
+            if (before < 0) ends = true;
+            else g.tile = -1;
+          }
+        }
+      } else if (g.tile == -1) {
+        can_move = true;
+        if (rnd() % 2) {
+          const uint32_t t = ticket[g.pass]++;
+          if (t < tiles) {
+            g.tile = t;
+          } else {
+            g.tile = -2;
+            if (++g.pass == passes) ends = true;
+          }
+        }
+      } else {
+        can_move = true;  // every lower tile has been drawn before this one, by a workgroup that runs or is through
+        if (rnd() % 3) {
+          const uint32_t t = (uint32_t)g.tile;
+          if (written[g.pass][t]++) return false;
+          held[g.pass][counter_of(t)] += (int)g.pass == bad_pass && t == bad_tile ? COUNT_GAVE_UP : 1u;
+          g.tile = -1;
+        }
+      }
+      if (ends) ++ended;
+      else keep.push_back(g);
+    }
+    resident.swap(keep);
+    if (!can_move) return false;
+  }
+  for (uint32_t p = 0; p < passes; ++p)
+    for (uint32_t t = 0; t < tiles; ++t)
+      if (written[p][t] != (bad_pass < 0 || (int)p <= bad_pass ? 1 : 0)) return false;
+  return true;
+}
+
 // Every written tile is counted on a counter of its own slot, and the counters hold what is due exactly when all are.
 static bool counts(uint32_t tiles) {
   std::vector<uint32_t> held(COUNTERS, 0);
@@ -141,6 +217,14 @@ int main() {
           return 1;
         }
     }
+  for (uint32_t tiles : {1u, 2u, 6u, 7u, 8u, 50u, 171u})
+    for (uint32_t slots : {1u, 2u, 5u, 64u, 171u})
+      for (uint32_t seed = 1; seed <= 6; ++seed)
+        for (int bad = -1; bad < 3; ++bad)
+          if (!shares_launch(tiles, 3, slots, seed, bad, seed * 13 % tiles)) {
+            std::printf("passes in one launch: tiles=%u, %u slots, seed %u, gives up in pass %d\n", tiles, slots, seed, bad);
+            return 1;
+          }
   std::printf("PASSED\n");
   return 0;
 }
