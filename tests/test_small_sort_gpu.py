@@ -8,7 +8,7 @@ from thrust_amd import datagen
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [2, 63, 65, 255, 257, 2047, 2048, 2049, 4095, 8191, 8192, 8193]
+SIZES = [2, 63, 65, 255, 257, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097, 8191, 8192, 8193]
 
 
 def _keys(kind, dtype, n):

@@ -7,15 +7,20 @@
 namespace ta {
 
 // Four waves have fewer barriers to wait at, sixteen rank faster (copy and sort of 2048 uint32: 12.9 us with
-// 256 threads, 10.9 with 1024; of 1000: 10 us with either).
+// 256 threads, 10.9 with 1024; of 1000: 10 us with either).  Kernels for no more keys per thread than a size needs: with
+// code and loads for eight, copy and sort of 1025 (uint64, uint64) took 13.8 us (12.8 with each load behind its own
+// predicate), now 11.5; 3001 uint32 13.0 -> 12.3, with uint32 values 14.1 -> 13.0, 1000 (uint64, uint64) 11.3 -> 10.7.
 constexpr uint32_t SMALL_SORT_NARROW_MAX = 1024;
 
 template <typename K, typename V, bool HAS_VALUES>
 static int run_small_sort(K* keys, V* values, uint32_t n, const KeyCodec<K>& codec, int begin_bit, int end_bit, hipStream_t stream) {
-  if (n <= SMALL_SORT_NARROW_MAX)
-    TA_LAUNCH("small_sort", stream, (small_sort_kernel<K, V, HAS_VALUES, 256>), dim3(1), dim3(256), keys, values, n, codec, begin_bit, end_bit);
-  else
-    TA_LAUNCH("small_sort", stream, (small_sort_kernel<K, V, HAS_VALUES, 1024>), dim3(1), dim3(1024), keys, values, n, codec, begin_bit, end_bit);
+  auto launch = [&](auto kernel, uint32_t block) {
+    TA_LAUNCH("small_sort", stream, kernel, dim3(1), dim3(block), keys, values, n, codec, begin_bit, end_bit);
+  };
+  if (n <= SMALL_SORT_NARROW_MAX) launch(small_sort_kernel<K, V, HAS_VALUES, 256, 4>, 256);
+  else if (n <= 2 * 1024) launch(small_sort_kernel<K, V, HAS_VALUES, 1024, 2>, 1024);
+  else if (n <= 4 * 1024) launch(small_sort_kernel<K, V, HAS_VALUES, 1024, 4>, 1024);
+  else launch(small_sort_kernel<K, V, HAS_VALUES, 1024, SMALL_ITEMS>, 1024);
   TA_CHECK_LAUNCH();
   return 0;
 }

@@ -12,9 +12,10 @@
 //     Should a group turn out larger than SMALL_GROUP_MAX, all digits get their pass, from the lowest
 //     (the arrangement so far is a stable one, so equal keys still come out in their original order).
 // One copy and one sort, back to back, against the same through the chained passes (eight launches):
-// 3001 uint32 53.7 -> 12.7 us, 8192 uint32 56.7 -> 20.9, 8192 float32 58.7 -> 24.3, 3001 (uint64, uint32)
-// 81.0 -> 17.3, 8192 float64 79.6 -> 30.  (All loads in flight at the start, the values' too, instead of one after
-// the other and the values behind the sort: 8192 uint32 23.0 -> 20.9, with uint32 values 29.1 -> 25.0.)  All digits of the float64 take 93 us: the passes' ranking is what
+// 3001 uint32 53.7 -> 12.0 us, 8192 uint32 56.7 -> 20.9, 8192 float32 58.7 -> 24.3, 3001 (uint64, uint32)
+// 81.0 -> 15.7, 8192 float64 79.6 -> 28.3.  (All loads in flight at the start, the values' too, instead of one after
+// the other and the values behind the sort: 8192 uint32 23.0 -> 20.9, with uint32 values 29.1 -> 25.0.)  All digits of
+// the float64 take 93 us: the passes' ranking is what
 // the time goes into, hence the effort to leave passes out.  Beyond 8192 keys one CU is no longer
 // fast enough (its ranking alone takes 3 us per pass and 8192 keys).
 // Values do not travel with the keys: every key carries its 16-bit index, the values wait in registers, are
@@ -32,11 +33,11 @@ constexpr int SMALL_GROUP_MAX = 24;
 constexpr uint32_t SMALL_GROUP_MEAN = 4;
 constexpr int SMALL_TOP_DIGITS_MAX = 4;
 
-template <typename K, typename V, bool HAS_VALUES, int BLOCK>
+template <typename K, typename V, bool HAS_VALUES, int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys, V* __restrict__ vals, uint32_t n,
                                                            KeyCodec<K> codec, int begin_bit, int end_bit) {
   constexpr int WAVES = BLOCK / WAVE;
-  constexpr int CAP = BLOCK * SMALL_ITEMS;
+  constexpr int CAP = BLOCK * ITEMS;
   constexpr int SAMPLE_WAVES = WAVES < 8 ? WAVES : 8;  // two per SIMD: more cost time, fewer see too little
   constexpr size_t ITEM = (HAS_VALUES && sizeof(V) > sizeof(K)) ? sizeof(V) : sizeof(K);
   static_assert(BLOCK >= RADIX_SIZE && CAP <= 65536, "a thread per digit; 16-bit indices");
@@ -51,27 +52,27 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
   V* s_vals = reinterpret_cast<V*>(s_items);
 
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int rounds = (int)((n + BLOCK - 1) / BLOCK);                    // uniform, <= SMALL_ITEMS
+  const int rounds = (int)((n + BLOCK - 1) / BLOCK);                    // uniform, <= ITEMS
   const uint32_t span = (uint32_t)wave * (WAVE * rounds) + lane;       // wave-striped: + r * WAVE
   uint32_t* my_cnt = s_cnt + wave * RADIX_SIZE;
   const K range = (K)((end_bit - begin_bit >= (int)sizeof(K) * 8 ? ~(K)0 : (K)(((K)1 << (end_bit - begin_bit)) - 1)) << begin_bit);
 
   // ---- load, keys and values, all in flight together: without predicates (a predicated load is waited for before
   // the next is issued), the last element in the place of those behind it; slots past the end sort last
-  K e[SMALL_ITEMS];
-  V v[HAS_VALUES ? SMALL_ITEMS : 1];
-  uint32_t idx[SMALL_ITEMS];
+  K e[ITEMS];
+  V v[HAS_VALUES ? ITEMS : 1];
+  uint32_t idx[ITEMS];
   K first = keys[0];
 #pragma unroll
-  for (int r = 0; r < SMALL_ITEMS; ++r) e[r] = keys[span + r * WAVE < n ? span + r * WAVE : n - 1];
+  for (int r = 0; r < ITEMS; ++r) e[r] = keys[span + r * WAVE < n ? span + r * WAVE : n - 1];
   if constexpr (HAS_VALUES) {
 #pragma unroll
-    for (int r = 0; r < SMALL_ITEMS; ++r) v[r] = vals[span + r * WAVE < n ? span + r * WAVE : n - 1];
+    for (int r = 0; r < ITEMS; ++r) v[r] = vals[span + r * WAVE < n ? span + r * WAVE : n - 1];
   }
   first = codec.encode(first);
   K differ = 0;
 #pragma unroll
-  for (int r = 0; r < SMALL_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const uint32_t pos = span + r * WAVE;
     idx[r] = pos;
     e[r] = codec.encode(e[r]);
@@ -97,10 +98,10 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
   // One stable pass over bits [lo, lo + nbits): afterwards e / idx hold, and s_keys / s_idx mirror, the
   // new arrangement.  s_cnt is all zero at entry and at exit.
   auto pass = [&](int lo, int nbits) {
-    uint32_t rank[SMALL_ITEMS];
+    uint32_t rank[ITEMS];
     auto digit_of = [&](K x) { return (uint32_t)(x >> lo) & ((1u << nbits) - 1u); };
 #pragma unroll
-    for (int r = 0; r < SMALL_ITEMS; ++r)
+    for (int r = 0; r < ITEMS; ++r)
       if (r < rounds) rank[r] = wave_rank_round(digit_of(e[r]), my_cnt);
     __syncthreads();
     uint32_t sum = 0, incl = 0;
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < SMALL_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
       if (r < rounds) {
         const uint32_t p = my_cnt[digit_of(e[r])] + rank[r];
         s_keys[p] = e[r];
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
     __syncthreads();
     for (int i = threadIdx.x; i < WAVES * RADIX_SIZE; i += BLOCK) s_cnt[i] = 0;
 #pragma unroll
-    for (int r = 0; r < SMALL_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
       if (r < rounds) {
         e[r] = s_keys[span + r * WAVE];
         if constexpr (HAS_VALUES) idx[r] = s_idx[span + r * WAVE];
@@ -182,10 +183,10 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
       if (whole) break;
       // groups of keys that share bits [top, hi] (and the constant bits above)
       const K upper = (K)(range & ~(((K)1 << top) - 1)), lower = (K)(range & (((K)1 << top) - 1));
-      uint32_t dest[SMALL_ITEMS];
+      uint32_t dest[ITEMS];
       bool large = false;
 #pragma unroll
-      for (int r = 0; r < SMALL_ITEMS; ++r) {
+      for (int r = 0; r < ITEMS; ++r) {
         const uint32_t p = span + r * WAVE;
         dest[r] = p;
         if (r < rounds && p < n) {
@@ -219,7 +220,7 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
         continue;
       }
 #pragma unroll
-      for (int r = 0; r < SMALL_ITEMS; ++r) {
+      for (int r = 0; r < ITEMS; ++r) {
         if (r < rounds) {
           s_keys[dest[r]] = e[r];
           if constexpr (HAS_VALUES) s_idx[dest[r]] = (uint16_t)idx[r];
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
       }
       __syncthreads();
 #pragma unroll
-      for (int r = 0; r < SMALL_ITEMS; ++r) {
+      for (int r = 0; r < ITEMS; ++r) {
         if (r < rounds) {
           e[r] = s_keys[span + r * WAVE];
           if constexpr (HAS_VALUES) idx[r] = s_idx[span + r * WAVE];
@@ -241,14 +242,14 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(K* __restrict__ keys,
   // ---- store
   if constexpr (HAS_VALUES) {
 #pragma unroll
-    for (int r = 0; r < SMALL_ITEMS; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
       const uint32_t pos = span + r * WAVE;
       if (r < rounds && pos < n) s_vals[pos] = v[r];
     }
     __syncthreads();
   }
 #pragma unroll
-  for (int r = 0; r < SMALL_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const uint32_t pos = span + r * WAVE;
     if (r < rounds && pos < n) {
       keys[pos] = codec.decode(e[r]);
